@@ -4,8 +4,9 @@
     python build.py [--force] [--jobs N]
 
 Sources are compiled in parallel into _build/ and linked into lib/libcatabrafft.so.  The radix
-codelets (csrc/codelets.h) are regenerated first by gen/gen_codelets.py.  Without --force an
-object is rebuilt only when a source or header is newer than it.
+codelets (csrc/codelets.h) and the list of fixed lines (csrc/fixed_table.h) are regenerated first
+by gen/gen_codelets.py and gen/gen_lines.py.  Without --force an object is rebuilt only when a
+source or header is newer than it.
 """
 from __future__ import annotations
 
@@ -63,11 +64,27 @@ def _compile(src: str, force: bool) -> str:
     return obj
 
 
+def _generate(gen: str, out: str) -> None:
+    """Runs a generator; its header is replaced only when it changed."""
+    tmp = out + ".tmp"
+    subprocess.run([sys.executable, gen, tmp], check=True, capture_output=True)
+    with open(tmp, "rb") as f:
+        new = f.read()
+    old = b""
+    if os.path.exists(out):
+        with open(out, "rb") as f:
+            old = f.read()
+    if new == old:
+        os.remove(tmp)
+    else:
+        os.replace(tmp, out)
+
+
 def build(force: bool = False, jobs: int = 8) -> str:
     os.makedirs(BUILD, exist_ok=True)
     os.makedirs(LIBDIR, exist_ok=True)
-    subprocess.run([sys.executable, os.path.join(HERE, "gen", "gen_codelets.py"),
-                    os.path.join(CSRC, "codelets.h")], check=True, capture_output=True)
+    for gen, out in (("gen_codelets.py", "codelets.h"), ("gen_lines.py", "fixed_table.h")):
+        _generate(os.path.join(HERE, "gen", gen), os.path.join(CSRC, out))
     srcs = sources()
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
         objs = list(ex.map(lambda s: _compile(s, force), srcs))

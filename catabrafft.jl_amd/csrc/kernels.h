@@ -152,6 +152,19 @@ struct RealAuxArgs {
     const void* w;
 };
 
+// Rows kernel of one line whose radices are compile-time constants (fixed_line.h): np radices r
+// of a length N, Tt threads and Ls LDS elements per line; launch runs a.C lines per workgroup
+// (a.Ls = Ls; no convolution epilogue).  prepare lets the kernel use its LDS, once per plan.
+struct FixedRow {
+    const int* r;
+    int np, N, Tt, Ls;
+    hipError_t (*launch)(const void* in, void* out, const RowsArgs& a, const void* tw,
+                         hipStream_t st);
+    void (*prepare)();
+};
+// The fixed rows kernel of a radix sequence, nullptr where there is none.
+const FixedRow* find_fixed_row(Prec p, const PassTable& pt, int N);
+
 // Sets per-kernel attributes (large LDS) once; called when a context is created.
 void init_kernels();
 

@@ -1,4 +1,7 @@
 // kernels_dispatch.cpp -- launch_* entry points of kernels.h, dispatched on precision.
+#include <algorithm>
+#include <unordered_map>
+
 #include "kernels.h"
 #include "kernels_prec.h"
 #include "multi.h"
@@ -14,6 +17,37 @@ void init_kernels() {
     init_kernels_f16();
     init_kernels_pipe_f32();
     init_kernels_pipe_f64();
+}
+
+// Fixed kernels by length; each index is built at its first look-up.
+template <class F>
+static std::unordered_multimap<int, F> index_by_length(const std::vector<F>& rows) {
+    std::unordered_multimap<int, F> m;
+    for (const F& r : rows) m.emplace(r.N, r);
+    return m;
+}
+template <class F>
+static const F* find_in(const std::unordered_multimap<int, F>& m, const PassTable& pt, int N) {
+    const auto range = m.equal_range(N);
+    for (auto it = range.first; it != range.second; ++it)
+        if (it->second.np == pt.npass && std::equal(pt.radix, pt.radix + pt.npass, it->second.r))
+            return &it->second;
+    return nullptr;
+}
+const FixedRow* find_fixed_row(Prec p, const PassTable& pt, int N) {
+    static const auto f32 = [] {
+        std::vector<FixedRow> v;
+        fixed_rows_f32_0(v);
+        fixed_rows_f32_1(v);
+        return index_by_length(v);
+    }();
+    static const auto f64 = [] {
+        std::vector<FixedRow> v;
+        fixed_rows_f64_0(v);
+        fixed_rows_f64_1(v);
+        return index_by_length(v);
+    }();
+    return find_in(p == Prec::F32 ? f32 : f64, pt, N);
 }
 
 hipError_t launch_rows_pipe(Prec p, const void* in, void* out, const RowsArgs& a,

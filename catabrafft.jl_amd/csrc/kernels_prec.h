@@ -1,6 +1,8 @@
 // kernels_prec.h -- per-precision launch entry points (defined in kernels_f32.hip,
 // kernels_f64.hip and kernels_f16.hip, dispatched on Prec by kernels_dispatch.cpp).
 #pragma once
+#include <vector>
+
 #include "kernels.h"
 
 namespace cfft {
@@ -18,6 +20,12 @@ namespace cfft {
 CFFT_DECLARE_LAUNCHERS(f32)
 CFFT_DECLARE_LAUNCHERS(f64)
 #undef CFFT_DECLARE_LAUNCHERS
+
+// The fixed rows kernels, in parts compiled by a translation unit each (fixed_rows.h).
+void fixed_rows_f32_0(std::vector<FixedRow>& rows);
+void fixed_rows_f32_1(std::vector<FixedRow>& rows);
+void fixed_rows_f64_0(std::vector<FixedRow>& rows);
+void fixed_rows_f64_1(std::vector<FixedRow>& rows);
 
 hipError_t real_rows_f32(const void* in, void* out, const RealArgs& a, const PassTable& pt,
                          const void* tw, int E, hipStream_t st);

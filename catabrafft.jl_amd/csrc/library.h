@@ -69,6 +69,8 @@ struct Plan {
     FourStepPlan fs;
     mutable std::mutex scratch_mu;
     mutable DevBuf scratch;
+    const FixedRow* fixed = nullptr;  // direct: the line's own rows kernel, fixed_c lines per
+    int fixed_c = 1;                  // workgroup (nullptr: the run-time rows kernel)
     // Executions that use the plan's own work buffers are ordered on the device: each waits for
     // work_ev (recorded by the previous one, on whatever stream) before it starts.
     mutable std::mutex exec_mu;
