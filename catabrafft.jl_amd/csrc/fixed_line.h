@@ -86,7 +86,13 @@ struct FixedLds {
 
 // Pass I of line Q with TT threads: src.at<STEP>(e, j) is element e + j STEP of its input,
 // dst.put_at<STEP>(e, k, v) stores element e + k STEP of its output.  BAR: a barrier between the
-// reads and the writes (both go to the same LDS).  Twiddles load first, as in stockham_pass.
+// reads and the writes (both go to the same LDS).  Twiddles load first, and a source's post_at
+// runs once all of the pass's loads are issued, as in stockham_pass.
+template <class S, class = void>
+struct HasPostAt : std::false_type {};
+template <class S>
+struct HasPostAt<S, std::void_t<decltype(&S::template post_at<1>)>> : std::true_type {};
+
 template <typename T, class Q, int TT, int I, bool BAR, typename W, class SRC, class DST>
 __device__ __forceinline__ void fixed_pass(const int t, const bool active,
                                            const W* __restrict__ tw, const SRC& src,
@@ -118,6 +124,16 @@ __device__ __forceinline__ void fixed_pass(const int t, const bool active,
             for (int j = 0; j < R; ++j) v[ib][j] = src.template at<nb>(b, j);
         }
     }
+    if constexpr (HasPostAt<SRC>::value) {
+#pragma unroll
+        for (int ib = 0; ib < MB; ++ib) {
+            const int b = t + ib * TT;
+            if (active && (full || b < nb)) {
+#pragma unroll
+                for (int j = 0; j < R; ++j) v[ib][j] = src.template post_at<nb>(b, j, v[ib][j]);
+            }
+        }
+    }
     if constexpr (BAR) __syncthreads();
 #pragma unroll
     for (int ib = 0; ib < MB; ++ib) {
@@ -138,14 +154,16 @@ __device__ __forceinline__ void fixed_pass(const int t, const bool active,
     }
 }
 
-// The passes of line Q from src through lds to dst.
-template <typename T, class Q, int TT, int I = 0, typename W, class SRC, class DST, class LDS>
+// The passes of line Q from src through lds to dst.  ALIAS: a line of one pass reads and writes
+// the same memory (a barrier between the two).
+template <typename T, class Q, int TT, int I = 0, bool ALIAS = false, typename W, class SRC,
+          class DST, class LDS>
 __device__ __forceinline__ void fixed_line(const int t, const bool active,
                                            const W* __restrict__ tw, const SRC& src,
                                            const DST& dst, const LDS& lds) {
     constexpr bool first = I == 0, last = I == Q::np - 1;
     if constexpr (first && last) {
-        fixed_pass<T, Q, TT, I, false>(t, active, tw, src, dst);
+        fixed_pass<T, Q, TT, I, ALIAS>(t, active, tw, src, dst);
     } else if constexpr (first) {
         fixed_pass<T, Q, TT, I, false>(t, active, tw, src, lds);
     } else if constexpr (last) {

@@ -165,6 +165,24 @@ struct FixedRow {
 // The fixed rows kernel of a radix sequence, nullptr where there is none.
 const FixedRow* find_fixed_row(Prec p, const PassTable& pt, int N);
 
+// Four-step passes of one line as compile-time constants (fixed_fs.h): Tt threads and elements
+// of `elem` LDS bytes per line (per pair of adjacent lines where width = 2; then in, out and the
+// distances must keep every pair aligned).  a.Ls: LDS elements per line (pair), at least
+// fixed_at(N - 1) + 1 with one pad element per 2^pad (pad < 0: none).
+struct FixedFs {
+    const int* r;
+    int np, N, Tt, max_threads, width, elem, pad;
+    hipError_t (*launch_a)(const void* in, void* out, const FourStepAArgs& a, const void* tw,
+                           hipStream_t st);
+    hipError_t (*launch_b)(const void* in, void* out, const FourStepBArgs& a, const void* tw,
+                           hipStream_t st);
+    void (*prepare)();
+};
+// F32Pair: two ComplexF32 lines per thread; F16Pair: the same with the plan's input (pass A) and
+// output (pass B) in ComplexF16.
+enum class FixedFsKind : int { F32 = 0, F64, F32Pair, F16Pair };
+const FixedFs* find_fixed_fs(FixedFsKind kind, const PassTable& pt, int N);
+
 // Sets per-kernel attributes (large LDS) once; called when a context is created.
 void init_kernels();
 

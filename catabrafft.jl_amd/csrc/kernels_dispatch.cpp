@@ -49,6 +49,16 @@ const FixedRow* find_fixed_row(Prec p, const PassTable& pt, int N) {
     }();
     return find_in(p == Prec::F32 ? f32 : f64, pt, N);
 }
+const FixedFs* find_fixed_fs(FixedFsKind kind, const PassTable& pt, int N) {
+    auto make = [](void (*fill)(std::vector<FixedFs>&)) {
+        std::vector<FixedFs> v;
+        fill(v);
+        return index_by_length(v);
+    };
+    static const std::unordered_multimap<int, FixedFs> m[4] = {
+        make(fixed_fs_f32), make(fixed_fs_f64), make(fixed_fs_pair), make(fixed_fs_f16)};
+    return find_in(m[(int)kind], pt, N);
+}
 
 hipError_t launch_rows_pipe(Prec p, const void* in, void* out, const RowsArgs& a,
                             const PassTable& pt, const void* tw, size_t twn, hipStream_t st) {

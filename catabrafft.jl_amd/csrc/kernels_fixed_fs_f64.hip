@@ -1,0 +1,15 @@
+// kernels_fixed_fs_f64.hip -- fixed four-step passes (fixed_fs.h) with T = double and lines stored
+// as double2.
+#include "fixed_fs.h"
+
+namespace cfft {
+#ifdef CFFT_EMU_LANES
+#define CFFT_LINES CFFT_FS_LINES_FEW
+#else
+#define CFFT_LINES CFFT_FS_LINES
+#endif
+#define CFFT_FS(...) rows.push_back(FixedFsOf<double, double2, Rad<__VA_ARGS__>>::entry());
+void fixed_fs_f64(std::vector<FixedFs>& rows) {
+    CFFT_LINES(CFFT_FS)
+}
+}  // namespace cfft

@@ -26,6 +26,11 @@ void fixed_rows_f32_0(std::vector<FixedRow>& rows);
 void fixed_rows_f32_1(std::vector<FixedRow>& rows);
 void fixed_rows_f64_0(std::vector<FixedRow>& rows);
 void fixed_rows_f64_1(std::vector<FixedRow>& rows);
+// The fixed four-step passes (fixed_fs.h).
+void fixed_fs_f32(std::vector<FixedFs>& rows);
+void fixed_fs_f64(std::vector<FixedFs>& rows);
+void fixed_fs_pair(std::vector<FixedFs>& rows);
+void fixed_fs_f16(std::vector<FixedFs>& rows);
 
 hipError_t real_rows_f32(const void* in, void* out, const RealArgs& a, const PassTable& pt,
                          const void* tw, int E, hipStream_t st);

@@ -536,6 +536,81 @@ static int fs_line_stride(Ctx* ctx, Prec pr, const LinePlan& lp, int C, size_t r
     return best;
 }
 
+// LDS line stride of a fixed four-step pass (FixedFs) with `cols` lines (line pairs) per
+// workgroup: the same model on its own layout.  One element is elem / 4 words (re, im together);
+// an access of the wave runs as groups of lanes that move 256 bytes, over 64 banks (weight 4;
+// tie-break: 128 bytes over 32).
+static int fixed_fs_stride(Ctx* ctx, const FixedFs& f, int cols, size_t reserve) {
+    static std::mutex mu;
+    static std::map<std::tuple<const FixedFs*, int, size_t>, int> cache;
+    const auto key = std::make_tuple(&f, cols, ctx->lds_max - std::min(ctx->lds_max, reserve));
+    {
+        std::lock_guard<std::mutex> g(mu);
+        auto it = cache.find(key);
+        if (it != cache.end()) return it->second;
+    }
+    const int ew = f.elem / 4, threads = cols * f.Tt;
+    auto at = [&f](int e) { return f.pad < 0 ? e : e + (e >> f.pad); };
+    const int base = at(f.N - 1) + 1;
+    int best = base, word[64], acc[64];
+    long best_cost = -1;
+    for (int Ls = base; Ls < base + 64; ++Ls) {
+        if ((size_t)f.elem * cols * Ls + reserve > ctx->lds_max) break;
+        long cost = 0;
+        auto over = [&] { return best_cost >= 0 && cost >= best_cost; };
+        int s = 1;
+        for (int ip = 0; ip < f.np && !over(); ++ip) {
+            const int R = f.r[ip], nb = f.N / R, MB = (nb + f.Tt - 1) / f.Tt;
+            for (int ib = 0; ib < MB && !over(); ++ib)
+                for (int j = 0; j < R && !over(); ++j)
+                    for (int wr = 0; wr < 2; ++wr) {
+                        if (wr ? ip + 1 == f.np : ip == 0) continue;  // global memory
+                        for (int L = 0; L < 64; ++L) {
+                            const int b = L / cols + ib * f.Tt;
+                            word[L] = -1;
+                            if (L >= threads || b >= nb) continue;
+                            const int p = b / s, q = b - p * s;
+                            word[L] = (L % cols * Ls + at(wr ? q + s * R * p + s * j : b + j * nb)) * ew;
+                        }
+                        for (int banks = 64; banks >= 32; banks /= 2)
+                            for (int L0 = 0; L0 < 64; L0 += banks / ew) {
+                                int n = 0;
+                                for (int L = L0; L < L0 + banks / ew; ++L)
+                                    for (int x = 0; word[L] >= 0 && x < ew; ++x) acc[n++] = word[L] + x;
+                                if (n) cost += (banks == 64 ? 4 : 1) * bank_cost(acc, n, banks);
+                            }
+                    }
+            s *= R;
+        }
+        if (best_cost < 0 || cost < best_cost) {
+            best_cost = cost;
+            best = Ls;
+        }
+    }
+    std::lock_guard<std::mutex> g(mu);
+    cache[key] = best;
+    return best;
+}
+
+// A fixed pass for a line (nullptr: none, or its tile does not fit): `C` lines per workgroup, a
+// power of two, halved until they fit the workgroup and the LDS beside `reserve` bytes.
+static const FixedFs* pick_fixed_fs(Ctx* ctx, FixedFsKind kind, const LinePlan& lp, size_t reserve,
+                                    int* C, int* Ls) {
+    const FixedFs* f = find_fixed_fs(kind, lp.pt, lp.N);
+    if (!f) return nullptr;
+    const size_t per = (size_t)f->elem * ((f->pad < 0 ? lp.N : lp.N + (lp.N >> f->pad)) + 64);
+    int c = *C / f->width;
+    auto fits = [&](int k) {
+        return k >= 1 && k * f->Tt <= f->max_threads && k * per + reserve <= ctx->lds_max;
+    };
+    while (c > 1 && !fits(c)) c /= 2;
+    if (!fits(c)) return nullptr;
+    *C = c * f->width;
+    *Ls = fixed_fs_stride(ctx, *f, c, reserve);
+    f->prepare();
+    return f;
+}
+
 static int pick_tile(Ctx* ctx, const LinePlan& lp, Prec pr, int want, size_t reserve = 0) {
     const size_t per = 2 * (size_t)(pr == Prec::F32 ? 4 : 8) * lp.Ls;
     const size_t room = ctx->lds_max > reserve + 16 ? ctx->lds_max - reserve - 16 : 0;
@@ -929,6 +1004,27 @@ static void fs_pipe_setup(Ctx* ctx, Plan& p, int mask) {
     }
 }
 
+// The passes' own kernels for a default four-step plan, at its tiles.
+static void fs_fixed_setup(Ctx* ctx, Plan& p) {
+    FourStepPlan& fs = p.fs;
+    const bool f64 = p.prec == Prec::F64, half = p.dtype == CFFT_C16;
+    auto kind = [&](int across) {  // `across`: lines side by side (the pairs' count is even)
+        if (f64) return FixedFsKind::F64;
+        if (half) return FixedFsKind::F16Pair;
+        return across % 2 ? FixedFsKind::F32 : FixedFsKind::F32Pair;
+    };
+    if (half && (fs.N1 % 2 || fs.N2 % 2)) return;
+    const size_t table = (size_t)tw3_entries(fs.tbits, fs.tnc) * esize(p.prec);
+    // Tiles (halved until they fit), timed over 13 lengths from 20,000 to 2^22 with pass A tiles of
+    // 4, 8, 16 and pass B tiles of 4 to 32 lines.  F32: pass A 4 (8 lines: 24,000 x 512 105.7 ->
+    // 116.9 us, 2^20 x 64 505 -> 556), pass B 16 (8 lines: 2^20 x 64 525, 4: 580).  F64: 8 and 16
+    // (4 and 4 lines: 20,000 x 512 145.6 -> 157.7 us, 2^18 x 128 453 -> 475, 2^17 x 64 123 -> 127).
+    fs.FCA = f64 ? 8 : 4;
+    fs.FCB = 16;
+    fs.fixed_a = pick_fixed_fs(ctx, kind(fs.N2), fs.a, 16, &fs.FCA, &fs.FLsA);
+    fs.fixed_b = pick_fixed_fs(ctx, kind(fs.N1), fs.b, table + 16, &fs.FCB, &fs.FLsB);
+}
+
 // Two lines per thread for the ComplexF32 four-step passes in `mask` (bit 0: A, bit 1: B) whose
 // tile holds an even number of lines of an even-length stride (N2 for A, N1 for B) and whose
 // pair layout fits the LDS.  The pair LDS line (C / 2 lines of 8-byte words) gets its own
@@ -1040,6 +1136,7 @@ static int plan_fft_core(Ctx* ctx, Plan& p, const PlanOptions& o) {
         const int pair = o.pair >= 0 ? o.pair
                                      : (p.prec != Prec::F32 ? 0 : (p.fs.a.E == 8 ? 3 : 1));
         if (pair > 0) fs_pair_setup(ctx, p, pair);
+        if (!o.E && !o.Eb && o.pair < 0 && !pipe_mask && chunk == 0) fs_fixed_setup(ctx, p);
         return CFFT_OK;
     }
     return plan_conv(ctx, p, o);
@@ -1072,6 +1169,8 @@ static std::string describe(const Plan& p) {
                << " Ls=" << p.fs.a.Ls << " N2=" << p.fs.N2 << " " << rad(p.fs.b)
                << " CB=" << p.fs.CB << " Ls=" << p.fs.b.Ls;
             if (p.fs.chunk) os << " chunk=" << p.fs.chunk;
+            if (p.fs.fixed_a || p.fs.fixed_b)
+                os << " fixed=" << (p.fs.fixed_a ? "A" : "") << (p.fs.fixed_b ? "B" : "");
             if (p.fs.pipe_a || p.fs.pipe_b)
                 os << " pipe=" << (p.fs.pipe_a ? "A" : "") << (p.fs.pipe_b ? "B" : "");
             if (p.fs.pair_a || p.fs.pair_b)
@@ -1140,7 +1239,15 @@ static int run_fourstep(const Plan& p, const void* in, void* mid, void* out, int
         a.mid_plain = fs.chunk > 0;  // a chunk's middle is read back while still cached
         const int64_t es_ = esize(p.prec);
         auto al16 = [](const void* q) { return ((uintptr_t)q & 15) == 0; };
-        if (p.half) {
+        // a fixed pass's pairs of adjacent lines are 2 * eio (es in the middle) bytes apart
+        auto fits = [](const FixedFs* f, const void* q, int64_t dist, size_t elem) {
+            return f->width == 1 || (((uintptr_t)q & (2 * elem - 1)) == 0 && dist % 2 == 0);
+        };
+        if (fs.fixed_a && fits(fs.fixed_a, inb, idist, eio)) {
+            a.C = fs.FCA;
+            a.Ls = fs.FLsA;
+            CFFT_HIP(fs.fixed_a->launch_a(inb, midb, a, fs.a.dtw.p, st));
+        } else if (p.half) {
             CFFT_HIP(launch_fourstep_a_f16(inb, midb, a, fs.a.pt, fs.a.dtw.p, st));
         } else if (fs.pair_a && al16(inb) && al16(midb) && idist % 2 == 0 && mdist % 2 == 0) {
             a.Ls = fs.LsA2;
@@ -1171,7 +1278,12 @@ static int run_fourstep(const Plan& p, const void* in, void* mid, void* out, int
         b.tnc = fs.tnc;
         b.tw3 = fs.tw3.p;
         b.xcd = 1;
-        if (p.half) {
+        if (fs.fixed_b && !epi.K && fits(fs.fixed_b, midb, mdist, es) &&
+            fits(fs.fixed_b, outb, odist, eio)) {
+            b.C = fs.FCB;
+            b.Ls = fs.FLsB;
+            CFFT_HIP(fs.fixed_b->launch_b(midb, outb, b, fs.b.dtw.p, st));
+        } else if (p.half) {
             CFFT_HIP(launch_fourstep_b_f16(midb, outb, b, fs.b.pt, fs.b.dtw.p, st));
         } else if (fs.pair_b && !epi.K && al16(midb) && al16(outb) && mdist % 2 == 0 &&
                    odist % 2 == 0) {
@@ -1328,6 +1440,13 @@ static int run_fft_s(const Plan& p, const void* in, void* out, int sgn, double s
             b.scale = scale;
             b.epi = epi;
             b.xcd = 1;
+            const FixedFs* f = p.fs.fixed_b;
+            if (f && (f->width == 1 || ((((uintptr_t)in | (uintptr_t)out) & 15) == 0))) {
+                b.C = p.fs.FCB;
+                b.Ls = p.fs.FLsB;
+                CFFT_HIP(f->launch_b(in, out, b, p.fs.b.dtw.p, st));
+                return CFFT_OK;
+            }
             CFFT_HIP(launch_fourstep_b(p.prec, in, out, b, p.fs.b.pt, p.fs.b.dtw.p, st));
             return CFFT_OK;
         }
@@ -1639,11 +1758,24 @@ int plan_nd_create(Ctx* ctx, int rank, const int64_t* dims, int64_t axes_mask, i
             s->idist = s->odist = inner * N2;
             s->fs.N1 = (int)inner;
             s->fs.N2 = (int)N2;
-            if ((rc = make_line(s->fs.b, N2, p->prec, 16, 1024))) return rc;
+            // lines of 128 and 256 points in three light passes instead of two with a radix 16
+            // (which holds twice the registers): 256^3 F32 144.5 -> 135.5 us
+            std::vector<int> rad = fourstep_line_radices(N2);
+            if (N2 == 128) rad = {2, 8, 8};
+            if (N2 == 256) rad = {4, 8, 8};
+            if ((rc = make_line(s->fs.b, N2, p->prec, 16, 1024, &rad))) return rc;
             s->fs.CB = pick_tile(ctx, s->fs.b, p->prec, p->prec == Prec::F32 ? 16 : 8);
             s->fs.b.Ls = fs_line_stride(ctx, p->prec, s->fs.b, s->fs.CB, 16);
+            // its own kernel where the block's byte offsets fit 32 bits
+            if (inner * N2 * esize(p->prec) < ((int64_t)1 << 32)) {
+                s->fs.FCB = p->prec == Prec::F32 ? 16 : 8;
+                s->fs.fixed_b = pick_fixed_fs(ctx, p->prec == Prec::F64 ? FixedFsKind::F64
+                                                   : inner % 2          ? FixedFsKind::F32
+                                                                        : FixedFsKind::F32Pair,
+                                              s->fs.b, 16, &s->fs.FCB, &s->fs.FLsB);
+            }
             os << " | axis " << a << ": strided lines N=" << N2 << " x " << inner << " C="
-               << s->fs.CB;
+               << (s->fs.fixed_b ? s->fs.FCB : s->fs.CB) << (s->fs.fixed_b ? " fixed" : "");
         }
         p->parts.push_back(std::move(s));
     }

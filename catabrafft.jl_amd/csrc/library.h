@@ -48,6 +48,10 @@ struct FourStepPlan {
     // of a line pair; a call whose addresses or distances are not 16-byte aligned runs the float
     // kernels on the same tiles
     int pair_a = 0, pair_b = 0, LsA2 = 0, LsB2 = 0;
+    // the passes' own kernels, their tiles and LDS line strides (nullptr: the run-time kernels,
+    // which also run where a pair kernel's alignment is not met)
+    const FixedFs *fixed_a = nullptr, *fixed_b = nullptr;
+    int FCA = 1, FCB = 1, FLsA = 0, FLsB = 0;
     int64_t chunk = 0;  // transforms per pass-A/pass-B round (0 = the whole batch)
 };
 
@@ -65,12 +69,12 @@ struct Plan {
     LinePlan line;
     int C = 1;
     int pipe_res = 0;  // direct: resident workgroups of the pipelined rows kernel (0 = not used)
+    const FixedRow* fixed = nullptr;  // direct: the line's own rows kernel, fixed_c lines per
+    int fixed_c = 1;                  // workgroup (nullptr: the run-time rows kernel)
     // four-step
     FourStepPlan fs;
     mutable std::mutex scratch_mu;
     mutable DevBuf scratch;
-    const FixedRow* fixed = nullptr;  // direct: the line's own rows kernel, fixed_c lines per
-    int fixed_c = 1;                  // workgroup (nullptr: the run-time rows kernel)
     // Executions that use the plan's own work buffers are ordered on the device: each waits for
     // work_ev (recorded by the previous one, on whatever stream) before it starts.
     mutable std::mutex exec_mu;

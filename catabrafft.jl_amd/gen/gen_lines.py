@@ -5,7 +5,8 @@
 
 A line is a length and its radix sequence, the one the planner takes by default for that length
 (line_radices in library.cpp).  The rows kernels cover every 7-smooth length from 16 to 8192: the
-lengths a workgroup holds in both precisions.  The lists are split in parts so that several
+lengths a workgroup holds in both precisions.  The four-step passes cover every 7-smooth length
+from 16 to 2048, and 4096: the factors of the lengths up to 2^22 and of 2^24.  The lists are split in parts so that several
 translation units compile them in parallel; the _FEW list is the part that the CPU emulation
 build of the tests compiles.
 """
@@ -37,6 +38,17 @@ def line_radices(n):
     return sorted(r, reverse=True)
 
 
+def fourstep_radices(n):
+    """Powers of two: the fewest passes, the bits spread evenly, smallest radix first; others as
+    line_radices (fourstep_line_radices in library.cpp)."""
+    if n & (n - 1):
+        return line_radices(n)
+    k = n.bit_length() - 1
+    passes = (k + 3) // 4
+    base, extra = divmod(k, passes)
+    return [1 << (base + (i >= passes - extra)) for i in range(passes)]
+
+
 def macro(name, lines):
     out = [f"#define {name}(X) \\"]
     out += [f"    X({', '.join(map(str, r))}) \\" for r in lines]
@@ -56,9 +68,14 @@ def main():
     ]
     for k in range(PARTS):
         parts.append(macro(f"CFFT_ROW_LINES_{k}", rows[k::PARTS]))
+    fs = [fourstep_radices(n) for n in list(range(16, 2049)) + [4096] if line_radices(n)]
+    fs += [[2, 8, 8], [4, 8, 8]]  # the strided axes of N-D transforms: no radix 16
+    parts.append(macro("CFFT_FS_LINES_FEW", [r for i, r in enumerate(fs) if i % 16 == 3]
+                       + [fourstep_radices(n) for n in (16, 128, 256, 1024)] + fs[-2:]))
+    parts.append(macro("CFFT_FS_LINES", fs))
     with open(out, "w") as f:
         f.write("\n".join(parts) + "\n")
-    print(f"wrote {os.path.normpath(out)}: {len(rows)} row lines")
+    print(f"wrote {os.path.normpath(out)}: {len(rows)} row lines, {len(fs)} four-step lines")
 
 
 if __name__ == "__main__":

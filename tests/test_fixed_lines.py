@@ -19,12 +19,12 @@ TABLE = os.path.join(ROOT, "catabrafft.jl_amd", "csrc", "fixed_table.h")
 
 
 def _lengths(prefix):
-    """The lengths of the lists whose macro name starts with prefix."""
+    """The lengths of the lists whose macro name is prefix or prefix with a part number."""
     out, on = set(), False
     with open(TABLE) as f:
         for line in f:
             if line.startswith("#define"):
-                on = line.split()[1].startswith(prefix)
+                on = line.split()[1].split("(")[0] == prefix
             m = re.match(r"\s+X\(([\d, ]+)\)", line)
             if on and m:
                 out.add(int(np.prod([int(v) for v in m.group(1).split(",")])))
@@ -118,3 +118,71 @@ def test_fixed_rows_match_the_run_time_kernel(gpu_ready, tmp_path, dt):
         err = float((z - ref).norm() / ref.norm())
         # four roundings of eps / 2 a pass and one for the table, as in the parity tests
         assert err < (1e-6 if code == 0 else 4 * np.finfo(float).eps * np.log2(n)), (n, err)
+
+
+# ------------------------------------------------------------------------------ four-step passes
+FS_FEW = _lengths("CFFT_FS_LINES_FEW")
+FS_ALL = _lengths("CFFT_FS_LINES")
+FORCED = "16 64 {n1} 2 2 -1 0 0 pr=0"  # the run-time kernels, one line per thread
+OWN = "0 64 {n1} 0 0 -1 -1 0"          # the lines' own kernels, at their tiles
+
+
+def _emu_four_step(emu, tmp_path, n1, n2, batch, dt, fields, dist, shift):
+    """A four-step of n1 x n2 in the emulation, its rows `dist` apart and its buffers `shift`
+    elements past a 16-byte boundary: forward out of place, inverse in place."""
+    n, code = n1 * n2, (0 if dt == np.complex64 else 1)
+    w = tmp_path / "w.txt"
+    w.write_text(f"{n} {batch} {dist} {dist} {code} 1 : {fields.format(n1=n1)}\n")
+    ctx, p = ctypes.c_void_p(), ctypes.c_void_p()
+    assert emu.cfft_init(0, ctypes.byref(ctx)) == 0
+    assert emu.cfft_wisdom_import(ctx, str(w).encode()) == 0
+    assert emu.cfft_plan_1d(ctx, n, batch, dist, dist, code, 1, ctypes.byref(p)) == 0
+    x = np.zeros(batch * dist + 2, dtype=dt)[shift:][:batch * dist]
+    x[:] = seeded_complex(batch * dist, seed=n, dtype=dt)
+    y = np.zeros(batch * dist + 2, dtype=dt)[shift:][:batch * dist]
+    assert emu.cfft_exec(p, x.ctypes.data, y.ctypes.data, -1, 0, None) == 0
+    assert emu.cfft_exec(p, x.ctypes.data, x.ctypes.data, 1, 1, None) == 0
+    d = _desc(emu, p)
+    emu.cfft_plan_destroy(p)
+    emu.cfft_finalize(ctx)
+    return d, y, x
+
+
+@pytest.mark.parametrize("dt", [np.complex64, np.complex128])
+@pytest.mark.parametrize("n2", [16, 35])  # an even and an odd number of lines side by side
+@pytest.mark.parametrize("n1", FS_FEW)
+def test_emulated_fixed_four_step_matches_the_run_time_kernels(emu, tmp_path, n1, n2, dt):
+    for a, b, dist, shift in ((n1, n2, n1 * n2, 0), (n2, n1, n1 * n2 + 1, 1)):
+        if n2 == 35 and n2 not in FS_FEW and a == n2:
+            continue
+        d0, y0, x0 = _emu_four_step(emu, tmp_path, a, b, 3, dt, FORCED, dist, shift)
+        d1, y1, x1 = _emu_four_step(emu, tmp_path, a, b, 3, dt, OWN, dist, shift)
+        assert "fixed" not in d0 and "fixed=" in d1, (d0, d1)
+        assert np.array_equal(y0, y1) and np.array_equal(x0, x1), (a, b, dist)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [np.complex64, np.complex128])
+def test_fixed_four_step_matches_the_run_time_kernels(gpu_ready, tmp_path, dt):
+    import torch
+
+    import catabrafft as C
+
+    code, batch = (0 if dt == np.complex64 else 1), 2
+    for line in FS_ALL:
+        for n1, n2 in ((line, 16), (48, line), (line, 15)):
+            n = n1 * n2
+            got = []
+            for fields in (FORCED, OWN):
+                w = tmp_path / "w.txt"
+                w.write_text(f"{n} {batch} {n} {n} {code} 1 : {fields.format(n1=n1)}\n")
+                C.import_wisdom(str(w))
+                p = C.Plan(n, batch, dt, flags=C.MEASURE)
+                print(f"{np.dtype(dt)} {p.describe()}", flush=True)
+                own = "A" if n2 == 15 else "AB"
+                assert ("fixed=" + own in p.describe()) == (fields is OWN), p.describe()
+                x = torch.from_numpy(seeded_complex(n, batch=batch, seed=n, dtype=dt)).cuda()
+                y = p.exec_torch(x, direction=1, normalize=True)
+                p.exec_torch(x, x)
+                got.append((torch.view_as_real(y), torch.view_as_real(x)))
+            assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]), (n1, n2)
