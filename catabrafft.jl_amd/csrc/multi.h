@@ -82,6 +82,8 @@ struct MultiLaunch {
     const MItem* items;  // device table
     int64_t nitems;
     const MPlan* plans;  // device table
+    int phase;           // launches of a lower phase come first
+    double cost;         // estimated time, us
 };
 
 enum class MultiKernel : int {

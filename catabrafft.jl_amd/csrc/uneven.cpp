@@ -493,9 +493,15 @@ int WorkList::finalize(DevBuf& dplans, DevBuf& ditems, DevBuf& dtable,
     const size_t bt = std::max<size_t>(1, table_.size()) * sizeof(uint64_t);
     const size_t bi = std::max<size_t>(1, nitems) * sizeof(MItem);
     // grow with headroom, so that buffers reused round after round are rarely reallocated
-    if (dplans.bytes < bp && (rc = dplans.alloc(bp + bp / 2))) return rc;
-    if (dtable.bytes < bt && (rc = dtable.alloc(bt + bt / 2))) return rc;
-    if (ditems.bytes < bi && (rc = ditems.alloc(bi + bi / 2))) return rc;
+    // (a staged upload puts the three tables into dplans, one copy)
+    const bool staged = async && stage;
+    const size_t ot = (bp + 255) & ~(size_t)255, oi = (ot + bt + 255) & ~(size_t)255;
+    const size_t need = staged ? oi + bi : bp;
+    if (dplans.bytes < need && (rc = dplans.alloc(need + need / 2))) return rc;
+    if (!staged && dtable.bytes < bt && (rc = dtable.alloc(bt + bt / 2))) return rc;
+    if (!staged && ditems.bytes < bi && (rc = ditems.alloc(bi + bi / 2))) return rc;
+    unsigned char* const table_at = staged ? (unsigned char*)dplans.p + ot : (unsigned char*)dtable.p;
+    unsigned char* const items_at = staged ? (unsigned char*)dplans.p + oi : (unsigned char*)ditems.p;
     std::vector<MItem> all;
     all.reserve(nitems);
     for (const Group* g : gs) {
@@ -518,25 +524,39 @@ int WorkList::finalize(DevBuf& dplans, DevBuf& ditems, DevBuf& dtable,
         L.cprec = g->cprec;
         L.block = g->block;
         L.lds = g->lds;
-        L.items = reinterpret_cast<const MItem*>(ditems.p) + all.size();
+        L.items = reinterpret_cast<const MItem*>(items_at) + all.size();
         L.nitems = (int64_t)order.size();
         L.plans = reinterpret_cast<const MPlan*>(dplans.p);
+        L.phase = g->phase;
+        // microseconds, roughly: the longest item alone (1.5e-4 per unit of its cost on MI355X: a
+        // rows item of 8192 points 22 us, a convolution of 8190 points 55), then the rest of the
+        // items on about 400 resident workgroups
+        double total = 0, longest = 0;
+        for (size_t k = 0; k < g->runs.size(); ++k) {
+            const size_t end = k + 1 < g->runs.size() ? g->runs[k + 1].second : g->items.size();
+            total += g->runs[k].first * (double)(end - g->runs[k].second);
+            longest = std::max(longest, g->runs[k].first);
+        }
+        L.cost = 1.5e-4 * (longest + total / 400) * (g->cprec == (int)Prec::F64 ? 1.5 : 1.0);
         for (size_t k : order) {
             MItem it = g->items[k];
-            if (it.flags & kLineTable) it.aux += (uint64_t)dtable.p;
+            if (it.flags & kLineTable) it.aux += (uint64_t)table_at;
             all.push_back(it);
         }
         out.push_back(L);
     }
+    if (staged) {
+        if (stage->reserve(need)) return fail(CFFT_ERR_NOMEM, "pinned staging failed");
+        unsigned char* h = static_cast<unsigned char*>(stage->p);
+        std::memcpy(h, mplans_.data(), bp);
+        if (!table_.empty()) std::memcpy(h + ot, table_.data(), table_.size() * 8);
+        if (!all.empty()) std::memcpy(h + oi, all.data(), all.size() * sizeof(MItem));
+        CFFT_HIP(hipMemcpyAsync(dplans.p, h, need, hipMemcpyHostToDevice, st));
+        return CFFT_OK;
+    }
     if (async) {
-        unsigned char* h;
-        if (stage) {
-            if (stage->reserve(bp + bt + bi)) return fail(CFFT_ERR_NOMEM, "pinned staging failed");
-            h = static_cast<unsigned char*>(stage->p);
-        } else {
-            host_.resize(bp + bt + bi);
-            h = host_.data();
-        }
+        host_.resize(bp + bt + bi);
+        unsigned char* h = host_.data();
         std::memcpy(h, mplans_.data(), bp);
         if (!table_.empty()) std::memcpy(h + bp, table_.data(), table_.size() * 8);
         if (!all.empty()) std::memcpy(h + bp + bt, all.data(), all.size() * sizeof(MItem));
@@ -554,11 +574,18 @@ int WorkList::finalize(DevBuf& dplans, DevBuf& ditems, DevBuf& dtable,
 }
 
 // ----------------------------------------------------------------------------- uneven plans
+// Branches of the captured graph besides the main one.  Small launches do not fill the GPU, and a
+// launch that runs alone costs the latency of its longest item (20-50 us): independent ones run side
+// by side (1000 transforms of 64 to 2^18 points: 1250 -> 1118 us).
+constexpr int kCaptureSides = 3;
+
 struct UnevenState {
     std::vector<std::unique_ptr<Plan>> plans;
     DevBuf dplans, ditems, dtable, work;
     std::vector<MultiLaunch> launches;
     hipStream_t cap = nullptr;
+    hipStream_t side[kCaptureSides] = {};
+    hipEvent_t fork = nullptr, join[kCaptureSides] = {};
     std::mutex mu;
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
@@ -571,11 +598,65 @@ struct UnevenState {
         if (gexec) (void)hipGraphExecDestroy(gexec);
         if (graph) (void)hipGraphDestroy(graph);
         if (cap) (void)hipStreamDestroy(cap);
+        if (fork) (void)hipEventDestroy(fork);
+        for (int i = 0; i < kCaptureSides; ++i) {
+            if (side[i]) (void)hipStreamDestroy(side[i]);
+            if (join[i]) (void)hipEventDestroy(join[i]);
+        }
     }
 };
 
 static int run_launches(const std::vector<MultiLaunch>& ls, const MultiArgs& ma, hipStream_t st) {
     for (const MultiLaunch& L : ls) CFFT_HIP(launch_multi(L, ma, st));
+    return CFFT_OK;
+}
+
+// The launches as branches of the capture on st->cap.  A chain (the two four-step passes, the three
+// launches of the large convolutions, per precision) stays in order on one branch; rows and fused
+// convolutions are chains of one launch.  The unfused large convolutions share their phases' four-
+// step launches with the four-step plans: lists that hold them run in one branch.
+static int capture_launches(UnevenState& st, const MultiArgs& ma) {
+    std::map<int, std::vector<const MultiLaunch*>> chains;
+    std::map<int, double> cost;
+    int single = 0;
+    for (const MultiLaunch& L : st.launches) {
+        int key;
+        switch ((MultiKernel)L.kernel) {
+            case MultiKernel::Gather:
+            case MultiKernel::Scatter: return run_launches(st.launches, ma, st.cap);
+            case MultiKernel::FourStepA:
+            case MultiKernel::FourStepB: key = -1 - L.prec; break;
+            case MultiKernel::ConvLA:
+            case MultiKernel::ConvLBA:
+            case MultiKernel::ConvLC: key = -10 - 2 * L.prec - L.cprec; break;
+            default: key = single++;
+        }
+        chains[key].push_back(&L);
+        cost[key] += L.cost;
+    }
+    std::vector<int> order;
+    for (const auto& c : chains) order.push_back(c.first);
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cost[a] > cost[b]; });
+    double load[kCaptureSides + 1] = {};
+    bool forked[kCaptureSides] = {};
+    CFFT_HIP(hipEventRecord(st.fork, st.cap));
+    for (int key : order) {
+        int k = 0;
+        for (int i = 1; i <= kCaptureSides; ++i)
+            if (load[i] < load[k]) k = i;
+        load[k] += cost[key];
+        hipStream_t s = k ? st.side[k - 1] : st.cap;
+        if (k && !forked[k - 1]) {
+            CFFT_HIP(hipStreamWaitEvent(s, st.fork, 0));
+            forked[k - 1] = true;
+        }
+        for (const MultiLaunch* L : chains[key]) CFFT_HIP(launch_multi(*L, ma, s));
+    }
+    for (int i = 0; i < kCaptureSides; ++i) {
+        if (!forked[i]) continue;
+        CFFT_HIP(hipEventRecord(st.join[i], st.side[i]));
+        CFFT_HIP(hipStreamWaitEvent(st.cap, st.join[i], 0));
+    }
     return CFFT_OK;
 }
 
@@ -742,6 +823,11 @@ int uneven_create(Ctx* ctx, int64_t count, const int64_t* lengths, const int64_t
     }
     if ((rc = W.finalize(st->dplans, st->ditems, st->dtable, st->launches))) return rc;
     CFFT_HIP(hipStreamCreateWithFlags(&st->cap, hipStreamNonBlocking));
+    CFFT_HIP(hipEventCreateWithFlags(&st->fork, hipEventDisableTiming));
+    for (int i = 0; i < kCaptureSides; ++i) {
+        CFFT_HIP(hipStreamCreateWithFlags(&st->side[i], hipStreamNonBlocking));
+        CFFT_HIP(hipEventCreateWithFlags(&st->join[i], hipEventDisableTiming));
+    }
     size_t bytes = st->dplans.bytes + st->ditems.bytes + st->dtable.bytes + st->work.bytes;
     for (auto& p : st->plans) bytes += plan_device_bytes(*p);
     P->uneven_bytes = bytes;
@@ -772,7 +858,7 @@ int uneven_exec(const Plan& p, const void* in, void* out, int direction, int nor
         st->gexec = nullptr;
         st->graph = nullptr;
         CFFT_HIP(hipStreamBeginCapture(st->cap, hipStreamCaptureModeThreadLocal));
-        int rc = run_launches(st->launches, ma, st->cap);
+        int rc = capture_launches(*st, ma);
         hipGraph_t graph = nullptr;
         const hipError_t e = hipStreamEndCapture(st->cap, &graph);
         if (rc) {

@@ -45,6 +45,7 @@ static void entry(int idx) {
 struct Stream {
     bool capturing = false;
     std::vector<std::function<void()>>* graph = nullptr;
+    std::vector<Stream*> joined;  // capturing: the streams that joined this one's capture
 };
 
 static void run_block(const std::function<void()>& body, unsigned nthreads) {
@@ -119,6 +120,7 @@ int cfft_emu_lane_xor(int v, int d) {
 
 struct emu_event {
     double t = 0;
+    emu::Stream* capturing = nullptr;  // the stream it was last recorded on, if that captured
 };
 struct emu_graph {
     std::vector<std::function<void()>> ops;
@@ -181,7 +183,19 @@ hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t* e) { *e = new emu_event(); return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCreate(e); }
 hipError_t hipEventDestroy(hipEvent_t e) { delete e; return hipSuccess; }
-hipError_t hipEventRecord(hipEvent_t e, hipStream_t) { e->t = now_ms(); return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+    e->t = now_ms();
+    e->capturing = s && s->capturing ? s : nullptr;
+    return hipSuccess;
+}
+hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
+    if (s && !s->capturing && e->capturing && e->capturing->capturing) {
+        s->capturing = true;
+        s->graph = e->capturing->graph;
+        e->capturing->joined.push_back(s);
+    }
+    return hipSuccess;
+}
 hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b) { *ms = (float)(b->t - a->t); return hipSuccess; }
@@ -197,6 +211,11 @@ hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t* g) {
     delete s->graph;
     s->graph = nullptr;
     s->capturing = false;
+    for (emu::Stream* j : s->joined) {
+        j->graph = nullptr;
+        j->capturing = false;
+    }
+    s->joined.clear();
     return hipSuccess;
 }
 hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t g, hipGraphNode_t*, char*, size_t) {
