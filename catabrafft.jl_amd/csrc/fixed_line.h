@@ -84,6 +84,13 @@ struct FixedLds {
     __device__ __forceinline__ void put_at(int e, int k, V v) const { p[fixed_at<SH, STEP>(e, k)] = v; }
 };
 
+// A destination may load ahead what its stores need (HasPrepAt): prep_at<STEP>(e, k) before the
+// butterflies, handed back to put_at.
+template <class D, class = void>
+struct HasPrepAt : std::false_type {};
+template <class D>
+struct HasPrepAt<D, std::void_t<typename D::Prep>> : std::true_type {};
+
 // Pass I of line Q with TT threads: src.at<STEP>(e, j) is element e + j STEP of its input,
 // dst.put_at<STEP>(e, k, v) stores element e + k STEP of its output.  BAR: a barrier between the
 // reads and the writes (both go to the same LDS).  Twiddles load first, and a source's post_at
@@ -139,17 +146,36 @@ __device__ __forceinline__ void fixed_pass(const int t, const bool active,
     for (int ib = 0; ib < MB; ++ib) {
         const int b = t + ib * TT;
         if (active && (full || b < nb)) {
-            Dft<R>::run(v[ib]);
             const int p = (int)((unsigned)b / s), q = b - p * s;
-            if constexpr (twiddled) {
+            if constexpr (HasPrepAt<DST>::value) {
+                static_assert(!twiddled, "a last pass");
+                // (8 at a time: a radix 16 would hold as many registers again)
+                constexpr int H = R <= 8 ? R : 8;
+                typename DST::Prep pr[H];
 #pragma unroll
-                for (int k = 1; k <= KP; ++k) v[ib][k] = cmul(v[ib][k], w[ib][k - 1]);
+                for (int k = 0; k < H; ++k) pr[k] = dst.template prep_at<s>(q + s * R * p, k);
+                Dft<R>::run(v[ib]);
 #pragma unroll
-                for (int k = KP + 1; k < R; ++k) v[ib][k] = cmul(v[ib][k], tp[p * (R - 1) + k - 1]);
+                for (int k = 0; k < H; ++k)
+                    dst.template put_at<s>(q + s * R * p, k, v[ib][k], pr[k]);
+#pragma unroll
+                for (int k = H; k < R; ++k) pr[k - H] = dst.template prep_at<s>(q + s * R * p, k);
+#pragma unroll
+                for (int k = H; k < R; ++k)
+                    dst.template put_at<s>(q + s * R * p, k, v[ib][k], pr[k - H]);
+            } else {
+                Dft<R>::run(v[ib]);
+                if constexpr (twiddled) {
+#pragma unroll
+                    for (int k = 1; k <= KP; ++k) v[ib][k] = cmul(v[ib][k], w[ib][k - 1]);
+#pragma unroll
+                    for (int k = KP + 1; k < R; ++k)
+                        v[ib][k] = cmul(v[ib][k], tp[p * (R - 1) + k - 1]);
+                }
+                const int base = q + s * R * p;
+#pragma unroll
+                for (int k = 0; k < R; ++k) dst.template put_at<s>(base, k, v[ib][k]);
             }
-            const int base = q + s * R * p;
-#pragma unroll
-            for (int k = 0; k < R; ++k) dst.template put_at<s>(base, k, v[ib][k]);
         }
     }
 }

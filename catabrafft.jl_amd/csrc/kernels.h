@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <vector>
 
 #include "engine.h"
 
@@ -182,6 +183,38 @@ struct FixedFs {
 // output (pass B) in ComplexF16.
 enum class FixedFsKind : int { F32 = 0, F64, F32Pair, F16Pair };
 const FixedFs* find_fixed_fs(FixedFsKind kind, const PassTable& pt, int N);
+
+// Fused convolution over a length N whose radices are compile-time constants (fixed_conv.h), its
+// spectrum in the order of conv_order: Tt threads per line, a.C lines per workgroup of at most
+// max_threads; a.Ls LDS elements per line, at least fixed_at(max(n, N) - 1) + 1 with one pad element
+// per 2^pad (pad < 0: none), and one slot.
+struct FixedConv {
+    const int* r;
+    int np, N, Tt, pad, max_threads;
+    hipError_t (*launch)(const void* in, void* out, const ConvSmallArgs& a, const void* tw,
+                         hipStream_t st);
+    void (*prepare)();
+};
+// The fixed convolution of the shortest length N >= m (exact: N == m), nullptr where there is none.
+const FixedConv* find_fixed_conv(Prec p, int64_t m, bool exact);
+
+// The three launches of a large convolution (ConvLArgs) on lines of N points whose radices are
+// compile-time constants (fixed_convl.h): A runs lines of radices r, Tt threads and LDS padding
+// pad, at most max_a threads a workgroup; BA (in place, padding pad_b) and C (pad_c) lines of
+// radices rb, Tb threads, max_b.  A plan uses A and C of its N1 and BA of its N2; its tables are in
+// their order.
+struct FixedConvL {
+    const int *r, *rb;
+    int np, N, Tt, Tb, pad, pad_b, pad_c, max_a, max_b;
+    hipError_t (*launch_a)(const void* x, const ConvLArgs& a, const void* tw, hipStream_t st);
+    hipError_t (*launch_ba)(const ConvLArgs& a, const void* tw, hipStream_t st);
+    hipError_t (*launch_c)(void* y, const ConvLArgs& a, const void* tw, hipStream_t st);
+    void (*prepare)();
+};
+// pio: precision of x and y, pc: precision of the convolution.
+const FixedConvL* find_fixed_convl(Prec pio, Prec pc, int64_t N);
+// Every length of the lines, ascending.
+const std::vector<int>& fixed_convl_lengths();
 
 // Sets per-kernel attributes (large LDS) once; called when a context is created.
 void init_kernels();

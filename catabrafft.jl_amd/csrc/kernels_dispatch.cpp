@@ -17,6 +17,11 @@ void init_kernels() {
     init_kernels_f16();
     init_kernels_pipe_f32();
     init_kernels_pipe_f64();
+    init_kernels_fixed_convl_multi_f32_f32();
+    init_kernels_fixed_convl_multi_f32_f64();
+    init_kernels_fixed_convl_multi_f64_f64();
+    init_kernels_fixed_conv_multi_f32();
+    init_kernels_fixed_conv_multi_f64();
 }
 
 // Fixed kernels by length; each index is built at its first look-up.
@@ -58,6 +63,47 @@ const FixedFs* find_fixed_fs(FixedFsKind kind, const PassTable& pt, int N) {
     static const std::unordered_multimap<int, FixedFs> m[4] = {
         make(fixed_fs_f32), make(fixed_fs_f64), make(fixed_fs_pair), make(fixed_fs_f16)};
     return find_in(m[(int)kind], pt, N);
+}
+
+const FixedConv* find_fixed_conv(Prec p, int64_t m, bool exact) {
+    auto make = [](void (*fill)(std::vector<FixedConv>&)) {
+        std::vector<FixedConv> v;
+        fill(v);
+        std::sort(v.begin(), v.end(),
+                  [](const FixedConv& a, const FixedConv& b) { return a.N < b.N; });
+        return v;
+    };
+    static const std::vector<FixedConv> t[2] = {make(fixed_conv_f32), make(fixed_conv_f64)};
+    const auto& v = t[p == Prec::F64];
+    const auto it = std::lower_bound(v.begin(), v.end(), m,
+                                     [](const FixedConv& a, int64_t x) { return a.N < x; });
+    return it == v.end() || (exact && it->N != m) ? nullptr : &*it;
+}
+
+static const std::vector<FixedConvL>& convl_rows(Prec pio, Prec pc) {
+    auto make = [](void (*fill)(std::vector<FixedConvL>&)) {
+        std::vector<FixedConvL> v;
+        fill(v);
+        std::sort(v.begin(), v.end(),
+                  [](const FixedConvL& a, const FixedConvL& b) { return a.N < b.N; });
+        return v;
+    };
+    static const std::vector<FixedConvL> t[3] = {
+        make(fixed_convl_f32_f32), make(fixed_convl_f32_f64), make(fixed_convl_f64_f64)};
+    return t[pio == Prec::F64 ? 2 : pc == Prec::F64 ? 1 : 0];
+}
+const FixedConvL* find_fixed_convl(Prec pio, Prec pc, int64_t N) {
+    for (const FixedConvL& f : convl_rows(pio, pc))
+        if (f.N == N) return &f;
+    return nullptr;
+}
+const std::vector<int>& fixed_convl_lengths() {
+    static const std::vector<int> v = [] {
+        std::vector<int> n;
+        for (const FixedConvL& f : convl_rows(Prec::F32, Prec::F32)) n.push_back(f.N);
+        return n;
+    }();
+    return v;
 }
 
 hipError_t launch_rows_pipe(Prec p, const void* in, void* out, const RowsArgs& a,
@@ -187,6 +233,14 @@ hipError_t launch_multi(const MultiLaunch& L, const MultiArgs& ma, hipStream_t s
                                              : gs_multi_f32_f64(L, ma, st);
         return gs_multi_f64_f64(L, ma, st);
     }
+    if (k == MultiKernel::ConvFA || k == MultiKernel::ConvFBA || k == MultiKernel::ConvFC) {
+        if (L.prec == (int)Prec::F64) return convl_fixed_multi_f64_f64(L, ma, st);
+        return L.cprec == (int)Prec::F64 ? convl_fixed_multi_f32_f64(L, ma, st)
+                                         : convl_fixed_multi_f32_f32(L, ma, st);
+    }
+    if (k == MultiKernel::ConvFixed || k == MultiKernel::ConvFixedWide)
+        return L.prec == (int)Prec::F32 ? conv_fixed_multi_f32(L, ma, st)
+                                        : conv_fixed_multi_f64(L, ma, st);
     return L.prec == (int)Prec::F32 ? multi_f32(L, ma, st)
                                     : multi_f64(L, ma, st);
 }

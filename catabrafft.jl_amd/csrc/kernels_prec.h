@@ -31,6 +31,18 @@ void fixed_fs_f32(std::vector<FixedFs>& rows);
 void fixed_fs_f64(std::vector<FixedFs>& rows);
 void fixed_fs_pair(std::vector<FixedFs>& rows);
 void fixed_fs_f16(std::vector<FixedFs>& rows);
+// The fixed convolutions (fixed_conv.h).
+void fixed_conv_f32(std::vector<FixedConv>& rows);
+void fixed_conv_f64(std::vector<FixedConv>& rows);
+// The fixed large convolutions (fixed_convl.h).
+void fixed_convl_f32_f32(std::vector<FixedConvL>& rows);
+void fixed_convl_f32_f64(std::vector<FixedConvL>& rows);
+void fixed_convl_f64_f64(std::vector<FixedConvL>& rows);
+void init_kernels_fixed_convl_multi_f32_f32();
+void init_kernels_fixed_convl_multi_f32_f64();
+void init_kernels_fixed_convl_multi_f64_f64();
+void init_kernels_fixed_conv_multi_f32();
+void init_kernels_fixed_conv_multi_f64();
 
 hipError_t real_rows_f32(const void* in, void* out, const RealArgs& a, const PassTable& pt,
                          const void* tw, int E, hipStream_t st);

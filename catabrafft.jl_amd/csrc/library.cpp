@@ -536,14 +536,20 @@ static int fs_line_stride(Ctx* ctx, Prec pr, const LinePlan& lp, int C, size_t r
     return best;
 }
 
-// LDS line stride of a fixed four-step pass (FixedFs) with `cols` lines (line pairs) per
-// workgroup: the same model on its own layout.  One element is elem / 4 words (re, im together);
+// LDS line stride of fixed lines (fixed_line.h) with `cols` of them (line pairs) side by side in a
+// workgroup: the same model on their layout.  One element is elem / 4 words (re, im together);
 // an access of the wave runs as groups of lanes that move 256 bytes, over 64 banks (weight 4;
-// tie-break: 128 bytes over 32).
-static int fixed_fs_stride(Ctx* ctx, const FixedFs& f, int cols, size_t reserve) {
+// tie-break: 128 bytes over 32).  in_place: the passes of fixed_conv.h.
+struct FixedShape {
+    const int* r;
+    int np, N, Tt, elem, pad;
+    bool in_place;
+};
+static int fixed_stride(Ctx* ctx, const FixedShape& f, int cols, size_t reserve) {
     static std::mutex mu;
-    static std::map<std::tuple<const FixedFs*, int, size_t>, int> cache;
-    const auto key = std::make_tuple(&f, cols, ctx->lds_max - std::min(ctx->lds_max, reserve));
+    static std::map<std::tuple<const int*, int, int, bool, int, size_t>, int> cache;
+    const auto key = std::make_tuple(f.r, f.Tt, f.elem, f.in_place, cols,
+                                     ctx->lds_max - std::min(ctx->lds_max, reserve));
     {
         std::lock_guard<std::mutex> g(mu);
         auto it = cache.find(key);
@@ -564,13 +570,17 @@ static int fixed_fs_stride(Ctx* ctx, const FixedFs& f, int cols, size_t reserve)
             for (int ib = 0; ib < MB && !over(); ++ib)
                 for (int j = 0; j < R && !over(); ++j)
                     for (int wr = 0; wr < 2; ++wr) {
-                        if (wr ? ip + 1 == f.np : ip == 0) continue;  // global memory
+                        // (global memory: the first reads and, but for in place, the last writes)
+                        if (wr ? ip + 1 == f.np && !f.in_place : ip == 0) continue;
                         for (int L = 0; L < 64; ++L) {
                             const int b = L / cols + ib * f.Tt;
                             word[L] = -1;
                             if (L >= threads || b >= nb) continue;
-                            const int p = b / s, q = b - p * s;
-                            word[L] = (L % cols * Ls + at(wr ? q + s * R * p + s * j : b + j * nb)) * ew;
+                            const int p = b / s, q = b - p * s, n1 = nb / s;
+                            const int e = f.in_place ? b / n1 * (n1 * R) + b % n1 + j * n1
+                                          : wr       ? q + s * R * p + s * j
+                                                     : b + j * nb;
+                            word[L] = (L % cols * Ls + at(e)) * ew;
                         }
                         for (int banks = 64; banks >= 32; banks /= 2)
                             for (int L0 = 0; L0 < 64; L0 += banks / ew) {
@@ -606,7 +616,7 @@ static const FixedFs* pick_fixed_fs(Ctx* ctx, FixedFsKind kind, const LinePlan& 
     while (c > 1 && !fits(c)) c /= 2;
     if (!fits(c)) return nullptr;
     *C = c * f->width;
-    *Ls = fixed_fs_stride(ctx, *f, c, reserve);
+    *Ls = fixed_stride(ctx, FixedShape{f->r, f->np, f->N, f->Tt, f->elem, f->pad, false}, c, reserve);
     f->prepare();
     return f;
 }
@@ -761,7 +771,66 @@ static int plan_large(Ctx* ctx, Plan& p, const PlanOptions& o) {
 
 // Convolution data of a Rader (prime n) or Bluestein transform: permutations or chirp, and the
 // zero-padded kernel b whose spectrum the convolution multiplies by.
-int conv_data(int64_t n, ConvData& d) {
+// Length of a convolution that needs at least m points: the shortest of the fixed kernels' lengths
+// where there is one (they are the lengths that no longer one with fewer passes beats), else the
+// shortest 7-smooth one.
+// Beyond the fused lengths: the cheapest product of two lines of the fixed large convolutions
+// (points times the passes over them, and six for the work lines' trips through memory).
+struct ConvSplit {
+    int64_t L = 0;
+    int N1 = 0, N2 = 0;
+    double cost = 0;
+};
+static int smooth7_passes(int n) { return (int)fourstep_line_radices(n).size(); }
+static const std::vector<ConvSplit>& conv_splits() {  // ascending L, each the cheapest from there on
+    static const std::vector<ConvSplit> v = [] {
+        std::vector<ConvSplit> all, out;
+        const std::vector<int>& n = fixed_convl_lengths();
+        for (int a : n)
+            for (int b : n) {
+                if (a < b || a > 4 * b) continue;
+                ConvSplit c{(int64_t)a * b, a, b, 0};
+                c.cost = (double)c.L * (2 * smooth7_passes(a) + 2 * smooth7_passes(b) + 6);
+                all.push_back(c);
+            }
+        std::sort(all.begin(), all.end(), [](const ConvSplit& x, const ConvSplit& y) {
+            return std::make_tuple(-x.L, x.cost, x.N1) < std::make_tuple(-y.L, y.cost, y.N1);
+        });
+        double best = 1e300;
+        for (const ConvSplit& c : all)
+            if (c.cost < best) {
+                best = c.cost;
+                out.push_back(c);
+            }
+        std::reverse(out.begin(), out.end());
+        return out;
+    }();
+    return v;
+}
+// The split of length L itself (L = 0 in the result: none): N1 >= N2, the most even one (launch A
+// reads its columns in longer runs), but N2 > N1 where that keeps the F64 lines of launch C at 1024
+// points: four of 2048 fill a CU's LDS, and one workgroup's butterflies and scatter do not overlap
+// (L = 2^21, 16 lines: 2048 x 1024 337 + 475 + 480 us, 1024 x 2048 327 + 533 + 352).
+static ConvSplit conv_split_of(int64_t L, Prec prec) {
+    const int most = prec == Prec::F64 ? 1024 : 1 << 30;
+    ConvSplit best;
+    auto rank = [&](int a, int b) { return std::make_tuple(a > most, a < b, std::max(a, b)); };
+    for (int a : fixed_convl_lengths())
+        for (int b : fixed_convl_lengths())
+            if ((int64_t)a * b == L && a <= 4 * b && b <= 4 * a &&
+                (!best.L || rank(a, b) < rank(best.N1, best.N2)))
+                best = ConvSplit{L, a, b, 0};
+    return best;
+}
+static int64_t conv_length(int64_t m, Prec prec) {
+    if (const FixedConv* f = find_fixed_conv(prec, m, false)) return f->N;
+    const std::vector<ConvSplit>& v = conv_splits();
+    const auto it = std::lower_bound(v.begin(), v.end(), m,
+                                     [](const ConvSplit& c, int64_t x) { return c.L < x; });
+    return it != v.end() ? it->L : next_smooth(m);
+}
+
+int conv_data(int64_t n, Prec prec, ConvData& d) {
     const bool rader = is_prime(n);
     d.mode = rader ? ConvMode::Rader : ConvMode::Bluestein;
     d.perm.clear();
@@ -769,7 +838,12 @@ int conv_data(int64_t n, ConvData& d) {
     d.chirp.clear();
     if (rader) {
         const int64_t N = n - 1;
-        d.L = is_smooth(N) ? N : next_smooth(2 * N - 1);
+        // no padding where n - 1 is smooth, unless it is short and has no kernel of its own: a padded
+        // length that has one then costs no more (F32 rows: n = 1031 at L = 2304 1.35 TB/s, n = 2003
+        // at L = 2002 on the run-time kernel 1.31; n = 4099 at 9216 0.99, n = 3001 at 3000 1.29),
+        // and spares a work list the launches of the few run-time convolutions
+        const bool exact = is_smooth(N) && (N > 2048 || find_fixed_conv(prec, N, true));
+        d.L = exact ? N : conv_length(2 * N - 1, prec);
         const int64_t g = primitive_root(n);
         const int64_t ginv = powmod(g, n - 2, n);
         d.perm.resize(N);
@@ -789,7 +863,7 @@ int conv_data(int64_t n, ConvData& d) {
         for (int64_t m = d.L - N + 1; m < d.L; ++m) d.b[m] = w[m - (d.L - N)];
         d.g = g;
     } else {
-        d.L = next_smooth(2 * n - 1);
+        d.L = conv_length(2 * n - 1, prec);
         d.chirp.resize(n);
         const OmegaTable om(2 * n);
         for (int64_t m = 0; m < n; ++m) {
@@ -827,11 +901,35 @@ static int cached_plan_1d(Ctx* c, int64_t n, int64_t batch, int dtype, std::shar
     return CFFT_OK;
 }
 
-int conv_spectrum(Ctx* ctx, const std::vector<cld>& b, Prec cprec, DevBuf& K) {
+std::vector<int> conv_order(const FixedConv& f) {
+    const int R = f.r[f.np - 1], nb = f.N / R;
+    std::vector<int> o(f.N);
+    for (int pos = 0; pos < f.N; ++pos) {
+        // digit i of the position (its first, most significant, is pass 0's) counts the product
+        // of the radices before pass i in the frequency
+        int freq = 0, s = 1, rest = pos, g = f.N;
+        for (int i = 0; i < f.np; ++i) {
+            g /= f.r[i];
+            freq += s * (rest / g);
+            rest %= g;
+            s *= f.r[i];
+        }
+        o[(size_t)(pos % R) * nb + pos / R] = freq;  // butterfly pos / R, output pos mod R
+    }
+    return o;
+}
+
+int conv_spectrum(Ctx* ctx, const std::vector<cld>& b, Prec cprec, DevBuf& K,
+                  const std::vector<int>* order) {
     const int64_t L = (int64_t)b.size();
     if (L <= 4096) {
         std::vector<cld> h = b;
         if (!host_fft_ld(h)) return fail(CFFT_ERR_UNSUPPORTED, "kernel spectrum length not smooth");
+        if (order) {
+            std::vector<cld> o(order->size());
+            for (size_t i = 0; i < o.size(); ++i) o[i] = h[(*order)[i]];
+            h.swap(o);
+        }
         return upload(K, h, cprec);
     }
     // the FP64 plan comes from the context's cache: convolutions of nearby lengths share L
@@ -843,18 +941,121 @@ int conv_spectrum(Ctx* ctx, const std::vector<cld>& b, Prec cprec, DevBuf& K) {
     if ((rc = out.alloc((size_t)L * 16))) return rc;
     if ((rc = plan_exec(*t, in.p, out.p, CFFT_FORWARD, 0, ctx->stream))) return rc;
     CFFT_HIP(hipStreamSynchronize(ctx->stream));
-    if (cprec == Prec::F64) {
+    if (cprec == Prec::F64 && !order) {
         std::swap(K.p, out.p);
         std::swap(K.bytes, out.bytes);
         return CFFT_OK;
     }
-    std::vector<double> h((size_t)2 * L);
+    std::vector<std::complex<double>> h((size_t)L);
     CFFT_HIP(hipMemcpy(h.data(), out.p, (size_t)L * 16, hipMemcpyDeviceToHost));
-    std::vector<float> f((size_t)2 * L);
-    for (size_t i = 0; i < f.size(); ++i) f[i] = (float)h[i];
-    if ((rc = K.alloc((size_t)L * 8))) return rc;
-    CFFT_HIP(hipMemcpy(K.p, f.data(), (size_t)L * 8, hipMemcpyHostToDevice));
+    if (order) {
+        std::vector<std::complex<double>> o(order->size());
+        for (size_t i = 0; i < o.size(); ++i) o[i] = h[(*order)[i]];
+        h.swap(o);
+    }
+    if (cprec == Prec::F64) {
+        if ((rc = K.alloc(h.size() * 16))) return rc;
+        CFFT_HIP(hipMemcpy(K.p, h.data(), h.size() * 16, hipMemcpyHostToDevice));
+        return CFFT_OK;
+    }
+    std::vector<float> f(2 * h.size());
+    for (size_t i = 0; i < h.size(); ++i) {
+        f[2 * i] = (float)h[i].real();
+        f[2 * i + 1] = (float)h[i].imag();
+    }
+    if ((rc = K.alloc(h.size() * 8))) return rc;
+    CFFT_HIP(hipMemcpy(K.p, f.data(), h.size() * 8, hipMemcpyHostToDevice));
     return CFFT_OK;
+}
+
+// Lines per workgroup of a fixed large convolution's launch: 8 in F32, 4 in F64 (64-byte runs),
+// halved until they fit; 0 when even one does not.
+static int convl_tile_lines(Ctx* ctx, const FixedShape& f, int max_threads, size_t reserve, int* Ls) {
+    const size_t per = (size_t)f.elem * ((f.pad < 0 ? f.N : f.N + (f.N >> f.pad)) + 64);
+    int c = 64 / f.elem;
+    while (c > 0 && (c * f.Tt > max_threads || c * per + reserve > ctx->lds_max)) c /= 2;
+    if (c > 0) *Ls = fixed_stride(ctx, f, c, reserve);
+    return c;
+}
+
+// Plans a large convolution on the fixed kernels: its lines, tiles and tables (fixed_convl.h).
+// CFFT_ERR_UNSUPPORTED: the length has no such split.
+static int plan_fixed_convl(Ctx* ctx, Plan& p, const ConvData& d, bool alloc_work) {
+    const ConvSplit sp = conv_split_of(p.L, p.cprec);
+    const FixedConvL* f1 = sp.L ? find_fixed_convl(p.prec, p.cprec, sp.N1) : nullptr;
+    const FixedConvL* f2 = sp.L ? find_fixed_convl(p.prec, p.cprec, sp.N2) : nullptr;
+    if (!f1 || !f2) return CFFT_ERR_UNSUPPORTED;
+    auto sub = std::unique_ptr<Plan>(new Plan());
+    Plan& s = *sub;
+    s.ctx = ctx;
+    s.n = p.L;
+    s.batch = p.batch;
+    s.idist = s.odist = p.L;
+    s.prec = p.cprec;
+    s.dtype = p.cprec == Prec::F32 ? CFFT_C32 : CFFT_C64;
+    s.kind = Kind::FourStep;
+    FourStepPlan& fs = s.fs;
+    fs.N1 = sp.N1;
+    fs.N2 = sp.N2;
+    const std::vector<int> ra(f1->r, f1->r + f1->np), rb(f2->rb, f2->rb + f2->np);
+    int rc;
+    if ((rc = make_line(fs.a, sp.N1, p.cprec, 16, 1 << 16, &ra))) return rc;
+    if ((rc = make_line(fs.b, sp.N2, p.cprec, 16, 1 << 16, &rb))) return rc;
+    const std::vector<int> rcv(f1->rb, f1->rb + f1->np);  // launch C's line
+    if ((rc = make_line(p.line, sp.N1, p.cprec, 16, 1 << 16, &rcv))) return rc;
+    set_tw3_shape(fs, p.L);
+    if ((rc = upload_tw3(fs, p.L, p.cprec))) return rc;
+    const int el = (int)esize(p.cprec);
+    const size_t table = (size_t)(tw3_entries(fs.tbits, fs.tnc) + 1) * el + 16;
+    const FixedShape A{f1->r, f1->np, f1->N, f1->Tt, el, f1->pad, false};
+    const FixedShape B{f2->rb, f2->np, f2->N, f2->Tb, el, f2->pad_b, true};
+    p.convl_ca = convl_tile_lines(ctx, A, f1->max_a, 16, &p.convl_lsa);
+    p.convl_cb = convl_tile_lines(ctx, B, f2->max_b, table, &p.convl_lsb);
+    const FixedShape Cs{f1->rb, f1->np, f1->N, f1->Tb, el, f1->pad_c, false};
+    p.convl_cc = convl_tile_lines(ctx, Cs, f1->max_b, table, &p.convl_lsc);
+    if (!p.convl_ca || !p.convl_cb || !p.convl_cc) return CFFT_ERR_UNSUPPORTED;
+    const int N1 = sp.N1, N2 = sp.N2;
+    auto blocks = [](int lines, int C) { return (size_t)((lines + C - 1) / C) * C; };
+    if (p.mode == ConvMode::Rader) {
+        auto blocked = [&](const std::vector<int>& src, int C, DevBuf& buf) {
+            std::vector<int> v(blocks(N2, C) * N1, 0);
+            int* o = v.data();
+            for (int j0 = 0; j0 < N2; j0 += C)
+                for (int64_t e = 0; e < N1; ++e, o += C) {
+                    const int64_t i = e * N2 + j0;
+                    const int64_t m = std::min<int64_t>(std::min(C, N2 - j0), p.n - 1 - i);
+                    for (int64_t c = 0; c < m; ++c) o[c] = src[(size_t)(i + c)];
+                }
+            return upload_int(buf, v);
+        };
+        if ((rc = blocked(d.perm, p.convl_ca, p.perm))) return rc;
+        if ((rc = blocked(d.iperm, p.convl_cc, p.iperm))) return rc;
+    } else if ((rc = upload(p.chirp, d.chirp, p.cprec))) {
+        return rc;
+    }
+    {
+        const FixedConv lineb{f2->rb, f2->np, f2->N, 0, 0, 0, nullptr, nullptr};
+        const std::vector<int> f = conv_order(lineb);  // frequency of [k N2 / R + b]
+        const int C = p.convl_cb;
+        std::vector<int> order(blocks(N1, C) * N2, 0);
+        int* o = order.data();
+        for (int k0 = 0; k0 < N1; k0 += C)
+            for (int x = 0; x < N2; ++x, o += C)
+                for (int c = 0; c < std::min(C, N1 - k0); ++c) o[c] = k0 + c + N1 * f[(size_t)x];
+        if ((rc = conv_spectrum(ctx, d.b, p.cprec, p.K, &order))) return rc;
+    }
+    f1->prepare();
+    f2->prepare();
+    p.kind = Kind::ConvLarge;
+    p.sub = std::move(sub);
+    p.convl = true;
+    p.fcl1 = f1;
+    p.fcl2 = f2;
+    if (!alloc_work) return CFFT_OK;
+    const size_t wbytes = (size_t)p.batch * p.L * esize(p.cprec);
+    if ((rc = p.w1.alloc(wbytes))) return rc;
+    if ((rc = p.w2.alloc(wbytes))) return rc;
+    return p.dc.alloc((size_t)p.batch * 2 * esize(p.cprec));
 }
 
 // Precision of a convolution's work: a Rader convolution of F32 data with p > 2^16 runs in FP64
@@ -869,11 +1070,11 @@ Prec conv_precision(int64_t n, Prec io, ConvMode mode) {
 static int plan_conv(Ctx* ctx, Plan& p, const PlanOptions& o) {
     const int64_t n = p.n;
     ConvData d;
-    conv_data(n, d);
+    p.cprec = conv_precision(n, p.prec, is_prime(n) ? ConvMode::Rader : ConvMode::Bluestein);
+    conv_data(n, p.cprec, d);
     p.mode = d.mode;
     p.L = d.L;
     p.g = d.g;
-    p.cprec = conv_precision(n, p.prec, p.mode);
     const std::vector<int>& perm = d.perm;
     const std::vector<int>& iperm = d.iperm;
     const std::vector<cld>& chirp = d.chirp;
@@ -882,7 +1083,28 @@ static int plan_conv(Ctx* ctx, Plan& p, const PlanOptions& o) {
     // fused small shape?
     const int E = o.E ? o.E : 16;
     bool small = false;
-    if (p.cprec == p.prec && line_fits(ctx, p.L, p.prec, E)) {
+    // the length's own kernel, unless the shape is forced: 4099 x 4093 lines in ComplexF32 283 us
+    // against 516 on the run-time kernel
+    if (p.cprec == p.prec && o.wave <= 0 && !kWaveDefault && (!o.E || !o.explicit_opts)) {
+        const FixedConv* f = find_fixed_conv(p.prec, p.L, true);
+        if (f) {
+            const std::vector<int> rad(f->r, f->r + f->np);
+            // (the kernel has its own thread count: the run-time line's is no limit)
+            if ((rc = make_line(p.line, p.L, p.prec, 16, 1 << 16, &rad))) return rc;
+            const int last = (int)std::max<int64_t>(n, p.L) - 1;
+            p.LsC = (f->pad < 0 ? last + 1 : last + (last >> f->pad) + 1) | 1;
+            const size_t per = (size_t)esize(p.prec) * (p.LsC + 1);
+            if (per <= ctx->lds_max) {
+                small = true;
+                int c = std::max(1, o.target_threads / f->Tt);
+                c = std::min<int64_t>(c, std::max<size_t>(1, std::max(ctx->lds_rows_budget, per) / per));
+                p.C = (int)std::min<int64_t>(c, std::max<int64_t>(1, p.batch));
+                p.fconv = f;
+                f->prepare();
+            }
+        }
+    }
+    if (!small && p.cprec == p.prec && line_fits(ctx, p.L, p.prec, E)) {
         rc = make_line(p.line, p.L, p.prec, E, 1024);
         if (rc) return rc;
         if (!p.half && (o.wave > 0 || (o.wave < 0 && kWaveDefault))) apply_wave_tail(p.line);
@@ -901,13 +1123,21 @@ static int plan_conv(Ctx* ctx, Plan& p, const PlanOptions& o) {
             p.C = c;
         }
     }
+    // large, on the fixed kernels, unless the shape is forced: 1.05 to 1.6 times the run-time
+    // kernels' rate over n = 8209 .. 2000003 (ComplexF32 20011 x 512 326 us against 406, 300007 x 16
+    // 315 against 474, 1048573 x 16 1208 against 1266; ComplexF64 100003 x 64 389 against 441)
+    if (!small && o.fuse_conv != 0 && !o.large && (!o.E || !o.explicit_opts)) {
+        rc = plan_fixed_convl(ctx, p, d, o.alloc_work);
+        if (rc != CFFT_ERR_UNSUPPORTED) return rc;
+    }
     if (rader) {
         if ((rc = upload_int(p.perm, perm))) return rc;
         if ((rc = upload_int(p.iperm, iperm))) return rc;
     } else {
         if ((rc = upload(p.chirp, chirp, p.cprec))) return rc;
     }
-    if ((rc = conv_spectrum(ctx, d.b, p.cprec, p.K))) return rc;
+    const std::vector<int> order = p.fconv ? conv_order(*p.fconv) : std::vector<int>();
+    if ((rc = conv_spectrum(ctx, d.b, p.cprec, p.K, p.fconv ? &order : nullptr))) return rc;
     if (small) {
         p.kind = Kind::ConvSmall;
         return CFFT_OK;
@@ -1184,13 +1414,15 @@ static std::string describe(const Plan& p) {
             os << (p.mode == ConvMode::Rader ? "rader" : "bluestein") << "-fused L=" << p.L << " "
                << rad(p.line) << " C=" << p.C;
             if (p.line.pt.wave) os << " wave";
+            if (p.fconv) os << " fixed Tt=" << p.fconv->Tt;
             if (p.mode == ConvMode::Rader) os << " g=" << p.g;
             break;
         case Kind::ConvLarge:
             os << (p.mode == ConvMode::Rader ? "rader" : "bluestein") << "-large L=" << p.L
                << " conv=" << (p.cprec == Prec::F32 ? "f32" : "f64");
             if (p.convl)
-                os << " fused3 CA=" << p.convl_ca << " CB=" << p.convl_cb << " CC=" << p.convl_cc;
+                os << " fused3 CA=" << p.convl_ca << " CB=" << p.convl_cb << " CC=" << p.convl_cc
+                   << (p.fcl1 ? " fixed" : "");
             os << " {" << describe(*p.sub) << "}";
             if (p.mode == ConvMode::Rader) os << " g=" << p.g;
             break;
@@ -1208,6 +1440,13 @@ static int run_fft(const Plan& p, const void* in, void* out, int sgn, double sca
     ExecShape sh;
     sh.batch = p.batch;
     return run_fft_s(p, in, out, sgn, scale, epi, st, sh);
+}
+
+static bool al16(const void* q) { return ((uintptr_t)q & 15) == 0; }
+// Whether a fixed pass may run on lines of elements of `elem` bytes at q: its pairs of adjacent
+// lines are read and written as one access of 2 elem bytes.
+static bool pair_fits(const FixedFs* f, const void* q, int64_t dist, size_t elem) {
+    return f->width == 1 || (((uintptr_t)q & (2 * elem - 1)) == 0 && dist % 2 == 0);
 }
 
 // Runs the two passes over the batch in chunks of fs.chunk transforms (0 = the whole batch, the
@@ -1479,7 +1718,10 @@ static int run_fft_s(const Plan& p, const void* in, void* out, int sgn, double s
             a.iperm = (const int*)p.iperm.p;
             a.chirp = p.chirp.p;
             a.K = p.K.p;
-            CFFT_HIP(launch_conv_small(p.prec, in, out, a, p.line.pt, p.line.dtw.p, st));
+            if (p.fconv)
+                CFFT_HIP(p.fconv->launch(in, out, a, p.line.dtw.p, st));
+            else
+                CFFT_HIP(launch_conv_small(p.prec, in, out, a, p.line.pt, p.line.dtw.p, st));
             return CFFT_OK;
         }
         case Kind::ConvLarge: {
@@ -1520,6 +1762,14 @@ static int run_fft_s(const Plan& p, const void* in, void* out, int sgn, double s
                 a.tw3 = f.tw3.p;
                 a.tbits = f.tbits;
                 a.tnc = f.tnc;
+                if (p.fcl1) {
+                    if ((int64_t)std::max(f.N1, f.N2) * B > 0x7fffffff)
+                        return fail(CFFT_ERR_UNSUPPORTED, "too many convolution tiles");
+                    CFFT_HIP(p.fcl1->launch_a(in, a, f.a.dtw.p, st));
+                    CFFT_HIP(p.fcl2->launch_ba(a, f.b.dtw.p, st));
+                    CFFT_HIP(p.fcl1->launch_c(out, a, p.line.dtw.p, st));
+                    return CFFT_OK;
+                }
                 CFFT_HIP(launch_convl(p.prec, p.cprec, in, out, a, f.a.pt, f.a.dtw.p, f.b.pt,
                                       f.b.dtw.p, st));
                 return CFFT_OK;

@@ -96,12 +96,15 @@ struct Plan {
     ConvMode mode = ConvMode::Rader;
     int64_t L = 0, g = 0;
     int LsC = 0;  // fused convolution: LDS line stride (input and work lines share it)
+    const FixedConv* fconv = nullptr;  // fused convolution: the length's own kernel
     Prec cprec = Prec::F32;
     DevBuf perm, iperm, chirp, K, dc, w1, w2;
     std::unique_ptr<Plan> sub;  // large convolution: FFT_L; six-step: the M-point row FFTs
     // large convolution whose FFT_L is a four-step, run as three fused launches: the tile and
     // LDS line stride of the last launch (lines of N1 points over the second FFT's middle)
     bool convl = false;
+    // their fixed lines (N1: launches A and C, N2: BA); nullptr: the run-time kernels
+    const FixedConvL *fcl1 = nullptr, *fcl2 = nullptr;
     int convl_ca = 0, convl_lsa = 0, convl_cb = 0, convl_lsb = 0, convl_cc = 0, convl_lsc = 0;
     // real-input transforms: 1 = fused (n even, n/2 fits a workgroup), 2 = even via a complex
     // sub-plan of n/2, 3 = odd via a complex sub-plan of n; idist / odist hold rdist (reals) and
@@ -250,8 +253,14 @@ struct ConvData {
     std::vector<int> perm, iperm;
     std::vector<std::complex<long double>> chirp, b;
 };
-int conv_data(int64_t n, ConvData& d);
-int conv_spectrum(Ctx* ctx, const std::vector<std::complex<long double>>& b, Prec cprec, DevBuf& K);
+// prec: the precision of the convolution (fused convolutions prefer the lengths of its fixed
+// kernels).
+int conv_data(int64_t n, Prec prec, ConvData& d);
+// K[i] = FFT_L(b)[order[i]] (nullptr: natural order).
+int conv_spectrum(Ctx* ctx, const std::vector<std::complex<long double>>& b, Prec cprec, DevBuf& K,
+                  const std::vector<int>* order = nullptr);
+// The frequency at each position of a fixed convolution's spectrum.
+std::vector<int> conv_order(const FixedConv& f);
 Prec conv_precision(int64_t n, Prec io, ConvMode mode);
 int upload_cld(DevBuf& buf, const std::vector<std::complex<long double>>& v, Prec pr);
 int upload_ints(DevBuf& buf, const std::vector<int>& v);

@@ -88,7 +88,10 @@ struct MultiLaunch {
 
 enum class MultiKernel : int {
     Rows = 0, FourStepA, FourStepB, ConvSmall, Gather, Scatter,
-    ConvLA, ConvLBA, ConvLC  // the three fused launches of a large convolution
+    ConvLA, ConvLBA, ConvLC,  // the three fused launches of a large convolution
+    ConvFixed, ConvFixedWide, // fused convolutions of fixed lengths (MPlan::L): workgroups of
+                              // up to 512 threads, and of up to 1024
+    ConvFA, ConvFBA, ConvFC   // large convolutions over fixed lines (MPlan::N1, N2)
 };
 
 // Launch-wide arguments of a work-list launch.
@@ -102,6 +105,11 @@ hipError_t launch_multi(const MultiLaunch& L, const MultiArgs& a, hipStream_t st
 // Per-precision entry points (kernels_f32.hip / kernels_f64.hip).
 hipError_t multi_f32(const MultiLaunch& L, const MultiArgs& a, hipStream_t st);
 hipError_t multi_f64(const MultiLaunch& L, const MultiArgs& a, hipStream_t st);
+hipError_t convl_fixed_multi_f32_f32(const MultiLaunch& L, const MultiArgs& a, hipStream_t st);
+hipError_t convl_fixed_multi_f32_f64(const MultiLaunch& L, const MultiArgs& a, hipStream_t st);
+hipError_t convl_fixed_multi_f64_f64(const MultiLaunch& L, const MultiArgs& a, hipStream_t st);
+hipError_t conv_fixed_multi_f32(const MultiLaunch& L, const MultiArgs& a, hipStream_t st);
+hipError_t conv_fixed_multi_f64(const MultiLaunch& L, const MultiArgs& a, hipStream_t st);
 hipError_t gs_multi_f32_f32(const MultiLaunch& L, const MultiArgs& a, hipStream_t st);
 hipError_t gs_multi_f32_f64(const MultiLaunch& L, const MultiArgs& a, hipStream_t st);
 hipError_t gs_multi_f64_f64(const MultiLaunch& L, const MultiArgs& a, hipStream_t st);

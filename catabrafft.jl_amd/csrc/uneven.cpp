@@ -247,9 +247,12 @@ void WorkList::add_transforms(const PlanEntry& e, const std::vector<XformRef>& x
             break;
         }
         case Kind::ConvSmall: {
-            const int block = p.C * p.line.Tt;
+            const int block = p.C * (p.fconv ? p.fconv->Tt : p.line.Tt);
             const size_t lds = 2 * (esz(pr) / 2) * (size_t)p.C * p.LsC + esz(pr) * p.C;
-            add_lines(1, MultiKernel::ConvSmall, p, e.mplan, pr, p.C, block, lds, xs,
+            const MultiKernel mk = !p.fconv                       ? MultiKernel::ConvSmall
+                                   : p.fconv->max_threads <= 512 ? MultiKernel::ConvFixed
+                                                                 : MultiKernel::ConvFixedWide;
+            add_lines(1, mk, p, e.mplan, pr, p.C, block, lds, xs,
                       4.0 * p.L * std::log2((double)p.L), false, 0);
             break;
         }
@@ -301,6 +304,18 @@ void WorkList::add_transforms(const PlanEntry& e, const std::vector<XformRef>& x
                 const size_t lda = 2 * ce * (size_t)CA * p.convl_lsa;
                 const size_t ldb = fsb_tw_offset(ce, CB, p.convl_lsb) + table;
                 const size_t ldc = fsb_tw_offset(ce, p.convl_cc, p.convl_lsc) + table;
+                const bool fx = p.fcl1 != nullptr;
+                const size_t more = fx ? 2 * ce : 0;  // the fixed kernels' element after the table
+                const int ta_thr = fx ? p.fcl1->Tt : f.a.Tt, tb_thr = fx ? p.fcl2->Tb : f.b.Tt;
+                const int tc_thr = fx ? p.fcl1->Tb : f.a.Tt;
+                const MultiKernel ka = fx ? MultiKernel::ConvFA : MultiKernel::ConvLA;
+                const MultiKernel kb = fx ? MultiKernel::ConvFBA : MultiKernel::ConvLBA;
+                const MultiKernel kc = fx ? MultiKernel::ConvFC : MultiKernel::ConvLC;
+                // (a fixed line keeps to the kernel of its block: 512 threads, or 1024)
+                auto threads = [fx](int n, int most) { return fx && most > 512 ? std::max(n, 513) : n; };
+                const int na = threads(CA * ta_thr, fx ? p.fcl1->max_a : 0);
+                const int nb = threads(CB * tb_thr, fx ? p.fcl2->max_b : 0);
+                const int nc = threads(p.convl_cc * tc_thr, fx ? p.fcl1->max_b : 0);
                 const int ta = (f.N2 + CA - 1) / CA, tb = (f.N1 + CB - 1) / CB;
                 const int tc = (f.N2 + p.convl_cc - 1) / p.convl_cc;
                 const double la = std::log2((double)f.N1), lb = std::log2((double)f.N2);
@@ -316,7 +331,7 @@ void WorkList::add_transforms(const PlanEntry& e, const std::vector<XformRef>& x
                         it.in = x.in;
                         it.out = x.w1;
                         it.flags = x.in_sel | (kAbs << kSelOutShift) | dirf;
-                        add_item(1, MultiKernel::ConvLA, pr, cp, CA * f.a.Tt, lda, it,
+                        add_item(1, ka, pr, cp, na, lda, it,
                                  (double)CA * f.N1 * la);
                     }
                     for (int t = 0; t < tb; ++t) {
@@ -324,7 +339,7 @@ void WorkList::add_transforms(const PlanEntry& e, const std::vector<XformRef>& x
                         it.in = x.w1;
                         it.out = x.w2;
                         it.flags = kAbs | (kAbs << kSelOutShift) | dirf;
-                        add_item(2, MultiKernel::ConvLBA, pr, cp, CB * f.b.Tt, ldb, it,
+                        add_item(2, kb, pr, cp, nb, ldb + more, it,
                                  2.0 * CB * f.N2 * lb);
                     }
                     for (int t = 0; t < tc; ++t) {
@@ -332,7 +347,7 @@ void WorkList::add_transforms(const PlanEntry& e, const std::vector<XformRef>& x
                         it.in = x.w2;
                         it.out = x.out;
                         it.flags = kAbs | (x.out_sel << kSelOutShift) | dirf;
-                        add_item(3, MultiKernel::ConvLC, pr, cp, p.convl_cc * f.a.Tt, ldc, it,
+                        add_item(3, kc, pr, cp, nc, ldc + more, it,
                                  (double)p.convl_cc * f.N1 * la);
                     }
                 }
@@ -441,6 +456,11 @@ int WorkList::finalize(DevBuf& dplans, DevBuf& ditems, DevBuf& dtable,
         // groups join only if neither block nor LDS grows by more than 2x: the merged launch runs
         // every item at the larger of both, which costs occupancy
         auto close = [](const Group& a, const Group& b) {
+            // (workgroups of up to 512 threads and larger ones run different kernels)
+            const MultiKernel k = (MultiKernel)a.kernel;
+            if ((k == MultiKernel::ConvFA || k == MultiKernel::ConvFBA || k == MultiKernel::ConvFC) &&
+                (a.block <= 512) != (b.block <= 512))
+                return false;
             return std::max(a.block, b.block) <= 2 * std::min(a.block, b.block) &&
                    std::max(a.lds, b.lds) <= 2 * std::min(a.lds, b.lds);
         };
@@ -629,6 +649,9 @@ static int capture_launches(UnevenState& st, const MultiArgs& ma) {
             case MultiKernel::ConvLA:
             case MultiKernel::ConvLBA:
             case MultiKernel::ConvLC: key = -10 - 2 * L.prec - L.cprec; break;
+            case MultiKernel::ConvFA:
+            case MultiKernel::ConvFBA:
+            case MultiKernel::ConvFC: key = -20 - 2 * L.prec - L.cprec; break;
             default: key = single++;
         }
         chains[key].push_back(&L);

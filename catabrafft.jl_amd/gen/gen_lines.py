@@ -6,10 +6,12 @@
 A line is a length and its radix sequence, the one the planner takes by default for that length
 (line_radices in library.cpp).  The rows kernels cover every 7-smooth length from 16 to 8192: the
 lengths a workgroup holds in both precisions.  The four-step passes cover every 7-smooth length
-from 16 to 2048, and 4096: the factors of the lengths up to 2^22 and of 2^24.  The lists are split in parts so that several
+from 16 to 2048, and 4096: the factors of the lengths up to 2^22 and of 2^24.  The fused convolutions pad to
+the lengths of conv_lines, the large ones to products of two of convl_lines.  The lists are split in parts so that several
 translation units compile them in parallel; the _FEW list is the part that the CPU emulation
 build of the tests compiles.
 """
+import math
 import os
 import sys
 
@@ -49,6 +51,39 @@ def fourstep_radices(n):
     return [1 << (base + (i >= passes - extra)) for i in range(passes)]
 
 
+def conv_lines():
+    """Convolution lengths 2^a m up to 16384, 16s first and the odd radices last: those that no
+    longer length with fewer passes beats (cost: length x (passes + 0.3)), at least 6 % apart."""
+    cand = []
+    for a in range(1, 15):
+        for m in (1, 3, 5, 7, 9, 15, 21, 25, 27, 35, 45, 49, 63, 75, 81):
+            if not 16 <= m << a <= 16384:
+                continue
+            q, rem = divmod(a, 4)
+            r = [16] * q
+            if rem == 1 and q:
+                r = r[:-1] + [8, 4]
+            elif rem:
+                r.append(1 << rem)
+            for p in (9, 7, 5, 3):
+                while m % p == 0:
+                    r.append(p)
+                    m //= p
+            cand.append(r)
+    best, keep = float("inf"), []
+    for r in sorted(cand, key=lambda r: -math.prod(r)):
+        cost = math.prod(r) * (len(r) + 0.3)
+        if cost < best and (not keep or math.prod(keep[-1]) >= 1.06 * math.prod(r)):
+            best = cost
+            keep.append(r)
+    return keep[::-1]
+
+
+def convl_lines():
+    """Lines of the large convolutions: 2^a {1, 3, 5, 7, 9} from 64 to 2048 points."""
+    return sorted({m << a for m in (1, 3, 5, 7, 9) for a in range(3, 12) if 64 <= m << a <= 2048})
+
+
 def macro(name, lines):
     out = [f"#define {name}(X) \\"]
     out += [f"    X({', '.join(map(str, r))}) \\" for r in lines]
@@ -73,9 +108,20 @@ def main():
     parts.append(macro("CFFT_FS_LINES_FEW", [r for i, r in enumerate(fs) if i % 16 == 3]
                        + [fourstep_radices(n) for n in (16, 128, 256, 1024)] + fs[-2:]))
     parts.append(macro("CFFT_FS_LINES", fs))
+    conv = conv_lines()
+    parts.append(macro("CFFT_CONV_LINES", conv))
+    parts.append(macro("CFFT_CONV_LINES_F64", [r for r in conv if math.prod(r) <= 8192]))
+    two = []
+    for n in convl_lines():
+        q = fourstep_radices(n)
+        two.append([f"CFFT_Q({', '.join(map(str, r))})" for r in (q, sorted(q, reverse=True))])
+    parts.append("// X(radices of launch A, radices of launches BA and C), CFFT_Q(...) a sequence")
+    parts.append("#define CFFT_Q(...) Rad<__VA_ARGS__>")
+    parts.append(macro("CFFT_CONVL_LINES", two))
     with open(out, "w") as f:
         f.write("\n".join(parts) + "\n")
-    print(f"wrote {os.path.normpath(out)}: {len(rows)} row lines, {len(fs)} four-step lines")
+    print(f"wrote {os.path.normpath(out)}: {len(rows)} row lines, {len(fs)} four-step lines, "
+          f"{len(conv)} convolution lengths, {len(two)} lines of large convolutions")
 
 
 if __name__ == "__main__":

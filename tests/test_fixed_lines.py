@@ -186,3 +186,157 @@ def test_fixed_four_step_matches_the_run_time_kernels(gpu_ready, tmp_path, dt):
                 p.exec_torch(x, x)
                 got.append((torch.view_as_real(y), torch.view_as_real(x)))
             assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]), (n1, n2)
+
+
+# ------------------------------------------------------------------------------ convolutions
+def _factor_smooth(n, primes=(2, 3, 5, 7, 11, 13)):
+    for p in primes:
+        while n % p == 0:
+            n //= p
+    return n == 1
+
+
+def _prime(n):
+    return n > 1 and all(n % d for d in range(2, int(n ** 0.5) + 1))
+
+
+def _conv_lengths(lines):
+    """Per convolution length L: the longest prime whose padded convolution fits it (Rader) and the
+    longest length with a large prime factor that does (Bluestein)."""
+    out, prev = [], 0
+    for L in lines:
+        for need, ok in ((lambda n: 2 * (n - 1) - 1, lambda n: _prime(n) and not _factor_smooth(n - 1)),
+                         (lambda n: 2 * n - 1, lambda n: not _prime(n) and not _factor_smooth(n))):
+            n = L // 2 + 2
+            while n > 2 and not (prev < need(n) <= L and ok(n)):
+                n -= 1
+            if n > 2:
+                out.append((L, n))
+        prev = L
+    return out
+
+
+CONV = {np.complex64: _conv_lengths(_lengths("CFFT_CONV_LINES")),
+        np.complex128: _conv_lengths(_lengths("CFFT_CONV_LINES_F64"))}
+
+
+def _bound(n, dt):
+    """The parity bounds: ComplexF32 1e-6, ComplexF64 4 eps log2 n (relative L2)."""
+    return 1e-6 if dt == np.complex64 else 4 * np.finfo(float).eps * max(1.0, np.log2(n))
+
+
+@pytest.mark.parametrize("dt", [np.complex64, np.complex128])
+def test_emulated_fixed_convolutions(emu, dt):
+    ctx, code, batch = ctypes.c_void_p(), (0 if dt == np.complex64 else 1), 5
+    assert emu.cfft_init(0, ctypes.byref(ctx)) == 0
+    for L, n in [(16, 17), (256, 257)] + CONV[dt][::5]:
+        p = ctypes.c_void_p()
+        assert emu.cfft_plan_1d(ctx, n, batch, n, n, code, 0, ctypes.byref(p)) == 0
+        assert f"fused L={L} " in _desc(emu, p) and "fixed" in _desc(emu, p), _desc(emu, p)
+        x = seeded_complex(n, batch=batch, seed=n, dtype=dt)
+        y, z = np.zeros_like(x), x.copy()
+        assert emu.cfft_exec(p, x.ctypes.data, y.ctypes.data, -1, 0, None) == 0
+        assert emu.cfft_exec(p, z.ctypes.data, z.ctypes.data, 1, 1, None) == 0
+        for got, ref in ((y, np.fft.fft(x.astype(np.clongdouble))),
+                         (z, np.fft.ifft(x.astype(np.clongdouble)))):
+            err = float(np.linalg.norm(got - ref) / np.linalg.norm(ref))
+            assert err < _bound(n, dt), (n, L, err)
+        emu.cfft_plan_destroy(p)
+    emu.cfft_finalize(ctx)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [np.complex64, np.complex128])
+def test_fixed_convolutions(gpu_ready, dt):
+    """Each length against numpy in long double, and one work list of all of them against the
+    plans alone, bit for bit."""
+    import torch
+
+    import catabrafft as C
+
+    lens = [17, 257] + [n for _, n in CONV[dt]]
+    offs = np.concatenate([[0], np.cumsum(lens)[:-1]]).astype(np.int64)
+    x = torch.from_numpy(seeded_complex(int(np.sum(lens)), seed=3, dtype=dt)).cuda()
+    u = C.UnevenPlan(lens, offs, dt)
+    y = u.exec_torch(x, torch.zeros_like(x))
+    for n, o in zip(lens, offs):
+        p = C.Plan(n, 1, dt)
+        print(f"{np.dtype(dt)} {p.describe()}", flush=True)
+        assert "fixed" in p.describe(), p.describe()
+        a = p.exec_torch(x[o:o + n])
+        assert torch.equal(torch.view_as_real(a), torch.view_as_real(y[o:o + n])), n
+        rows = torch.from_numpy(seeded_complex(n, batch=67, seed=n, dtype=dt)).cuda()
+        q = C.Plan(n, 67, dt)
+        got = q.exec_torch(rows, direction=1, normalize=True).cpu().numpy()
+        ref = np.fft.ifft(rows.cpu().numpy().astype(np.clongdouble))
+        err = float(np.linalg.norm(got - ref) / np.linalg.norm(ref))
+        assert err < _bound(n, dt), (n, err)
+
+
+# ------------------------------------------------------------------------------ large convolutions
+def _convl_lengths(lo, hi, count):
+    """Lengths spread over [lo, hi]: primes (Rader, padded or not) and composites with a large
+    prime factor (Bluestein) in turn, 65537 = 2^16 + 1 among them where it falls in the range."""
+    out = [65537] if lo <= 65537 <= hi else []
+    for i in range(count):
+        n = int(lo * (hi / lo) ** (i / (count - 1)))
+        while not ((_prime(n) and not _factor_smooth(n - 1)) if i % 2 else
+                   (not _prime(n) and not _factor_smooth(n))):
+            n += 1
+        out.append(n)
+    return out
+
+
+@pytest.mark.parametrize("dt,lo,hi,count", [(np.complex64, 8200, 140000, 9),
+                                            (np.complex128, 5200, 40000, 7)])
+def test_emulated_fixed_large_convolutions(emu, dt, lo, hi, count):
+    ctx, code = ctypes.c_void_p(), (0 if dt == np.complex64 else 1)
+    assert emu.cfft_init(0, ctypes.byref(ctx)) == 0
+    lens = np.array(_convl_lengths(lo, hi, count), dtype=np.int64)
+    offs = np.concatenate([[0], np.cumsum(lens)[:-1]]).astype(np.int64)
+    P, u = ctypes.POINTER(ctypes.c_int64), ctypes.c_void_p()
+    x = seeded_complex(int(lens.sum()), seed=5, dtype=dt)
+    y = np.zeros_like(x)
+    assert emu.cfft_plan_many_uneven(ctx, len(lens), lens.ctypes.data_as(P),
+                                     offs.ctypes.data_as(P), code, 0, ctypes.byref(u)) == 0
+    assert emu.cfft_exec(u, x.ctypes.data, y.ctypes.data, 1, 1, None) == 0
+    for n, o in zip(lens.tolist(), offs.tolist()):
+        p = ctypes.c_void_p()
+        assert emu.cfft_plan_1d(ctx, n, 1, n, n, code, 0, ctypes.byref(p)) == 0
+        assert "fused3" in _desc(emu, p) and "fixed" in _desc(emu, p), _desc(emu, p)
+        z = x[o:o + n].copy()
+        assert emu.cfft_exec(p, z.ctypes.data, z.ctypes.data, 1, 1, None) == 0
+        assert np.array_equal(z, y[o:o + n]), n
+        ref = np.fft.ifft(x[o:o + n].astype(np.clongdouble))
+        err = float(np.linalg.norm(z - ref) / np.linalg.norm(ref))
+        assert err < _bound(n, dt), (n, err)
+        emu.cfft_plan_destroy(p)
+    emu.cfft_plan_destroy(u)
+    emu.cfft_finalize(ctx)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt,lo,hi,count", [(np.complex64, 8200, 1500000, 40),
+                                            (np.complex128, 5200, 1500000, 40)])
+def test_fixed_large_convolutions(gpu_ready, dt, lo, hi, count):
+    import torch
+
+    import catabrafft as C
+
+    lens = _convl_lengths(lo, hi, count)
+    offs = np.concatenate([[0], np.cumsum(lens)[:-1]]).astype(np.int64)
+    x = torch.from_numpy(seeded_complex(int(np.sum(lens)), seed=3, dtype=dt)).cuda()
+    y = C.UnevenPlan(lens, offs, dt).exec_torch(x, torch.zeros_like(x))
+    for n, o in zip(lens, offs):
+        for batch in (1, 3):
+            p = C.Plan(n, batch, dt)
+            print(f"{np.dtype(dt)} {p.describe()}", flush=True)
+            assert "fixed" in p.describe(), p.describe()
+            rows = torch.stack([x[o:o + n]] * batch)
+            a = p.exec_torch(rows)
+            for r in range(batch):
+                assert torch.equal(torch.view_as_real(a[r]), torch.view_as_real(y[o:o + n])), n
+        p.exec_torch(rows, rows, direction=1, normalize=True)
+        ref = np.fft.ifft(x[o:o + n].cpu().numpy().astype(np.clongdouble))
+        err = float(np.linalg.norm(rows[-1].cpu().numpy() - ref) / np.linalg.norm(ref))
+        assert err < _bound(n, dt), (n, err)
