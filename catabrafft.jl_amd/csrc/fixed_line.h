@@ -180,8 +180,9 @@ __device__ __forceinline__ void fixed_pass(const int t, const bool active,
     }
 }
 
-// The passes of line Q from src through lds to dst.  ALIAS: a line of one pass reads and writes
-// the same memory (a barrier between the two).
+// The passes of line Q from src through lds to dst.  ALIAS: the last pass writes what it or its
+// source reads -- dst is the line's LDS, or a line of one pass works in place (a barrier between the
+// two).
 template <typename T, class Q, int TT, int I = 0, bool ALIAS = false, typename W, class SRC,
           class DST, class LDS>
 __device__ __forceinline__ void fixed_line(const int t, const bool active,
@@ -193,7 +194,7 @@ __device__ __forceinline__ void fixed_line(const int t, const bool active,
     } else if constexpr (first) {
         fixed_pass<T, Q, TT, I, false>(t, active, tw, src, lds);
     } else if constexpr (last) {
-        fixed_pass<T, Q, TT, I, false>(t, active, tw, lds, dst);
+        fixed_pass<T, Q, TT, I, ALIAS>(t, active, tw, lds, dst);
     } else {
         fixed_pass<T, Q, TT, I, true>(t, active, tw, lds, lds);
     }

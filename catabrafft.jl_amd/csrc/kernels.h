@@ -216,6 +216,20 @@ const FixedConvL* find_fixed_convl(Prec pio, Prec pc, int64_t N);
 // Every length of the lines, ascending.
 const std::vector<int>& fixed_convl_lengths();
 
+// The real-input ends of a four-step on fixed lines (fixed_real.h): pass B that untangles its
+// spectrum (a.C lines a tile, an even number; rw[k] = e^{-2 pi i k / n}), and pass A that builds its
+// input from one.
+struct FixedReal {
+    const int* r;
+    int np, N, Tt, max_threads, elem, pad;
+    hipError_t (*launch_b)(const void* in, void* out, const FourStepBArgs& a, const void* rw,
+                           const void* tw, hipStream_t st);
+    hipError_t (*launch_a)(const void* in, void* out, const FourStepAArgs& a, double scale,
+                           const void* rw, const void* tw, hipStream_t st);
+    void (*prepare)();
+};
+const FixedReal* find_fixed_real(Prec p, const PassTable& pt, int N);
+
 // Sets per-kernel attributes (large LDS) once; called when a context is created.
 void init_kernels();
 

@@ -65,6 +65,17 @@ const FixedFs* find_fixed_fs(FixedFsKind kind, const PassTable& pt, int N) {
     return find_in(m[(int)kind], pt, N);
 }
 
+const FixedReal* find_fixed_real(Prec p, const PassTable& pt, int N) {
+    auto make = [](void (*fill)(std::vector<FixedReal>&)) {
+        std::vector<FixedReal> v;
+        fill(v);
+        return index_by_length(v);
+    };
+    static const std::unordered_multimap<int, FixedReal> m[2] = {make(fixed_real_f32),
+                                                                 make(fixed_real_f64)};
+    return find_in(m[p == Prec::F64], pt, N);
+}
+
 const FixedConv* find_fixed_conv(Prec p, int64_t m, bool exact) {
     auto make = [](void (*fill)(std::vector<FixedConv>&)) {
         std::vector<FixedConv> v;

@@ -31,6 +31,9 @@ void fixed_fs_f32(std::vector<FixedFs>& rows);
 void fixed_fs_f64(std::vector<FixedFs>& rows);
 void fixed_fs_pair(std::vector<FixedFs>& rows);
 void fixed_fs_f16(std::vector<FixedFs>& rows);
+// The real-input four-step passes (fixed_real.h).
+void fixed_real_f32(std::vector<FixedReal>& rows);
+void fixed_real_f64(std::vector<FixedReal>& rows);
 // The fixed convolutions (fixed_conv.h).
 void fixed_conv_f32(std::vector<FixedConv>& rows);
 void fixed_conv_f64(std::vector<FixedConv>& rows);

@@ -1449,6 +1449,90 @@ static bool pair_fits(const FixedFs* f, const void* q, int64_t dist, size_t elem
     return f->width == 1 || (((uintptr_t)q & (2 * elem - 1)) == 0 && dist % 2 == 0);
 }
 
+// Pass A of nb transforms.
+static int fourstep_pass_a(const Plan& p, const void* inb, void* midb, int64_t idist,
+                           int64_t mdist, int sgn, hipStream_t st, int64_t nb) {
+    const FourStepPlan& fs = p.fs;
+    FourStepAArgs a{};
+    a.N1 = fs.N1;
+    a.N2 = fs.N2;
+    a.C = fs.CA;
+    a.Tt = fs.a.Tt;
+    a.Ls = fs.a.Ls;
+    a.E = fs.a.E;
+    a.batch = nb;
+    a.idist = idist;
+    a.odist = mdist;
+    a.sgn_in = sgn;
+    a.xcd = 1;
+    a.mid_plain = fs.chunk > 0;  // a chunk's middle is read back while still cached
+    const int64_t es_ = esize(p.prec);
+    const size_t eio = io_esize(p);
+    if (fs.fixed_a && pair_fits(fs.fixed_a, inb, idist, eio)) {
+        a.C = fs.FCA;
+        a.Ls = fs.FLsA;
+        CFFT_HIP(fs.fixed_a->launch_a(inb, midb, a, fs.a.dtw.p, st));
+    } else if (p.half) {
+        CFFT_HIP(launch_fourstep_a_f16(inb, midb, a, fs.a.pt, fs.a.dtw.p, st));
+    } else if (fs.pair_a && al16(inb) && al16(midb) && idist % 2 == 0 && mdist % 2 == 0) {
+        a.Ls = fs.LsA2;
+        CFFT_HIP(launch_fourstep_a_pair(inb, midb, a, fs.a.pt, fs.a.dtw.p, st));
+    } else if (fs.pipe_a > 0) {
+        a.grid = (int)std::min<int64_t>(fs.pipe_a, (int64_t)((fs.N2 + fs.CA - 1) / fs.CA) * nb);
+        CFFT_HIP(launch_fourstep_a_pipe(p.prec, inb, midb, a, fs.a.pt, fs.a.dtw.p,
+                                        fs.a.dtw.bytes / (size_t)es_, st));
+    } else {
+        CFFT_HIP(launch_fourstep_a(p.prec, inb, midb, a, fs.a.pt, fs.a.dtw.p, st));
+    }
+    return CFFT_OK;
+}
+
+// Pass B of nb transforms (epi.dc: of the first).
+static int fourstep_pass_b(const Plan& p, const void* midb, void* outb, int64_t mdist,
+                           int64_t odist, int sgn, double scale, ConvEpilogue epi, hipStream_t st,
+                           int64_t nb) {
+    const FourStepPlan& fs = p.fs;
+    const size_t es = esize(p.prec), eio = io_esize(p);
+    const int64_t es_ = (int64_t)es;
+    FourStepBArgs b{};
+    b.N1 = fs.N1;
+    b.N2 = fs.N2;
+    b.C = fs.CB;
+    b.Tt = fs.b.Tt;
+    b.Ls = fs.b.Ls;
+    b.E = fs.b.E;
+    b.batch = nb;
+    b.idist = mdist;
+    b.odist = odist;
+    b.sgn_in = 1;
+    b.sgn_out = sgn;
+    b.scale = scale;
+    b.epi = epi;
+    b.tbits = fs.tbits;
+    b.tnc = fs.tnc;
+    b.tw3 = fs.tw3.p;
+    b.xcd = 1;
+    if (fs.fixed_b && !epi.K && pair_fits(fs.fixed_b, midb, mdist, es) &&
+        pair_fits(fs.fixed_b, outb, odist, eio)) {
+        b.C = fs.FCB;
+        b.Ls = fs.FLsB;
+        CFFT_HIP(fs.fixed_b->launch_b(midb, outb, b, fs.b.dtw.p, st));
+    } else if (p.half) {
+        CFFT_HIP(launch_fourstep_b_f16(midb, outb, b, fs.b.pt, fs.b.dtw.p, st));
+    } else if (fs.pair_b && !epi.K && al16(midb) && al16(outb) && mdist % 2 == 0 &&
+               odist % 2 == 0) {
+        b.Ls = fs.LsB2;
+        CFFT_HIP(launch_fourstep_b_pair(midb, outb, b, fs.b.pt, fs.b.dtw.p, st));
+    } else if (fs.pipe_b > 0 && !epi.K) {
+        b.grid = (int)std::min<int64_t>(fs.pipe_b, (int64_t)((fs.N1 + fs.CB - 1) / fs.CB) * nb);
+        CFFT_HIP(launch_fourstep_b_pipe(p.prec, midb, outb, b, fs.b.pt, fs.b.dtw.p,
+                                        fs.b.dtw.bytes / (size_t)es_, st));
+    } else {
+        CFFT_HIP(launch_fourstep_b(p.prec, midb, outb, b, fs.b.pt, fs.b.dtw.p, st));
+    }
+    return CFFT_OK;
+}
+
 // Runs the two passes over the batch in chunks of fs.chunk transforms (0 = the whole batch, the
 // default: chunks small enough for the middle to stay in the Infinity Cache measured slower on
 // MI355X, their launch tails outweighing the saved HBM traffic).  Chunking stays a tuning knob.
@@ -1463,78 +1547,11 @@ static int run_fourstep(const Plan& p, const void* in, void* mid, void* out, int
         const char* inb = (const char*)in + (size_t)b0 * idist * eio;
         char* midb = (char*)mid + (size_t)b0 * mdist * es;
         char* outb = (char*)out + (size_t)b0 * odist * eio;
-        FourStepAArgs a{};
-        a.N1 = fs.N1;
-        a.N2 = fs.N2;
-        a.C = fs.CA;
-        a.Tt = fs.a.Tt;
-        a.Ls = fs.a.Ls;
-        a.E = fs.a.E;
-        a.batch = nb;
-        a.idist = idist;
-        a.odist = mdist;
-        a.sgn_in = sgn;
-        a.xcd = 1;
-        a.mid_plain = fs.chunk > 0;  // a chunk's middle is read back while still cached
-        const int64_t es_ = esize(p.prec);
-        auto al16 = [](const void* q) { return ((uintptr_t)q & 15) == 0; };
-        // a fixed pass's pairs of adjacent lines are 2 * eio (es in the middle) bytes apart
-        auto fits = [](const FixedFs* f, const void* q, int64_t dist, size_t elem) {
-            return f->width == 1 || (((uintptr_t)q & (2 * elem - 1)) == 0 && dist % 2 == 0);
-        };
-        if (fs.fixed_a && fits(fs.fixed_a, inb, idist, eio)) {
-            a.C = fs.FCA;
-            a.Ls = fs.FLsA;
-            CFFT_HIP(fs.fixed_a->launch_a(inb, midb, a, fs.a.dtw.p, st));
-        } else if (p.half) {
-            CFFT_HIP(launch_fourstep_a_f16(inb, midb, a, fs.a.pt, fs.a.dtw.p, st));
-        } else if (fs.pair_a && al16(inb) && al16(midb) && idist % 2 == 0 && mdist % 2 == 0) {
-            a.Ls = fs.LsA2;
-            CFFT_HIP(launch_fourstep_a_pair(inb, midb, a, fs.a.pt, fs.a.dtw.p, st));
-        } else if (fs.pipe_a > 0) {
-            a.grid = (int)std::min<int64_t>(fs.pipe_a, (int64_t)((fs.N2 + fs.CA - 1) / fs.CA) * nb);
-            CFFT_HIP(launch_fourstep_a_pipe(p.prec, inb, midb, a, fs.a.pt, fs.a.dtw.p,
-                                            fs.a.dtw.bytes / (size_t)es_, st));
-        } else {
-            CFFT_HIP(launch_fourstep_a(p.prec, inb, midb, a, fs.a.pt, fs.a.dtw.p, st));
-        }
-        FourStepBArgs b{};
-        b.N1 = fs.N1;
-        b.N2 = fs.N2;
-        b.C = fs.CB;
-        b.Tt = fs.b.Tt;
-        b.Ls = fs.b.Ls;
-        b.E = fs.b.E;
-        b.batch = nb;
-        b.idist = mdist;
-        b.odist = odist;
-        b.sgn_in = 1;
-        b.sgn_out = sgn;
-        b.scale = scale;
-        b.epi = epi;
-        if (epi.dc) b.epi.dc = (char*)epi.dc + (size_t)b0 * 2 * es;
-        b.tbits = fs.tbits;
-        b.tnc = fs.tnc;
-        b.tw3 = fs.tw3.p;
-        b.xcd = 1;
-        if (fs.fixed_b && !epi.K && fits(fs.fixed_b, midb, mdist, es) &&
-            fits(fs.fixed_b, outb, odist, eio)) {
-            b.C = fs.FCB;
-            b.Ls = fs.FLsB;
-            CFFT_HIP(fs.fixed_b->launch_b(midb, outb, b, fs.b.dtw.p, st));
-        } else if (p.half) {
-            CFFT_HIP(launch_fourstep_b_f16(midb, outb, b, fs.b.pt, fs.b.dtw.p, st));
-        } else if (fs.pair_b && !epi.K && al16(midb) && al16(outb) && mdist % 2 == 0 &&
-                   odist % 2 == 0) {
-            b.Ls = fs.LsB2;
-            CFFT_HIP(launch_fourstep_b_pair(midb, outb, b, fs.b.pt, fs.b.dtw.p, st));
-        } else if (fs.pipe_b > 0 && !epi.K) {
-            b.grid = (int)std::min<int64_t>(fs.pipe_b, (int64_t)((fs.N1 + fs.CB - 1) / fs.CB) * nb);
-            CFFT_HIP(launch_fourstep_b_pipe(p.prec, midb, outb, b, fs.b.pt, fs.b.dtw.p,
-                                            fs.b.dtw.bytes / (size_t)es_, st));
-        } else {
-            CFFT_HIP(launch_fourstep_b(p.prec, midb, outb, b, fs.b.pt, fs.b.dtw.p, st));
-        }
+        int rc = fourstep_pass_a(p, inb, midb, idist, mdist, sgn, st, nb);
+        if (rc) return rc;
+        ConvEpilogue e = epi;
+        if (e.dc) e.dc = (char*)epi.dc + (size_t)b0 * 2 * es;
+        if ((rc = fourstep_pass_b(p, midb, outb, mdist, odist, sgn, scale, e, st, nb))) return rc;
     }
     return CFFT_OK;
 }
@@ -2046,6 +2063,34 @@ int plan_nd_create(Ctx* ctx, int rank, const int64_t* dims, int64_t axes_mask, i
 }
 
 // ------------------------------------------------------------------------------- real input
+// The real-input passes of a four-step on fixed lines (fixed_real.h), for both directions or
+// none: tiles of 16 (pass B) and 8 lines, halved until they fit.
+static void real_fixed_setup(Ctx* ctx, Plan& p) {
+    const Plan& f = *p.rsub_fwd;
+    const FourStepPlan& fs = f.fs;
+    // both passes' own kernels, so that the sub-plans run unchunked default shapes
+    if (f.kind != Kind::FourStep || p.rsub_bwd->kind != Kind::FourStep || !fs.fixed_a ||
+        !fs.fixed_b || !p.rsub_bwd->fs.fixed_b || p.rsub_bwd->fs.N1 != fs.N1)
+        return;
+    const FixedReal* rb = find_fixed_real(p.prec, fs.b.pt, fs.N2);
+    const FixedReal* ra = find_fixed_real(p.prec, fs.a.pt, fs.N1);
+    if (!ra || !rb) return;
+    const size_t table = (size_t)tw3_entries(fs.tbits, fs.tnc) * esize(p.prec) + 16;
+    auto tile = [&](const FixedReal& r, int c, size_t reserve, int* Ls) {
+        const size_t per = (size_t)r.elem * ((r.pad < 0 ? r.N : r.N + (r.N >> r.pad)) + 64);
+        while (c > 1 && (c * r.Tt > r.max_threads || c * per + reserve > ctx->lds_max)) c /= 2;
+        *Ls = fixed_stride(ctx, FixedShape{r.r, r.np, r.N, r.Tt, r.elem, r.pad, false}, c, reserve);
+        return c;
+    };
+    p.frb_c = tile(*rb, 16, table, &p.frb_ls);
+    p.fra_c = tile(*ra, 8, 16, &p.fra_ls);
+    if (p.frb_c < 2) return;
+    ra->prepare();
+    rb->prepare();
+    p.freal_a = ra;
+    p.freal_b = rb;
+}
+
 // rfft / brfft / irfft (AbstractFFTs' real transforms; the reference's plan_rfft / plan_brfft
 // stubs at CatabraFFT.jl:199-208 build nothing usable).  Even n reads the reals as n/2 complex
 // values and untangles the spectrum with w^k = e^{-2 pi i k/n}; odd n goes through a full
@@ -2096,6 +2141,7 @@ int plan_real_create(Ctx* ctx, int64_t n, int64_t batch, int64_t rdist, int64_t 
         } else {
             if ((rc = sub(m, rdist / 2, m, p->rsub_fwd))) return rc;
             if ((rc = sub(m, m, rdist / 2, p->rsub_bwd))) return rc;
+            real_fixed_setup(ctx, *p);
             if ((rc = p->rs1.alloc((size_t)std::max<int64_t>(batch, 1) * m * es))) return rc;
             p->real = 2;
         }
@@ -2114,7 +2160,7 @@ int plan_real_create(Ctx* ctx, int64_t n, int64_t batch, int64_t rdist, int64_t 
         for (int i = 0; i < p->line.pt.npass; ++i) os << (i ? "," : "") << p->line.pt.radix[i];
         os << "] C=" << p->C;
     } else {
-        os << "{" << plan_description(*p->rsub_fwd) << "}";
+        os << (p->freal_b ? "fused ends " : "") << "{" << plan_description(*p->rsub_fwd) << "}";
     }
     p->desc = os.str();
     *out = p;
@@ -2162,6 +2208,40 @@ static int real_exec(const Plan& p, const void* in, void* out, int direction, in
         return CFFT_OK;
     }
     int rc;
+    if (p.freal_b && fwd) {
+        const Plan& s = *p.rsub_fwd;
+        const FourStepPlan& fs = s.fs;
+        if ((rc = fourstep_pass_a(s, in, p.rs1.p, rdist / 2, m, 1, st, p.batch))) return rc;
+        FourStepBArgs b{};
+        b.N1 = fs.N1;
+        b.N2 = fs.N2;
+        b.C = p.frb_c;
+        b.Ls = p.frb_ls;
+        b.batch = p.batch;
+        b.idist = m;
+        b.odist = cdist;
+        b.tbits = fs.tbits;
+        b.tnc = fs.tnc;
+        b.tw3 = fs.tw3.p;
+        b.xcd = 1;
+        CFFT_HIP(p.freal_b->launch_b(p.rs1.p, out, b, p.rw.p, fs.b.dtw.p, st));
+        return CFFT_OK;
+    }
+    if (p.freal_a && !fwd) {
+        const Plan& s = *p.rsub_bwd;
+        const FourStepPlan& fs = s.fs;
+        FourStepAArgs a{};
+        a.N1 = fs.N1;
+        a.N2 = fs.N2;
+        a.C = p.fra_c;
+        a.Ls = p.fra_ls;
+        a.batch = p.batch;
+        a.idist = cdist;
+        a.odist = m;
+        a.xcd = 1;
+        CFFT_HIP(p.freal_a->launch_a(in, p.rs1.p, a, scale, p.rw.p, fs.a.dtw.p, st));
+        return fourstep_pass_b(s, p.rs1.p, out, m, rdist / 2, -1, 1.0, none, st, p.batch);
+    }
     if (p.real == 2) {
         if (fwd) {
             if ((rc = run_fft(*p.rsub_fwd, in, p.rs1.p, 1, 1.0, none, st))) return rc;

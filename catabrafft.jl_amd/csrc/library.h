@@ -111,6 +111,10 @@ struct Plan {
     // cdist (complex elements)
     int real = 0;
     DevBuf rw, rs1, rs2;
+    // real = 2 over a four-step: the forward transform's pass B and the backward one's pass A on
+    // fixed lines, their tiles and LDS line strides (nullptr: elementwise passes of their own)
+    const FixedReal *freal_b = nullptr, *freal_a = nullptr;
+    int frb_c = 0, frb_ls = 0, fra_c = 0, fra_ls = 0;
     std::unique_ptr<Plan> rsub_fwd, rsub_bwd;
     // uneven batch
     std::vector<std::unique_ptr<Plan>> parts;

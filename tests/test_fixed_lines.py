@@ -340,3 +340,57 @@ def test_fixed_large_convolutions(gpu_ready, dt, lo, hi, count):
         ref = np.fft.ifft(x[o:o + n].cpu().numpy().astype(np.clongdouble))
         err = float(np.linalg.norm(rows[-1].cpu().numpy() - ref) / np.linalg.norm(ref))
         assert err < _bound(n, dt), (n, err)
+
+
+# ------------------------------------------------------------------------------ real input
+def _check_real(n, batch, dt, forward, backward):
+    """rfft and irfft of `batch` rows against numpy in long double, at the parity bounds."""
+    rng = np.random.Generator(np.random.PCG64(n))
+    x = rng.standard_normal((batch, n)).astype(dt)
+    bound = 1e-6 if dt == np.float32 else 4 * np.finfo(float).eps * np.log2(n)
+    ref = np.fft.rfft(x.astype(np.longdouble), axis=-1)
+    got = forward(x)
+    assert float(np.linalg.norm(got - ref) / np.linalg.norm(ref)) < bound, n
+    # the transform of a spectrum whose ends are real, as numpy takes them to be
+    X = (rng.standard_normal(got.shape) + 1j * rng.standard_normal(got.shape)).astype(got.dtype)
+    X[:, 0] = X[:, 0].real
+    X[:, -1] = X[:, -1].real
+    ref = np.fft.irfft(X.astype(np.clongdouble), n, axis=-1)
+    got = backward(X)
+    assert float(np.linalg.norm(got - ref) / np.linalg.norm(ref)) < bound, n
+
+
+@pytest.mark.parametrize("n,dt", [(2 * 1024 * 256, np.float32), (2 * 1024 * 128, np.float64)])
+def test_emulated_real_four_step_ends(emu, tmp_path, n, dt):
+    ctx, p, batch = ctypes.c_void_p(), ctypes.c_void_p(), 2
+    cdt = np.complex64 if dt == np.float32 else np.complex128
+    assert emu.cfft_init(0, ctypes.byref(ctx)) == 0
+    assert emu.cfft_plan_1d_real(ctx, n, batch, n, n // 2 + 1, 0 if dt == np.float32 else 1, 0,
+                                 ctypes.byref(p)) == 0
+    assert "fused ends" in _desc(emu, p), _desc(emu, p)
+
+    def run(a, out, direction):
+        assert emu.cfft_exec(p, a.ctypes.data, out.ctypes.data, direction, 1, None) == 0
+        return out
+
+    _check_real(n, batch, dt, lambda x: run(x, np.zeros((batch, n // 2 + 1), cdt), -1),
+                lambda X: run(X, np.zeros((batch, n), dt), 1))
+    emu.cfft_plan_destroy(p)
+    emu.cfft_finalize(ctx)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_real_four_step_ends(gpu_ready, dt):
+    import torch
+
+    import catabrafft as C
+
+    for m in (16807, 19683, 24000, 32768, 34300, 46656, 50625, 65536, 78125, 131072, 10 ** 6,
+              1 << 20, 2 * 3 ** 12):
+        p = C.RealPlan(2 * m, 3, dt)
+        print(p.describe(), flush=True)
+        assert "fused ends" in p.describe(), p.describe()
+        _check_real(2 * m, 3, dt,
+                    lambda x: p.forward_torch(torch.from_numpy(x).cuda()).cpu().numpy(),
+                    lambda X: p.backward_torch(torch.from_numpy(X).cuda(), True).cpu().numpy())
