@@ -35,11 +35,28 @@ struct FixedRowDst {
 // their butterflies: F32 512 30.6 us at 16 against 36.4 at 12 (37.0), 2048 33.5 against 35.9
 // (37.9); F64 1920 65.7 against 70.9 (101.8), 3840 74.6 against 80.6 (110.7).  At 12: F32 2520
 // 37.4 us (45.5), 720 34.7 (45.8), 3000 41.5 (65.7); F64 2520 79.9 (105.1), 360 61.7 (108.8).
+//
+// Batches larger than the Infinity Cache (30 x 2^20 elements in F32, 15 in F64) are less forgiving:
+// - lines under 192 points take 8, as many threads as the run-time kernel, whose stores run over
+//   more lanes: F32 64 144 us (208 at 12; run-time 149), 96 92 (148; 97); F64 48 119 (141; 119);
+// - F32 lines of radix 16 take 8 where 12 leaves more than a tenth of the waves' lanes without a
+//   thread: 384 125 us (149 at 12; run-time 128), 640 106 (126; 115), 960 96 (115; 107), 720 105
+//   (116; 127); where it does not, 12 stays better: 320 99 (142 at 8; 143), 1280 103 (117; 114).
+constexpr int lanes_percent(int TT) {
+    return TT <= 64 ? 64 / TT * TT * 100 / 64 : TT * 100 / ((TT + 63) / 64 * 64);
+}
 template <typename T, class Q>
 constexpr int fixed_row_capacity() {
+    if (Q::N < 192) return 8;
     if (sizeof(T) == 8 && Q::has(16)) return 16;
     if (Q::threads(12) > 1024) return 16;
-    return sizeof(T) == 4 && (Q::N & (Q::N - 1)) == 0 && Q::N >= 512 ? 16 : 12;
+    if (sizeof(T) == 8) return 12;
+    if ((Q::N & (Q::N - 1)) == 0) return Q::N >= 512 ? 16 : 12;
+    const int t8 = Q::threads(8), t12 = Q::threads(12);
+    return Q::has(16) && t8 <= 1024 && lanes_percent(t12) < 90 &&
+                   lanes_percent(t8) > lanes_percent(t12)
+               ? 8
+               : 12;
 }
 
 // a.C lines per workgroup, a.Tt = TT threads and a.Ls LDS elements each.  Bound by HBM: 2520 x

@@ -409,12 +409,19 @@ static int plan_direct(Ctx* ctx, Plan& p, int E, int target_threads, int pipe = 
                                target_threads);
     p.pipe_res = pipe > 0 ? pipe_resident(ctx, p) : 0;
     p.kind = Kind::Direct;
-    // A default plan's line takes its own kernel where there is one (every 7-smooth length from
-    // 16 to 8192; float and double storage).  On 15 lengths from 128 to 4096, 10.5 million
+    // A default plan's line takes its own kernel where there is one (7-smooth lengths from 16 to
+    // 8192; float and double storage).  On 15 lengths from 128 to 4096, 10.5 million
     // elements each, it is 1.0-1.6x as fast as the run-time kernel in F32 and 1.0-1.8x in F64
     // (1.0: short powers of two, at the copy rate either way).
     if (fixed && !p.half && !p.line.pt.wave && p.line.pad && !p.pipe_res) {
-        const FixedRow* f = find_fixed_row(p.prec, p.line.pt, (int)p.n);
+        // But not F64 lines of radix 16 and one more pass below 192 points (15 x 2^20 elements, n = 64:
+        // 103 us against 95, 112: 105 / 99, 144: 102 / 94, 48 and 128 the same), nor powers of two
+        // from 4096 in F32 (30 x 2^20 elements, 4096: 107 / 101, 8192: 124 / 123): both kernels run at
+        // the copy rate there.
+        const bool at_rate = p.prec == Prec::F64
+                                 ? p.n < 192 && p.line.pt.npass == 2 && p.line.pt.radix[0] == 16
+                                 : p.n >= 4096 && (p.n & (p.n - 1)) == 0;
+        const FixedRow* f = at_rate ? nullptr : find_fixed_row(p.prec, p.line.pt, (int)p.n);
         const size_t fper = f ? (size_t)esize(p.prec) * f->Ls : 0;
         if (f && fper <= ctx->lds_max) {
             int c = std::max(1, target_threads / f->Tt);

@@ -62,6 +62,14 @@ def _desc(lib, p):
     return buf.value.decode()
 
 
+def _run_time_row(n, dt, desc):
+    """Short F64 lines of radix 16 and one more pass, and long F32 powers of two, keep the run-time
+    kernel."""
+    if dt == np.complex128:
+        return n < 192 and re.search(r"direct \[16,\d+\]", desc) is not None
+    return n >= 4096 and n & (n - 1) == 0
+
+
 @pytest.mark.parametrize("dt", [np.complex64, np.complex128])
 @pytest.mark.parametrize("n", FEW)
 def test_emulated_fixed_rows_match_the_run_time_kernel(emu, tmp_path, n, dt):
@@ -78,7 +86,7 @@ def test_emulated_fixed_rows_match_the_run_time_kernel(emu, tmp_path, n, dt):
         p = ctypes.c_void_p()
         assert emu.cfft_plan_1d(ctx, n, batch, idist, odist, code, flags, ctypes.byref(p)) == 0
         d = _desc(emu, p)
-        assert ("fixed" in d) == (flags == 0), d
+        assert ("fixed" in d) == (flags == 0 and not _run_time_row(n, dt, d)), d
         got[flags] = []
         for direction, norm in ((-1, 0), (1, 1)):
             y = np.full((batch, odist), 7, dtype=dt)
@@ -106,7 +114,9 @@ def test_fixed_rows_match_the_run_time_kernel(gpu_ready, tmp_path, dt):
         print(f"fixed rows n={n} {np.dtype(dt)}", flush=True)
         x = torch.from_numpy(seeded_complex(n, batch=batch, seed=n, dtype=dt)).cuda()
         p, q = C.Plan(n, batch, dt), C.Plan(n, batch, dt, flags=C.MEASURE)
-        assert "fixed" in p.describe() and "fixed" not in q.describe(), (p.describe(), q.describe())
+        fixed = not _run_time_row(n, dt, p.describe())
+        assert ("fixed" in p.describe()) == fixed and "fixed" not in q.describe(), (
+            p.describe(), q.describe())
         for direction, norm in ((-1, False), (1, True)):
             a = p.exec_torch(x, direction=direction, normalize=norm)
             b = q.exec_torch(x, direction=direction, normalize=norm)
