@@ -83,9 +83,12 @@ template <typename T, class Q>
 struct FixedRowOf {
     static constexpr int TT = Q::threads(fixed_row_capacity<T, Q>());
     static constexpr int Ls = fixed_line_elems<Q>() | 1;  // odd: lines start in different banks
+    // what k_rows_fixed is compiled for: one line where TT > 128, else up to 256 threads
+    static constexpr int max_lines = TT > 128 ? 1 : 256 / TT;
     static_assert(TT <= 1024, "a line runs on one workgroup");
     static hipError_t launch(const void* in, void* out, const RowsArgs& a, const void* tw,
                              hipStream_t st) {
+        if (a.C < 1 || a.C > max_lines) return hipErrorInvalidValue;
         const size_t lds = sizeof(V_t<T>) * (size_t)a.C * Ls;
         const int64_t blocks = (a.nlines + a.C - 1) / a.C;
         hipLaunchKernelGGL((k_rows_fixed<T, Q, TT>), dim3((unsigned)blocks), dim3(a.C * TT), lds,
@@ -93,7 +96,7 @@ struct FixedRowOf {
         return hipGetLastError();
     }
     static void prepare() { detail::allow_big_lds(k_rows_fixed<T, Q, TT>); }
-    static FixedRow row() { return FixedRow{Q::r, Q::np, Q::N, TT, Ls, launch, prepare}; }
+    static FixedRow row() { return FixedRow{Q::r, Q::np, Q::N, TT, Ls, max_lines, launch, prepare}; }
 };
 
 }  // namespace cfft

@@ -130,6 +130,33 @@ def test_fixed_rows_match_the_run_time_kernel(gpu_ready, tmp_path, dt):
         assert err < (1e-6 if code == 0 else 4 * np.finfo(float).eps * np.log2(n)), (n, err)
 
 
+@pytest.mark.parametrize("threads", [64, 256, 512, 1024])
+@pytest.mark.parametrize("n,dt", [(16, np.complex64), (1024, np.complex128), (720, np.complex64),
+                                  (2520, np.complex64), (2520, np.complex128)])
+def test_emulated_fixed_rows_at_any_thread_count(emu, tmp_path, n, dt, threads):
+    """A plan that asks for the default capacity and its own thread count: kernels of 1 to 64
+    lines a workgroup, on both sides of one line per workgroup."""
+    code, batch = (0 if dt == np.complex64 else 1), 70
+    w = tmp_path / "w.txt"
+    w.write_text(f"{n} {batch} {n} {n} {code} 1 : 0 {threads} 0 0 0 -1 0 0\n")
+    ctx, p = ctypes.c_void_p(), ctypes.c_void_p()
+    assert emu.cfft_init(0, ctypes.byref(ctx)) == 0
+    assert emu.cfft_wisdom_import(ctx, str(w).encode()) == 0
+    assert emu.cfft_plan_1d(ctx, n, batch, n, n, code, 1, ctypes.byref(p)) == 0
+    d = _desc(emu, p)
+    tt, c = map(int, re.search(r"fixed Tt=(\d+) C=(\d+)", d).groups())
+    # the kernels' launch bounds: 256 threads, or one line of more
+    assert 1 <= c and (c == 1 if tt > 128 else c * tt <= 256), d
+    x = seeded_complex(n, batch=batch, seed=n, dtype=dt)
+    y = np.zeros_like(x)
+    assert emu.cfft_exec(p, x.ctypes.data, y.ctypes.data, -1, 0, None) == 0
+    ref = np.fft.fft(x.astype(np.clongdouble))
+    bound = 1e-6 if code == 0 else 4 * np.finfo(float).eps * np.log2(n)
+    assert float(np.linalg.norm(y - ref) / np.linalg.norm(ref)) < bound, d
+    emu.cfft_plan_destroy(p)
+    emu.cfft_finalize(ctx)
+
+
 # ------------------------------------------------------------------------------ four-step passes
 FS_FEW = _lengths("CFFT_FS_LINES_FEW")
 FS_ALL = _lengths("CFFT_FS_LINES")
