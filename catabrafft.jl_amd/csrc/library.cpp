@@ -1103,7 +1103,7 @@ static int plan_conv(Ctx* ctx, Plan& p, const PlanOptions& o) {
             const size_t per = (size_t)esize(p.prec) * (p.LsC + 1);
             if (per <= ctx->lds_max) {
                 small = true;
-                int c = std::max(1, o.target_threads / f->Tt);
+                int c = std::max(1, std::min(o.target_threads, f->max_threads) / f->Tt);
                 c = std::min<int64_t>(c, std::max<size_t>(1, std::max(ctx->lds_rows_budget, per) / per));
                 p.C = (int)std::min<int64_t>(c, std::max<int64_t>(1, p.batch));
                 p.fconv = f;

@@ -282,6 +282,30 @@ def test_emulated_fixed_convolutions(emu, dt):
     emu.cfft_finalize(ctx)
 
 
+@pytest.mark.parametrize("threads", [64, 512, 1024])
+@pytest.mark.parametrize("n,dt", [(19, np.complex64), (239, np.complex128), (1013, np.complex64)])
+def test_emulated_fixed_convolutions_at_any_thread_count(emu, tmp_path, n, dt, threads):
+    """A plan that asks for the default capacity and its own thread count keeps to the workgroups
+    its kernel is compiled for (512 threads in a work list, 1024 of a longer line)."""
+    code, batch = (0 if dt == np.complex64 else 1), 40 if n > 100 else 1000
+    w = tmp_path / "w.txt"
+    w.write_text(f"{n} {batch} {n} {n} {code} 1 : 0 {threads} 0 0 0 -1 0 0\n")
+    ctx, p = ctypes.c_void_p(), ctypes.c_void_p()
+    assert emu.cfft_init(0, ctypes.byref(ctx)) == 0
+    assert emu.cfft_wisdom_import(ctx, str(w).encode()) == 0
+    assert emu.cfft_plan_1d(ctx, n, batch, n, n, code, 1, ctypes.byref(p)) == 0
+    d = _desc(emu, p)
+    c, tt = map(int, re.search(r" C=(\d+) fixed Tt=(\d+)", d).groups())
+    assert 1 <= c and (c == 1 or c * tt <= 512), d
+    x = seeded_complex(n, batch=batch, seed=n, dtype=dt)
+    y = np.zeros_like(x)
+    assert emu.cfft_exec(p, x.ctypes.data, y.ctypes.data, -1, 0, None) == 0
+    ref = np.fft.fft(x.astype(np.clongdouble))
+    assert float(np.linalg.norm(y - ref) / np.linalg.norm(ref)) < _bound(n, dt), d
+    emu.cfft_plan_destroy(p)
+    emu.cfft_finalize(ctx)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", [np.complex64, np.complex128])
 def test_fixed_convolutions(gpu_ready, dt):
