@@ -244,6 +244,7 @@ static void copy_shape(const Plan& from, Plan& to) {
     to.dtype = from.dtype;
     to.flags = from.flags;
     to.prec = from.prec;
+    to.half = from.half;
 }
 
 // ------------------------------------------------------------------------------- wisdom
@@ -422,7 +423,7 @@ int autotune(Ctx* ctx, Plan& p, int flags, const PlanOptions& base) {
     }
     std::vector<PlanOptions> cands = candidates(ctx, p, flags);
     if (cands.size() <= 1 || p.batch == 0) return plan_build(ctx, p, base);
-    const size_t es = p.prec == Prec::F32 ? 8 : 16;
+    const size_t es = p.half ? 4 : p.prec == Prec::F32 ? 8 : 16;
     // time on the real shape, but never on more than 1 GiB per buffer
     int64_t tb = p.batch;
     const size_t per_in = (size_t)p.idist * es, per_out = (size_t)p.odist * es;

@@ -407,7 +407,7 @@ static int plan_direct(Ctx* ctx, Plan& p, int E, int target_threads, int pipe = 
     if (per > ctx->lds_max) return fail(CFFT_ERR_UNSUPPORTED, "line does not fit LDS");
     p.C = rows_lines_per_block(p.line, p.prec, p.batch, std::max<size_t>(per, ctx->lds_rows_budget),
                                target_threads);
-    p.pipe_res = pipe > 0 ? pipe_resident(ctx, p) : 0;
+    p.pipe_res = pipe > 0 && !p.half ? pipe_resident(ctx, p) : 0;
     p.kind = Kind::Direct;
     // A default plan's line takes its own kernel where there is one (7-smooth lengths from 16 to
     // 8192; float and double storage).  On 15 lengths from 128 to 4096, 10.5 million
@@ -1114,7 +1114,7 @@ static int plan_conv(Ctx* ctx, Plan& p, const PlanOptions& o) {
     if (!small && p.cprec == p.prec && line_fits(ctx, p.L, p.prec, E)) {
         rc = make_line(p.line, p.L, p.prec, E, 1024);
         if (rc) return rc;
-        if (!p.half && (o.wave > 0 || (o.wave < 0 && kWaveDefault))) apply_wave_tail(p.line);
+        if (o.wave > 0 || (o.wave < 0 && kWaveDefault)) apply_wave_tail(p.line);
         // the input lines and the convolution work share one LDS line (the kernel saves x0 and
         // separates reads from writes where they overlap)
         p.LsC = std::max(line_stride_for(p.prec, n), p.line.Ls);
@@ -1227,6 +1227,7 @@ static int64_t default_chunk(const Plan& p) {
 static void fs_pipe_setup(Ctx* ctx, Plan& p, int mask) {
     FourStepPlan& fs = p.fs;
     fs.pipe_a = fs.pipe_b = 0;
+    if (p.half) return;  // (nor line pairs: ComplexF16 lines run the plain kernels or their own)
     for (int pass = 0; pass < 2; ++pass) {
         if (!((mask >> pass) & 1)) continue;
         const LinePlan& lp = pass ? fs.b : fs.a;
@@ -1244,7 +1245,7 @@ static void fs_pipe_setup(Ctx* ctx, Plan& p, int mask) {
 // The passes' own kernels for a default four-step plan, at its tiles.
 static void fs_fixed_setup(Ctx* ctx, Plan& p) {
     FourStepPlan& fs = p.fs;
-    const bool f64 = p.prec == Prec::F64, half = p.dtype == CFFT_C16;
+    const bool f64 = p.prec == Prec::F64, half = p.half;
     auto kind = [&](int across) {  // `across`: lines side by side (the pairs' count is even)
         if (f64) return FixedFsKind::F64;
         if (half) return FixedFsKind::F16Pair;
@@ -1269,7 +1270,7 @@ static void fs_fixed_setup(Ctx* ctx, Plan& p) {
 static void fs_pair_setup(Ctx* ctx, Plan& p, int mask) {
     FourStepPlan& fs = p.fs;
     fs.pair_a = fs.pair_b = 0;
-    if (p.prec != Prec::F32) return;
+    if (p.prec != Prec::F32 || p.half) return;
     if ((mask & 1) && fs.pipe_a == 0 && fs.CA >= 2 && fs.CA % 2 == 0 && fs.N2 % 2 == 0) {
         fs.LsA2 = fs_line_stride(ctx, Prec::F64, fs.a, fs.CA / 2, 16);
         fs.pair_a = fs_pair_lds(0, fs.CA, fs.LsA2, 0, 0, false) <= ctx->lds_max;
@@ -2298,6 +2299,7 @@ int plan_create(Ctx* ctx, int64_t n, int64_t batch, int64_t idist, int64_t odist
     p->dtype = dtype;
     p->flags = flags;
     p->prec = dtype == CFFT_C64 ? Prec::F64 : Prec::F32;
+    p->half = dtype == CFFT_C16;  // a float plan with half-precision lines
     CFFT_HIP(hipSetDevice(ctx->device));
     int rc;
     if (flags == CFFT_NO_FLAG || opts.explicit_opts) {
@@ -2306,14 +2308,6 @@ int plan_create(Ctx* ctx, int64_t n, int64_t batch, int64_t idist, int64_t odist
         rc = autotune(ctx, *p, flags, opts);
     }
     if (rc) return rc;
-    if (dtype == CFFT_C16) {  // the float plan with half-precision lines (plain rows kernel)
-        p->half = true;
-        p->pipe_res = 0;
-        p->fixed = nullptr;
-        p->fs.pipe_a = p->fs.pipe_b = 0;
-        p->fs.pair_a = p->fs.pair_b = 0;
-        p->desc.clear();
-    }
     if (p->desc.empty()) p->desc = describe(*p);
     *out = p;
     return CFFT_OK;

@@ -375,3 +375,46 @@ def test_emulated_f16_sixstep_through_wisdom(E, tmp_path):
     for p in ps.values():
         lib.cfft_plan_destroy(p)
     lib.cfft_finalize(c2)
+
+
+@pytest.mark.timeout(120)
+@pytest.mark.parametrize("n,batch", [(64, 3), (1024, 2), (31250, 1)])
+def test_emulated_f16_tuning_times_half_plans(E, capfd, monkeypatch, n, batch):
+    """MEASURE times ComplexF16 candidates as ComplexF16 plans: half-precision lines on the kernels
+    the finished plan runs (no float rows kernels of their own, no pipelined or line-pair passes)."""
+    lib, ctx = E
+    monkeypatch.setenv("CFFT_TUNE_VERBOSE", "1")
+    p = ctypes.c_void_p()
+    assert lib.cfft_plan_1d(ctx, n, batch, n, n, C16, 1, ctypes.byref(p)) == 0
+    timed = [s for s in capfd.readouterr().err.splitlines() if s.startswith("tune ")]
+    assert len(timed) > 1
+    for s in timed:
+        assert "io=f16" in s and "pipe" not in s and "pair" not in s, s
+        assert "fixed" not in s or "fourstep" in s, s
+    xh = to_h(seeded_complex(n, batch=batch, seed=n))
+    y = np.zeros_like(xh)
+    assert lib.cfft_exec(p, xh.ctypes.data, y.ctypes.data, -1, 0, None) == 0
+    assert rel_l2(from_h(y), O.fft(from_h(xh), "d", -1, False)) < 2e-3
+    lib.cfft_plan_destroy(p)
+
+
+@pytest.mark.parametrize("n,knobs", [(1024, "16 64 0 0 0 -1 0 0 wv=1"), (1024, "16 64 0 0 0 -1 1 0"),
+                                     (31250, "16 64 250 4 4 -1 1 0"), (257, "16 64 0 0 0 -1 0 0 wv=1")])
+def test_emulated_f16_ignores_float_only_knobs(E, tmp_path, n, knobs):
+    """Wave tails and pipelined kernels asked for through wisdom: direct and four-step ComplexF16
+    lines have none and run their plain kernels, a convolution's staged float lines take them."""
+    lib = E[0]
+    w = tmp_path / "w.txt"
+    w.write_text(f"{n} 2 {n} {n} {C16} 1 : {knobs}\n")
+    ctx, p = ctypes.c_void_p(), ctypes.c_void_p()
+    assert lib.cfft_init(0, ctypes.byref(ctx)) == 0
+    assert lib.cfft_wisdom_import(ctx, str(w).encode()) == 0
+    assert lib.cfft_plan_1d(ctx, n, 2, n, n, C16, 1, ctypes.byref(p)) == 0
+    d = _desc(lib, p)
+    assert "(wisdom)" in d and ("wave" in d) == (n == 257) and "pipe" not in d, d
+    xh = to_h(seeded_complex(n, batch=2, seed=n))
+    y = np.zeros_like(xh)
+    assert lib.cfft_exec(p, xh.ctypes.data, y.ctypes.data, -1, 0, None) == 0
+    assert rel_l2(from_h(y), O.fft(from_h(xh), "d", -1, False)) < 2e-3, d
+    lib.cfft_plan_destroy(p)
+    lib.cfft_finalize(ctx)
