@@ -1374,7 +1374,10 @@ static int plan_fft_core(Ctx* ctx, Plan& p, const PlanOptions& o) {
         const int pair = o.pair >= 0 ? o.pair
                                      : (p.prec != Prec::F32 ? 0 : (p.fs.a.E == 8 ? 3 : 1));
         if (pair > 0) fs_pair_setup(ctx, p, pair);
-        if (!o.E && !o.Eb && o.pair < 0 && !pipe_mask && chunk == 0) fs_fixed_setup(ctx, p);
+        // the passes' own kernels have their own tiles: a plan with a knob of the run-time passes
+        // runs as asked
+        if (!o.E && !o.Eb && !o.ca && !o.cb && o.pair < 0 && !pipe_mask && chunk == 0)
+            fs_fixed_setup(ctx, p);
         return CFFT_OK;
     }
     return plan_conv(ctx, p, o);

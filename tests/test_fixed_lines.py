@@ -198,6 +198,20 @@ def test_emulated_fixed_four_step_matches_the_run_time_kernels(emu, tmp_path, n1
         assert np.array_equal(y0, y1) and np.array_equal(x0, x1), (a, b, dist)
 
 
+@pytest.mark.parametrize("dt", [np.complex64, np.complex128])
+@pytest.mark.parametrize("ca,cb", [(2, 0), (0, 8), (8, 4)])
+def test_emulated_four_step_keeps_the_tiles_it_is_given(emu, tmp_path, dt, ca, cb):
+    """Tiles asked for through wisdom at the default capacity are the ones that run, with the
+    default tiles' bits."""
+    n1, n2 = 256, 128
+    d0, y0, x0 = _emu_four_step(emu, tmp_path, n1, n2, 2, dt, OWN, n1 * n2, 0)
+    d1, y1, x1 = _emu_four_step(emu, tmp_path, n1, n2, 2, dt, f"0 64 {{n1}} {ca} {cb} -1 -1 0",
+                                n1 * n2, 0)
+    assert "fixed=AB" in d0 and "fixed" not in d1, (d0, d1)
+    assert (not ca or f" CA={ca} " in d1) and (not cb or f" CB={cb} " in d1), d1
+    assert np.array_equal(y0, y1) and np.array_equal(x0, x1)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", [np.complex64, np.complex128])
 def test_fixed_four_step_matches_the_run_time_kernels(gpu_ready, tmp_path, dt):
