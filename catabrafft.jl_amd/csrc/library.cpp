@@ -776,13 +776,8 @@ static int plan_large(Ctx* ctx, Plan& p, const PlanOptions& o) {
 }
 
 
-// Convolution data of a Rader (prime n) or Bluestein transform: permutations or chirp, and the
-// zero-padded kernel b whose spectrum the convolution multiplies by.
-// Length of a convolution that needs at least m points: the shortest of the fixed kernels' lengths
-// where there is one (they are the lengths that no longer one with fewer passes beats), else the
-// shortest 7-smooth one.
-// Beyond the fused lengths: the cheapest product of two lines of the fixed large convolutions
-// (points times the passes over them, and six for the work lines' trips through memory).
+// A length of the fixed large convolutions, the product of two of their lines, and its cost: points
+// times the passes over them, and six for the work lines' trips through memory.
 struct ConvSplit {
     int64_t L = 0;
     int N1 = 0, N2 = 0;
@@ -829,15 +824,22 @@ static ConvSplit conv_split_of(int64_t L, Prec prec) {
                 best = ConvSplit{L, a, b, 0};
     return best;
 }
-static int64_t conv_length(int64_t m, Prec prec) {
-    if (const FixedConv* f = find_fixed_conv(prec, m, false)) return f->N;
+// Length of a convolution that needs at least m points: the shortest of the fixed kernels' lengths
+// that the plan may run (fused: the lengths that no longer one with fewer passes beats; large: the
+// cheapest product of two lines), else the shortest 7-smooth one.
+static int64_t conv_length(int64_t m, Prec prec, ConvKernels own) {
+    const FixedConv* f = find_fixed_conv(prec, m, false);
+    if (f) return own.fused ? f->N : next_smooth(m);
+    if (!own.large) return next_smooth(m);
     const std::vector<ConvSplit>& v = conv_splits();
     const auto it = std::lower_bound(v.begin(), v.end(), m,
                                      [](const ConvSplit& c, int64_t x) { return c.L < x; });
     return it != v.end() ? it->L : next_smooth(m);
 }
 
-int conv_data(int64_t n, Prec prec, ConvData& d) {
+// Convolution data of a Rader (prime n) or Bluestein transform: permutations or chirp, and the
+// zero-padded kernel b whose spectrum the convolution multiplies by.
+int conv_data(int64_t n, Prec prec, ConvKernels own, ConvData& d) {
     const bool rader = is_prime(n);
     d.mode = rader ? ConvMode::Rader : ConvMode::Bluestein;
     d.perm.clear();
@@ -849,8 +851,9 @@ int conv_data(int64_t n, Prec prec, ConvData& d) {
         // length that has one then costs no more (F32 rows: n = 1031 at L = 2304 1.35 TB/s, n = 2003
         // at L = 2002 on the run-time kernel 1.31; n = 4099 at 9216 0.99, n = 3001 at 3000 1.29),
         // and spares a work list the launches of the few run-time convolutions
-        const bool exact = is_smooth(N) && (N > 2048 || find_fixed_conv(prec, N, true));
-        d.L = exact ? N : conv_length(2 * N - 1, prec);
+        const bool exact = is_smooth(N) &&
+                           (N > 2048 || !own.fused || find_fixed_conv(prec, N, true));
+        d.L = exact ? N : conv_length(2 * N - 1, prec, own);
         const int64_t g = primitive_root(n);
         const int64_t ginv = powmod(g, n - 2, n);
         d.perm.resize(N);
@@ -870,7 +873,7 @@ int conv_data(int64_t n, Prec prec, ConvData& d) {
         for (int64_t m = d.L - N + 1; m < d.L; ++m) d.b[m] = w[m - (d.L - N)];
         d.g = g;
     } else {
-        d.L = conv_length(2 * n - 1, prec);
+        d.L = conv_length(2 * n - 1, prec, own);
         d.chirp.resize(n);
         const OmegaTable om(2 * n);
         for (int64_t m = 0; m < n; ++m) {
@@ -1078,7 +1081,11 @@ static int plan_conv(Ctx* ctx, Plan& p, const PlanOptions& o) {
     const int64_t n = p.n;
     ConvData d;
     p.cprec = conv_precision(n, p.prec, is_prime(n) ? ConvMode::Rader : ConvMode::Bluestein);
-    conv_data(n, p.cprec, d);
+    // the lengths' own kernels, unless the shape is forced
+    const bool asked = o.E && o.explicit_opts;
+    const ConvKernels own{!asked && o.wave <= 0 && !kWaveDefault && p.cprec == p.prec,
+                          !asked && o.fuse_conv != 0 && !o.large};
+    conv_data(n, p.cprec, own, d);
     p.mode = d.mode;
     p.L = d.L;
     p.g = d.g;
@@ -1090,9 +1097,8 @@ static int plan_conv(Ctx* ctx, Plan& p, const PlanOptions& o) {
     // fused small shape?
     const int E = o.E ? o.E : 16;
     bool small = false;
-    // the length's own kernel, unless the shape is forced: 4099 x 4093 lines in ComplexF32 283 us
-    // against 516 on the run-time kernel
-    if (p.cprec == p.prec && o.wave <= 0 && !kWaveDefault && (!o.E || !o.explicit_opts)) {
+    // (4099 x 4093 lines in ComplexF32 283 us against 516 on the run-time kernel)
+    if (own.fused) {
         const FixedConv* f = find_fixed_conv(p.prec, p.L, true);
         if (f) {
             const std::vector<int> rad(f->r, f->r + f->np);
@@ -1130,10 +1136,10 @@ static int plan_conv(Ctx* ctx, Plan& p, const PlanOptions& o) {
             p.C = c;
         }
     }
-    // large, on the fixed kernels, unless the shape is forced: 1.05 to 1.6 times the run-time
-    // kernels' rate over n = 8209 .. 2000003 (ComplexF32 20011 x 512 326 us against 406, 300007 x 16
-    // 315 against 474, 1048573 x 16 1208 against 1266; ComplexF64 100003 x 64 389 against 441)
-    if (!small && o.fuse_conv != 0 && !o.large && (!o.E || !o.explicit_opts)) {
+    // large, on the fixed kernels: 1.05 to 1.6 times the run-time kernels' rate over n = 8209 ..
+    // 2000003 (ComplexF32 20011 x 512 326 us against 406, 300007 x 16 315 against 474, 1048573 x 16
+    // 1208 against 1266; ComplexF64 100003 x 64 389 against 441)
+    if (!small && own.large) {
         rc = plan_fixed_convl(ctx, p, d, o.alloc_work);
         if (rc != CFFT_ERR_UNSUPPORTED) return rc;
     }

@@ -257,9 +257,12 @@ struct ConvData {
     std::vector<int> perm, iperm;
     std::vector<std::complex<long double>> chirp, b;
 };
-// prec: the precision of the convolution (fused convolutions prefer the lengths of its fixed
-// kernels).
-int conv_data(int64_t n, Prec prec, ConvData& d);
+// Which of the fixed convolution kernels a plan may run: its length is then one of theirs.
+struct ConvKernels {
+    bool fused, large;
+};
+// prec: the precision of the convolution.
+int conv_data(int64_t n, Prec prec, ConvKernels own, ConvData& d);
 // K[i] = FFT_L(b)[order[i]] (nullptr: natural order).
 int conv_spectrum(Ctx* ctx, const std::vector<std::complex<long double>>& b, Prec cprec, DevBuf& K,
                   const std::vector<int>* order = nullptr);

@@ -320,6 +320,38 @@ def test_emulated_fixed_convolutions_at_any_thread_count(emu, tmp_path, n, dt, t
     emu.cfft_finalize(ctx)
 
 
+def _next_smooth(m):
+    while not _factor_smooth(m, (2, 3, 5, 7)):
+        m += 1
+    return m
+
+
+@pytest.mark.parametrize("n,dt", [(1031, np.complex64), (4099, np.complex64), (239, np.complex128),
+                                  (34, np.complex128), (8209, np.complex128)])
+@pytest.mark.parametrize("knobs", ["16 64 0 0 0 -1 0 0", "8 128 0 0 0 -1 0 0",
+                                   "0 64 0 0 0 -1 -1 0 wv=1 fc=0"])
+def test_emulated_forced_convolutions_pad_as_little_as_they_can(emu, tmp_path, n, dt, knobs):
+    """Shapes forced through wisdom run the run-time kernels, at the shortest smooth length: the
+    longer lengths of the kernels with compile-time radices are no gain there."""
+    code = 0 if dt == np.complex64 else 1
+    w = tmp_path / "w.txt"
+    w.write_text(f"{n} 2 {n} {n} {code} 1 : {knobs}\n")
+    ctx, p = ctypes.c_void_p(), ctypes.c_void_p()
+    assert emu.cfft_init(0, ctypes.byref(ctx)) == 0
+    assert emu.cfft_wisdom_import(ctx, str(w).encode()) == 0
+    assert emu.cfft_plan_1d(ctx, n, 2, n, n, code, 1, ctypes.byref(p)) == 0
+    d = _desc(emu, p)
+    L = _next_smooth(2 * (n - 1) - 1 if _prime(n) else 2 * n - 1)
+    assert f" L={L} " in d and "fixed" not in d, (L, d)
+    x = seeded_complex(n, batch=2, seed=n, dtype=dt)
+    y = np.zeros_like(x)
+    assert emu.cfft_exec(p, x.ctypes.data, y.ctypes.data, -1, 0, None) == 0
+    ref = np.fft.fft(x.astype(np.clongdouble))
+    assert float(np.linalg.norm(y - ref) / np.linalg.norm(ref)) < _bound(n, dt), d
+    emu.cfft_plan_destroy(p)
+    emu.cfft_finalize(ctx)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", [np.complex64, np.complex128])
 def test_fixed_convolutions(gpu_ready, dt):
