@@ -321,8 +321,10 @@ struct FixedConvOf {
         return hipGetLastError();
     }
     static void prepare() { detail::allow_big_lds(k_conv_fixed<T, Q>); }
-    static FixedConv row() {
-        return FixedConv{Q::r, Q::np, Q::N, TT, SH, fixed_conv_block<T, Q>(), launch, prepare};
+    // unpadded: of the list of exact lengths
+    static FixedConv row(bool unpadded = false) {
+        return FixedConv{Q::r, Q::np, Q::N, TT, SH, fixed_conv_block<T, Q>(), unpadded, launch,
+                         prepare};
     }
 };
 

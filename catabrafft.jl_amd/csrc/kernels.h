@@ -188,15 +188,18 @@ const FixedFs* find_fixed_fs(FixedFsKind kind, const PassTable& pt, int N);
 // Fused convolution over a length N whose radices are compile-time constants (fixed_conv.h), its
 // spectrum in the order of conv_order: Tt threads per line, a.C lines per workgroup of at most
 // max_threads; a.Ls LDS elements per line, at least fixed_at(max(n, N) - 1) + 1 with one pad element
-// per 2^pad (pad < 0: none), and one slot.
+// per 2^pad (pad < 0: none), and one slot.  unpadded: a length n - 1 of a prime n, which nothing
+// pads to.
 struct FixedConv {
     const int* r;
     int np, N, Tt, pad, max_threads;
+    bool unpadded;
     hipError_t (*launch)(const void* in, void* out, const ConvSmallArgs& a, const void* tw,
                          hipStream_t st);
     void (*prepare)();
 };
-// The fixed convolution of the shortest length N >= m (exact: N == m), nullptr where there is none.
+// The fixed convolution of length m (exact), or of the shortest length N >= m that convolutions pad
+// to; nullptr where there is none.
 const FixedConv* find_fixed_conv(Prec p, int64_t m, bool exact);
 
 // The three launches of a large convolution (ConvLArgs) on lines of N points whose radices are

@@ -22,6 +22,8 @@ void init_kernels() {
     init_kernels_fixed_convl_multi_f64_f64();
     init_kernels_fixed_conv_multi_f32();
     init_kernels_fixed_conv_multi_f64();
+    init_kernels_fixed_conv_exact_f32();
+    init_kernels_fixed_conv_exact_f64();
 }
 
 // Fixed kernels by length; each index is built at its first look-up.
@@ -84,11 +86,18 @@ const FixedConv* find_fixed_conv(Prec p, int64_t m, bool exact) {
                   [](const FixedConv& a, const FixedConv& b) { return a.N < b.N; });
         return v;
     };
-    static const std::vector<FixedConv> t[2] = {make(fixed_conv_f32), make(fixed_conv_f64)};
-    const auto& v = t[p == Prec::F64];
-    const auto it = std::lower_bound(v.begin(), v.end(), m,
-                                     [](const FixedConv& a, int64_t x) { return a.N < x; });
-    return it == v.end() || (exact && it->N != m) ? nullptr : &*it;
+    static const std::vector<FixedConv> padded[2] = {make(fixed_conv_f32), make(fixed_conv_f64)};
+    static const std::vector<FixedConv> unpadded[2] = {make(fixed_conv_exact_f32),
+                                                       make(fixed_conv_exact_f64)};
+    auto from = [m](const std::vector<FixedConv>& v) {
+        const auto it = std::lower_bound(v.begin(), v.end(), m,
+                                         [](const FixedConv& a, int64_t x) { return a.N < x; });
+        return it == v.end() ? nullptr : &*it;
+    };
+    const FixedConv* f = from(padded[p == Prec::F64]);
+    if (!exact || (f && f->N == m)) return f;
+    f = from(unpadded[p == Prec::F64]);
+    return f && f->N == m ? f : nullptr;
 }
 
 static const std::vector<FixedConvL>& convl_rows(Prec pio, Prec pc) {
@@ -249,6 +258,9 @@ hipError_t launch_multi(const MultiLaunch& L, const MultiArgs& ma, hipStream_t s
         return L.cprec == (int)Prec::F64 ? convl_fixed_multi_f32_f64(L, ma, st)
                                          : convl_fixed_multi_f32_f32(L, ma, st);
     }
+    if (k == MultiKernel::ConvExact)
+        return L.prec == (int)Prec::F32 ? conv_exact_multi_f32(L, ma, st)
+                                        : conv_exact_multi_f64(L, ma, st);
     if (k == MultiKernel::ConvFixed || k == MultiKernel::ConvFixedWide)
         return L.prec == (int)Prec::F32 ? conv_fixed_multi_f32(L, ma, st)
                                         : conv_fixed_multi_f64(L, ma, st);

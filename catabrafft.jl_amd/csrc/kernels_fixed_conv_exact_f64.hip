@@ -1,0 +1,42 @@
+// kernels_fixed_conv_exact_f64.hip -- fixed fused convolutions (fixed_conv.h) of the lengths n - 1 of
+// short primes n, in F64: alone, and the work-list kernel in which an item runs the body of its
+// plan's length.
+#include "fixed_conv.h"
+
+namespace cfft {
+#define CFFT_CONV(...) rows.push_back(FixedConvOf<double, Rad<__VA_ARGS__>>::row(true));
+void fixed_conv_exact_f64(std::vector<FixedConv>& rows) {
+    CFFT_CONV_EXACT_LINES(CFFT_CONV)
+}
+#undef CFFT_CONV
+
+__global__ void __launch_bounds__(512)
+k_conv_exact_multi_f64(MultiArgs ma, const MItem* __restrict__ items,
+                      const MPlan* __restrict__ plans) {
+    CFFT_DYN_LDS(smem);
+    const MItem it = items[blockIdx.x];
+    const MPlan* P = plans + it.plan;
+    int sgn;
+    double scale;
+    item_direction(it, P->n, ma, sgn, scale);
+    ItemLines<double> lines{ma.in_base, ma.out_base, &it};
+#define CFFT_CONV(...)                                                                          \
+    case Rad<__VA_ARGS__>::N:                                                                   \
+        static_assert(fixed_conv_block<double, Rad<__VA_ARGS__>>() == 512, "short lines");      \
+        fixed_conv_body<double, Rad<__VA_ARGS__>>(                                              \
+            smem, lines, it.count, P->n, P->C, P->Ls, P->mode, sgn, scale, P->perm, P->iperm,   \
+            (const V_t<double>*)P->chirp, (const V_t<double>*)P->K, (const V_t<double>*)P->line.tw); \
+        break;
+    switch (P->L) {
+        CFFT_CONV_EXACT_LINES(CFFT_CONV)
+        default: break;
+    }
+}
+
+hipError_t conv_exact_multi_f64(const MultiLaunch& L, const MultiArgs& ma, hipStream_t st) {
+    hipLaunchKernelGGL(k_conv_exact_multi_f64, dim3((unsigned)L.nitems), dim3(L.block), L.lds, st, ma,
+                       L.items, L.plans);
+    return hipGetLastError();
+}
+void init_kernels_fixed_conv_exact_f64() { detail::allow_big_lds(k_conv_exact_multi_f64); }
+}  // namespace cfft

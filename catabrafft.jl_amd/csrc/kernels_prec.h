@@ -37,6 +37,8 @@ void fixed_real_f64(std::vector<FixedReal>& rows);
 // The fixed convolutions (fixed_conv.h).
 void fixed_conv_f32(std::vector<FixedConv>& rows);
 void fixed_conv_f64(std::vector<FixedConv>& rows);
+void fixed_conv_exact_f32(std::vector<FixedConv>& rows);
+void fixed_conv_exact_f64(std::vector<FixedConv>& rows);
 // The fixed large convolutions (fixed_convl.h).
 void fixed_convl_f32_f32(std::vector<FixedConvL>& rows);
 void fixed_convl_f32_f64(std::vector<FixedConvL>& rows);
@@ -46,6 +48,8 @@ void init_kernels_fixed_convl_multi_f32_f64();
 void init_kernels_fixed_convl_multi_f64_f64();
 void init_kernels_fixed_conv_multi_f32();
 void init_kernels_fixed_conv_multi_f64();
+void init_kernels_fixed_conv_exact_f32();
+void init_kernels_fixed_conv_exact_f64();
 
 hipError_t real_rows_f32(const void* in, void* out, const RealArgs& a, const PassTable& pt,
                          const void* tw, int E, hipStream_t st);

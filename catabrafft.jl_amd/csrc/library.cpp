@@ -847,13 +847,12 @@ int conv_data(int64_t n, Prec prec, ConvKernels own, ConvData& d) {
     d.chirp.clear();
     if (rader) {
         const int64_t N = n - 1;
-        // no padding where n - 1 is smooth, unless it is short and has no kernel of its own: a padded
-        // length that has one then costs no more (F32 rows: n = 1031 at L = 2304 1.35 TB/s, n = 2003
-        // at L = 2002 on the run-time kernel 1.31; n = 4099 at 9216 0.99, n = 3001 at 3000 1.29),
-        // and spares a work list the launches of the few run-time convolutions
-        const bool exact = is_smooth(N) &&
-                           (N > 2048 || !own.fused || find_fixed_conv(prec, N, true));
-        d.L = exact ? N : conv_length(2 * N - 1, prec, own);
+        // No padding where n - 1 is smooth; up to n = 2049 these lengths have kernels of their own.
+        // On 8 million elements they take 0.71 (F32) and 0.63 (F64) of the time of the padded
+        // lengths' kernels, on 2 MB 1.03 and 0.98 (geometric means over 79 primes; n = 181 F32 103
+        // us padded, 43 here, 82 on the run-time kernel; n = 617 F64 212, 84, 131), and padding adds
+        // errors: n = 313 in F64 1.21, n = 71 1.16 of the unpadded ones.
+        d.L = is_smooth(N) ? N : conv_length(2 * N - 1, prec, own);
         const int64_t g = primitive_root(n);
         const int64_t ginv = powmod(g, n - 2, n);
         d.perm.resize(N);
@@ -1044,7 +1043,7 @@ static int plan_fixed_convl(Ctx* ctx, Plan& p, const ConvData& d, bool alloc_wor
         return rc;
     }
     {
-        const FixedConv lineb{f2->rb, f2->np, f2->N, 0, 0, 0, nullptr, nullptr};
+        const FixedConv lineb{f2->rb, f2->np, f2->N, 0, 0, 0, false, nullptr, nullptr};
         const std::vector<int> f = conv_order(lineb);  // frequency of [k N2 / R + b]
         const int C = p.convl_cb;
         std::vector<int> order(blocks(N1, C) * N2, 0);

@@ -91,6 +91,7 @@ enum class MultiKernel : int {
     ConvLA, ConvLBA, ConvLC,  // the three fused launches of a large convolution
     ConvFixed, ConvFixedWide, // fused convolutions of fixed lengths (MPlan::L): workgroups of
                               // up to 512 threads, and of up to 1024
+    ConvExact,                // those of the unpadded lengths
     ConvFA, ConvFBA, ConvFC   // large convolutions over fixed lines (MPlan::N1, N2)
 };
 
@@ -110,6 +111,8 @@ hipError_t convl_fixed_multi_f32_f64(const MultiLaunch& L, const MultiArgs& a, h
 hipError_t convl_fixed_multi_f64_f64(const MultiLaunch& L, const MultiArgs& a, hipStream_t st);
 hipError_t conv_fixed_multi_f32(const MultiLaunch& L, const MultiArgs& a, hipStream_t st);
 hipError_t conv_fixed_multi_f64(const MultiLaunch& L, const MultiArgs& a, hipStream_t st);
+hipError_t conv_exact_multi_f32(const MultiLaunch& L, const MultiArgs& a, hipStream_t st);
+hipError_t conv_exact_multi_f64(const MultiLaunch& L, const MultiArgs& a, hipStream_t st);
 hipError_t gs_multi_f32_f32(const MultiLaunch& L, const MultiArgs& a, hipStream_t st);
 hipError_t gs_multi_f32_f64(const MultiLaunch& L, const MultiArgs& a, hipStream_t st);
 hipError_t gs_multi_f64_f64(const MultiLaunch& L, const MultiArgs& a, hipStream_t st);

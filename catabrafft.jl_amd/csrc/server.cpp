@@ -365,7 +365,8 @@ static int srv_launch_round(Server* s, std::vector<SrvRequest*>& admitted, int s
     for (const MultiLaunch& L : R->launches) {
         const MultiKernel k = (MultiKernel)L.kernel;
         if (rc == CFFT_OK && k != MultiKernel::Rows && k != MultiKernel::ConvSmall &&
-            k != MultiKernel::ConvFixed && k != MultiKernel::ConvFixedWide)
+            k != MultiKernel::ConvFixed && k != MultiKernel::ConvFixedWide &&
+            k != MultiKernel::ConvExact)
             rc = fail(CFFT_ERR_UNSUPPORTED, "dependent work-list launches in a serving round");
         tasks.push_back({L.cost, &L, nullptr});
     }

@@ -250,6 +250,7 @@ void WorkList::add_transforms(const PlanEntry& e, const std::vector<XformRef>& x
             const int block = p.C * (p.fconv ? p.fconv->Tt : p.line.Tt);
             const size_t lds = 2 * (esz(pr) / 2) * (size_t)p.C * p.LsC + esz(pr) * p.C;
             const MultiKernel mk = !p.fconv                       ? MultiKernel::ConvSmall
+                                   : p.fconv->unpadded           ? MultiKernel::ConvExact
                                    : p.fconv->max_threads <= 512 ? MultiKernel::ConvFixed
                                                                  : MultiKernel::ConvFixedWide;
             add_lines(1, mk, p, e.mplan, pr, p.C, block, lds, xs,

@@ -352,6 +352,61 @@ def test_emulated_forced_convolutions_pad_as_little_as_they_can(emu, tmp_path, n
     emu.cfft_finalize(ctx)
 
 
+SHORT_PRIMES = [n for n in range(17, 2050) if _prime(n) and _factor_smooth(n - 1)]
+
+
+@pytest.mark.parametrize("dt", [np.complex64, np.complex128])
+def test_emulated_short_primes_convolve_without_padding(emu, dt):
+    """A prime n up to 2049 whose n - 1 is a product of radices: a convolution of n - 1 points on a
+    kernel of its own, alone and in a work list of all of them."""
+    ctx, code = ctypes.c_void_p(), (0 if dt == np.complex64 else 1)
+    assert emu.cfft_init(0, ctypes.byref(ctx)) == 0
+    lens = np.array(SHORT_PRIMES, dtype=np.int64)
+    offs = np.concatenate([[0], np.cumsum(lens)[:-1]]).astype(np.int64)
+    P, u = ctypes.POINTER(ctypes.c_int64), ctypes.c_void_p()
+    x = seeded_complex(int(lens.sum()), seed=7, dtype=dt)
+    y = np.zeros_like(x)
+    assert emu.cfft_plan_many_uneven(ctx, len(lens), lens.ctypes.data_as(P),
+                                     offs.ctypes.data_as(P), code, 0, ctypes.byref(u)) == 0
+    assert emu.cfft_exec(u, x.ctypes.data, y.ctypes.data, -1, 0, None) == 0
+    for n, o in zip(lens.tolist(), offs.tolist()):
+        p = ctypes.c_void_p()
+        assert emu.cfft_plan_1d(ctx, n, 3, n, n, code, 0, ctypes.byref(p)) == 0
+        d = _desc(emu, p)
+        assert f"rader-fused L={n - 1} " in d and "fixed" in d, d
+        rows = np.stack([x[o:o + n]] * 3)
+        assert emu.cfft_exec(p, rows.ctypes.data, rows.ctypes.data, -1, 0, None) == 0
+        assert all(np.array_equal(r, y[o:o + n]) for r in rows), n
+        ref = np.fft.fft(x[o:o + n].astype(np.clongdouble))
+        err = float(np.linalg.norm(rows[0] - ref) / np.linalg.norm(ref))
+        assert err < _bound(n, dt), (n, err)
+        emu.cfft_plan_destroy(p)
+    emu.cfft_plan_destroy(u)
+    emu.cfft_finalize(ctx)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [np.complex64, np.complex128])
+def test_short_primes_convolve_without_padding(gpu_ready, dt):
+    import torch
+
+    import catabrafft as C
+
+    lens = np.array(SHORT_PRIMES, dtype=np.int64)
+    offs = np.concatenate([[0], np.cumsum(lens)[:-1]]).astype(np.int64)
+    x = torch.from_numpy(seeded_complex(int(lens.sum()), seed=7, dtype=dt)).cuda()
+    y = C.UnevenPlan(lens, offs, dt).exec_torch(x, torch.zeros_like(x))
+    for n, o in zip(lens.tolist(), offs.tolist()):
+        p = C.Plan(n, 67, dt)
+        print(f"{np.dtype(dt)} {p.describe()}", flush=True)
+        rows = torch.stack([x[o:o + n]] * 67)
+        p.exec_torch(rows, rows)
+        assert all(torch.equal(torch.view_as_real(r), torch.view_as_real(y[o:o + n])) for r in rows)
+        ref = np.fft.fft(x[o:o + n].cpu().numpy().astype(np.clongdouble))
+        err = float(np.linalg.norm(rows[-1].cpu().numpy() - ref) / np.linalg.norm(ref))
+        assert err < _bound(n, dt), (n, err)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", [np.complex64, np.complex128])
 def test_fixed_convolutions(gpu_ready, dt):
