@@ -113,16 +113,18 @@ struct SrvRound {
     int slot = 0;
 };
 
-// The independent launches of a round are spread over its slot's stream and this many others, which
-// the slots share: a request's kernels have tens to hundreds of workgroups, too few to fill the GPU
-// in turn.  Created by the first round that spreads.  (A burst of 48 requests of 64 to 2^18 points:
-// 850 -> 692 us.)
+// The independent launches of a round are spread over its slot's stream and this many others of the
+// slot: a request's kernels have tens to hundreds of workgroups, too few to fill the GPU in turn.
+// (A burst of 48 requests of 64 to 2^18 points: 850 -> 692 us.)  No other slot's rounds run on them:
+// a round waits for none of another round's kernels in stream order.  Created by the slot's first
+// round that spreads; where they cannot be, the slot's rounds run on its own stream.
 constexpr int kSideStreams = 3;
 
 // A stream with the resources its rounds reuse (one round at a time per slot).
 struct SrvSlot {
     hipStream_t stream = nullptr;
     hipEvent_t done = nullptr;
+    hipStream_t side[kSideStreams] = {};
     hipEvent_t fork = nullptr, join[kSideStreams] = {};
     bool busy = false;
     DevBuf dplans, ditems, dtable;
@@ -131,6 +133,8 @@ struct SrvSlot {
         if (stream) (void)hipStreamDestroy(stream);
         if (done) (void)hipEventDestroy(done);
         if (fork) (void)hipEventDestroy(fork);
+        for (hipStream_t s : side)
+            if (s) (void)hipStreamDestroy(s);
         for (hipEvent_t e : join)
             if (e) (void)hipEventDestroy(e);
     }
@@ -140,7 +144,6 @@ struct Server {
     Ctx* ctx = nullptr;
     size_t cap = 0;
     std::vector<SrvSlot> slots;
-    hipStream_t side[kSideStreams] = {};
     std::thread worker;
     std::mutex mu;
     std::condition_variable cv_work, cv_done;
@@ -230,17 +233,18 @@ static void srv_release(Server* s, SrvRequest* r) {
     r->bytes = 0;
 }
 
-static bool srv_side_streams(Server* s, SrvSlot& sl) {
+// Whether the slot has its side streams and their events (created here at the first call).
+static bool srv_side_streams(SrvSlot& sl) {
     auto event = [](hipEvent_t* e) {
         return *e || hipEventCreateWithFlags(e, hipEventDisableTiming) == hipSuccess;
     };
-    if (!event(&sl.fork)) return false;
-    for (int i = 0; i < kSideStreams; ++i) {
-        if (!s->side[i] && hipStreamCreateWithFlags(&s->side[i], hipStreamNonBlocking) != hipSuccess)
-            return false;
-        if (!event(&sl.join[i])) return false;
-    }
-    return true;
+    bool ok = event(&sl.fork);
+    for (int i = 0; i < kSideStreams && ok; ++i)
+        ok = (sl.side[i] ||
+              hipStreamCreateWithFlags(&sl.side[i], hipStreamNonBlocking) == hipSuccess) &&
+             event(&sl.join[i]);
+    if (!ok) (void)hipGetLastError();
+    return ok;
 }
 
 // Builds and enqueues one round on slot `slot`.  Called with the lock held; the lock is released
@@ -382,9 +386,8 @@ static int srv_launch_round(Server* s, std::vector<SrvRequest*>& admitted, int s
     double load[kSideStreams + 1] = {};
     bool forked[kSideStreams] = {};
     // a round of work lists alone is short: the events would cost it more than they give
-    const bool spread = direct.size() > 1;
-    if (spread && rc == CFFT_OK &&
-        (!srv_side_streams(s, sl) || hipEventRecord(sl.fork, st) != hipSuccess))
+    const bool spread = direct.size() > 1 && rc == CFFT_OK && srv_side_streams(sl);
+    if (spread && hipEventRecord(sl.fork, st) != hipSuccess)
         rc = fail(CFFT_ERR_HIP, "forking the round's streams failed");
     for (const Task& t : tasks) {
         if (rc != CFFT_OK) break;
@@ -392,7 +395,7 @@ static int srv_launch_round(Server* s, std::vector<SrvRequest*>& admitted, int s
         for (int i = 1; i <= kSideStreams && spread; ++i)
             if (load[i] < load[k]) k = i;
         load[k] += t.cost;
-        hipStream_t ts = k ? s->side[k - 1] : st;
+        hipStream_t ts = k ? sl.side[k - 1] : st;
         if (k && !forked[k - 1]) {
             if (hipStreamWaitEvent(ts, sl.fork, 0) != hipSuccess) {
                 rc = fail(CFFT_ERR_HIP, "stream wait failed");
@@ -415,7 +418,7 @@ static int srv_launch_round(Server* s, std::vector<SrvRequest*>& admitted, int s
     }
     for (int i = 0; i < kSideStreams; ++i) {
         if (!forked[i]) continue;
-        if ((hipEventRecord(sl.join[i], s->side[i]) != hipSuccess ||
+        if ((hipEventRecord(sl.join[i], sl.side[i]) != hipSuccess ||
              hipStreamWaitEvent(st, sl.join[i], 0) != hipSuccess) &&
             rc == CFFT_OK)
             rc = fail(CFFT_ERR_HIP, "stream join failed");
@@ -436,7 +439,7 @@ static int srv_launch_round(Server* s, std::vector<SrvRequest*>& admitted, int s
     lk.lock();
     if (rc != CFFT_OK) {
         // nothing of this round may still run when its buffers return to the pool
-        for (hipStream_t ss : s->side)
+        for (hipStream_t ss : sl.side)
             if (ss) (void)hipStreamSynchronize(ss);
         (void)hipStreamSynchronize(st);
         sl.busy = false;
@@ -679,8 +682,6 @@ int cfft_server_destroy(cfft_server srv) {
     if (s->worker.joinable()) s->worker.join();
     (void)hipSetDevice(s->ctx->device);
     for (auto& sl : s->slots) sl.destroy();
-    for (hipStream_t st : s->side)
-        if (st) (void)hipStreamDestroy(st);
     delete s;
     delete srv;
     return CFFT_OK;

@@ -1,4 +1,5 @@
 // CPU emulation runtime for tests/emu/include/hip/hip_runtime.h (TEST INFRASTRUCTURE ONLY).
+#include <atomic>
 #include <hip/hip_runtime.h>
 #include <ucontext.h>
 
@@ -177,7 +178,15 @@ hipError_t hipMemcpy2DAsync(void* d, size_t dp, const void* s, size_t sp, size_t
 }
 hipError_t hipMemset(void* p, int v, size_t n) { std::memset(p, v, n); return hipSuccess; }
 hipError_t hipMemsetAsync(void* p, int v, size_t n, hipStream_t) { return hipMemset(p, v, n); }
-hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = new emu::Stream(); return hipSuccess; }
+// Streams that may still be created (-1: any number); set by the tests.
+static std::atomic<int> streams_left{-1};
+extern "C" void cfft_emu_streams_left(int n) { streams_left = n; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
+    if (streams_left == 0) return hipErrorOutOfMemory;
+    if (streams_left > 0) --streams_left;
+    *s = new emu::Stream();
+    return hipSuccess;
+}
 hipError_t hipStreamDestroy(hipStream_t s) { delete s; return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t* e) { *e = new emu_event(); return hipSuccess; }

@@ -157,6 +157,30 @@ def test_emulated_server_rounds(E):
     assert lib.cfft_server_destroy(srv) == 0
 
 
+@pytest.mark.parametrize("left", [-1, 0, 2])  # further streams that can be created
+def test_emulated_server_without_side_streams(E, left):
+    """Rounds of several plan-launched requests spread over further streams; where these cannot be
+    created the requests run all the same."""
+    lib, ctx = E
+    srv = ctypes.c_void_p()
+    assert lib.cfft_server_create(ctx, 1 << 30, 1, ctypes.byref(srv)) == 0
+    lib.cfft_emu_streams_left(left)
+    try:
+        reqs = []
+        for i, n in enumerate([20000, 1 << 15, 20000, 24000, 8209, 1 << 15, 60]):
+            x = seeded_complex(n, batch=1, seed=60 + i, dtype=np.complex64)
+            y, t = np.zeros_like(x), ctypes.c_int64()
+            assert lib.cfft_server_submit(srv, n, 1, 0, -1, 0, x.ctypes.data, y.ctypes.data, 1,
+                                          ctypes.byref(t)) == 0
+            reqs.append((t.value, x, y))
+        for t, x, y in reqs:
+            assert lib.cfft_server_wait(srv, t) == 0
+            assert rel_l2(y, O.fft(x.astype(np.complex128), "d")) < 1e-6
+    finally:
+        lib.cfft_emu_streams_left(-1)
+    assert lib.cfft_server_destroy(srv) == 0
+
+
 def test_emulated_server_in_place_requests(E):
     """On-device requests with in == out: a four-step length (its plan runs out of place, so the
     server stages its result through a pooled buffer) and a work-list length, in one round with
