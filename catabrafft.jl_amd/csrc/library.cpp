@@ -21,12 +21,14 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <set>
 #include <sstream>
 #include <string>
 #include <tuple>
 #include <vector>
 
 #include "catabrafft.h"
+#include "fixed_table.h"
 #include "hostmath.h"
 #include "kernels.h"
 #include "library.h"
@@ -776,38 +778,26 @@ static int plan_large(Ctx* ctx, Plan& p, const PlanOptions& o) {
 }
 
 
-// A length of the fixed large convolutions, the product of two of their lines, and its cost: points
-// times the passes over them, and six for the work lines' trips through memory.
+// A length of the fixed large convolutions, N1 N2 of their lines; its cost (points times the passes
+// over them, and six for the work lines' trips through memory) and rounding noise.
 struct ConvSplit {
     int64_t L = 0;
     int N1 = 0, N2 = 0;
-    double cost = 0;
+    double cost = 0, noise = 0;
 };
-static int smooth7_passes(int n) { return (int)fourstep_line_radices(n).size(); }
-static const std::vector<ConvSplit>& conv_splits() {  // ascending L, each the cheapest from there on
-    static const std::vector<ConvSplit> v = [] {
-        std::vector<ConvSplit> all, out;
-        const std::vector<int>& n = fixed_convl_lengths();
-        for (int a : n)
-            for (int b : n) {
-                if (a < b || a > 4 * b) continue;
-                ConvSplit c{(int64_t)a * b, a, b, 0};
-                c.cost = (double)c.L * (2 * smooth7_passes(a) + 2 * smooth7_passes(b) + 6);
-                all.push_back(c);
-            }
-        std::sort(all.begin(), all.end(), [](const ConvSplit& x, const ConvSplit& y) {
-            return std::make_tuple(-x.L, x.cost, x.N1) < std::make_tuple(-y.L, y.cost, y.N1);
-        });
-        double best = 1e300;
-        for (const ConvSplit& c : all)
-            if (c.cost < best) {
-                best = c.cost;
-                out.push_back(c);
-            }
-        std::reverse(out.begin(), out.end());
-        return out;
-    }();
+// Squared rounding error of an FFT over passes of these radices.
+static double line_noise(const std::vector<int>& r) {
+    int count[17] = {};
+    for (int R : r) ++count[R];
+    double v = 0;
+    for (int R = 2; R <= 16; ++R)
+        v += count[R] * kPassNoise[R] + count[R] * count[R] * kRepeatedNoise[R];
     return v;
+}
+// Two-line lengths in F32 round by 5 to 10 % more than the sum of their passes says where they have no
+// factor 5 (98 lengths from 16,464 to 2^21, on these kernels and on the run-time ones).
+static double two_line_noise(int64_t L, Prec prec) {
+    return prec == Prec::F32 && L % 5 ? 1.1 : 1.0;
 }
 // The split of length L itself (L = 0 in the result: none): N1 >= N2, the most even one (launch A
 // reads its columns in longer runs), but N2 > N1 where that keeps the F64 lines of launch C at 1024
@@ -820,26 +810,75 @@ static ConvSplit conv_split_of(int64_t L, Prec prec) {
     for (int a : fixed_convl_lengths())
         for (int b : fixed_convl_lengths())
             if ((int64_t)a * b == L && a <= 4 * b && b <= 4 * a &&
-                (!best.L || rank(a, b) < rank(best.N1, best.N2)))
-                best = ConvSplit{L, a, b, 0};
+                (!best.L || rank(a, b) < rank(best.N1, best.N2))) {
+                best = ConvSplit{L, a, b, 0, 0};
+                std::vector<int> r = fourstep_line_radices(a);
+                const std::vector<int> rb = fourstep_line_radices(b);
+                r.insert(r.end(), rb.begin(), rb.end());
+                best.cost = (double)L * (2 * r.size() + 6);
+                best.noise = line_noise(r) * two_line_noise(L, prec);
+            }
     return best;
 }
-// Length of a convolution that needs at least m points: the shortest of the fixed kernels' lengths
-// that the plan may run (fused: the lengths that no longer one with fewer passes beats; large: the
-// cheapest product of two lines), else the shortest 7-smooth one.
-static int64_t conv_length(int64_t m, Prec prec, ConvKernels own) {
+static const std::vector<ConvSplit>& conv_splits(Prec prec) {  // one per length, ascending
+    auto make = [](Prec pr) {
+        std::set<int64_t> lengths;
+        for (int a : fixed_convl_lengths())
+            for (int b : fixed_convl_lengths()) lengths.insert((int64_t)a * b);
+        std::vector<ConvSplit> v;
+        for (int64_t L : lengths) {
+            const ConvSplit c = conv_split_of(L, pr);
+            if (c.L) v.push_back(c);
+        }
+        return v;
+    };
+    static const std::vector<ConvSplit> t[2] = {make(Prec::F32), make(Prec::F64)};
+    return t[prec == Prec::F64];
+}
+// Length of a convolution that needs at least m points: of the fixed kernels' lengths that the plan
+// may run, the cheapest whose rounding noise is no more than that of the shortest 7-smooth length;
+// else that length.  (The shortest or cheapest one by itself had up to 18 % larger errors: F32 n =
+// 317 at L = 648 = 8 9 9 instead of 640 = 16 8 5.)  io: the transform's precision (the results of an
+// F64 convolution round by far more than it does where they are F32).
+static int64_t conv_length(int64_t m, Prec prec, Prec io, ConvKernels own) {
+    const int64_t shortest = next_smooth(m);
+    double noise = line_noise(line_radices(shortest));
     const FixedConv* f = find_fixed_conv(prec, m, false);
-    if (f) return own.fused ? f->N : next_smooth(m);
-    if (!own.large) return next_smooth(m);
-    const std::vector<ConvSplit>& v = conv_splits();
-    const auto it = std::lower_bound(v.begin(), v.end(), m,
-                                     [](const ConvSplit& c, int64_t x) { return c.L < x; });
-    return it != v.end() ? it->L : next_smooth(m);
+    int64_t L = 0;
+    double best = 1e300;
+    if (f && own.fused) {
+        for (; f; f = find_fixed_conv(prec, f->N + 1, false)) {
+            const double cost = f->N * (f->np + 0.3);
+            if (cost < best && line_noise(std::vector<int>(f->r, f->r + f->np)) <= noise) {
+                best = cost;
+                L = f->N;
+            }
+        }
+    } else if (!f && own.large) {
+        const std::vector<ConvSplit>& v = conv_splits(prec);
+        auto it = std::lower_bound(v.begin(), v.end(), m,
+                                   [](const ConvSplit& c, int64_t x) { return c.L < x; });
+        noise *= two_line_noise(shortest, prec);
+        double least = 1e300;
+        int64_t quiet = 0;  // the least noisy of the lengths up to 1.5 m, where all are noisier
+        for (; it != v.end(); ++it) {
+            if (it->cost < best && (prec != io || it->noise <= noise)) {
+                best = it->cost;
+                L = it->L;
+            }
+            if (2 * it->L <= 3 * m && it->noise < least) {
+                least = it->noise;
+                quiet = it->L;
+            }
+        }
+        if (!L) L = quiet;
+    }
+    return L ? L : shortest;
 }
 
 // Convolution data of a Rader (prime n) or Bluestein transform: permutations or chirp, and the
 // zero-padded kernel b whose spectrum the convolution multiplies by.
-int conv_data(int64_t n, Prec prec, ConvKernels own, ConvData& d) {
+int conv_data(int64_t n, Prec prec, Prec io, ConvKernels own, ConvData& d) {
     const bool rader = is_prime(n);
     d.mode = rader ? ConvMode::Rader : ConvMode::Bluestein;
     d.perm.clear();
@@ -852,7 +891,7 @@ int conv_data(int64_t n, Prec prec, ConvKernels own, ConvData& d) {
         // lengths' kernels, on 2 MB 1.03 and 0.98 (geometric means over 79 primes; n = 181 F32 103
         // us padded, 43 here, 82 on the run-time kernel; n = 617 F64 212, 84, 131), and padding adds
         // errors: n = 313 in F64 1.21, n = 71 1.16 of the unpadded ones.
-        d.L = is_smooth(N) ? N : conv_length(2 * N - 1, prec, own);
+        d.L = is_smooth(N) ? N : conv_length(2 * N - 1, prec, io, own);
         const int64_t g = primitive_root(n);
         const int64_t ginv = powmod(g, n - 2, n);
         d.perm.resize(N);
@@ -872,7 +911,7 @@ int conv_data(int64_t n, Prec prec, ConvKernels own, ConvData& d) {
         for (int64_t m = d.L - N + 1; m < d.L; ++m) d.b[m] = w[m - (d.L - N)];
         d.g = g;
     } else {
-        d.L = conv_length(2 * n - 1, prec, own);
+        d.L = conv_length(2 * n - 1, prec, io, own);
         d.chirp.resize(n);
         const OmegaTable om(2 * n);
         for (int64_t m = 0; m < n; ++m) {
@@ -1084,7 +1123,7 @@ static int plan_conv(Ctx* ctx, Plan& p, const PlanOptions& o) {
     const bool asked = o.E && o.explicit_opts;
     const ConvKernels own{!asked && o.wave <= 0 && !kWaveDefault && p.cprec == p.prec,
                           !asked && o.fuse_conv != 0 && !o.large};
-    conv_data(n, p.cprec, own, d);
+    conv_data(n, p.cprec, p.prec, own, d);
     p.mode = d.mode;
     p.L = d.L;
     p.g = d.g;

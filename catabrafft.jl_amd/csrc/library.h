@@ -261,8 +261,8 @@ struct ConvData {
 struct ConvKernels {
     bool fused, large;
 };
-// prec: the precision of the convolution.
-int conv_data(int64_t n, Prec prec, ConvKernels own, ConvData& d);
+// prec: the precision of the convolution; io: of the data.
+int conv_data(int64_t n, Prec prec, Prec io, ConvKernels own, ConvData& d);
 // K[i] = FFT_L(b)[order[i]] (nullptr: natural order).
 int conv_spectrum(Ctx* ctx, const std::vector<std::complex<long double>>& b, Prec cprec, DevBuf& K,
                   const std::vector<int>* order = nullptr);

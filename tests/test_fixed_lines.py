@@ -352,6 +352,33 @@ def test_emulated_forced_convolutions_pad_as_little_as_they_can(emu, tmp_path, n
     emu.cfft_finalize(ctx)
 
 
+@pytest.mark.parametrize("n,dt", [(34, np.complex128), (137, np.complex128), (310, np.complex128),
+                                  (317, np.complex64), (383, np.complex64), (1111, np.complex64),
+                                  (1523, np.complex64)])
+def test_emulated_padded_convolutions_are_as_accurate_as_the_shortest(emu, tmp_path, n, dt):
+    """The padded length of a default plan is chosen for its rounding errors too: they are no larger
+    than at the shortest smooth length, which a forced shape runs at.  Bound: the lengths' errors
+    are within 4 % (one standard deviation) of the model that chooses, so two of them within
+    1 + 2 sqrt(2) 0.04."""
+    code, batch = (0 if dt == np.complex64 else 1), max(8, 32768 // n)
+    x = seeded_complex(n, batch=batch, seed=n, dtype=dt)
+    ref = np.fft.fft(x.astype(np.clongdouble))
+    w = tmp_path / "w.txt"
+    w.write_text(f"{n} {batch} {n} {n} {code} 1 : 16 64 0 0 0 -1 0 0\n")
+    ctx, err = ctypes.c_void_p(), []
+    assert emu.cfft_init(0, ctypes.byref(ctx)) == 0
+    assert emu.cfft_wisdom_import(ctx, str(w).encode()) == 0
+    for flags in (0, 1):
+        p, y = ctypes.c_void_p(), np.zeros_like(x)
+        assert emu.cfft_plan_1d(ctx, n, batch, n, n, code, flags, ctypes.byref(p)) == 0
+        assert ("fixed" in _desc(emu, p)) == (flags == 0), _desc(emu, p)
+        assert emu.cfft_exec(p, x.ctypes.data, y.ctypes.data, -1, 0, None) == 0
+        err.append(float(np.linalg.norm(y - ref) / np.linalg.norm(ref)))
+        emu.cfft_plan_destroy(p)
+    assert err[0] < (1 + 2 * np.sqrt(2) * 0.04) * err[1], (n, err)
+    emu.cfft_finalize(ctx)
+
+
 SHORT_PRIMES = [n for n in range(17, 2050) if _prime(n) and _factor_smooth(n - 1)]
 
 
