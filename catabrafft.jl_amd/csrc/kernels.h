@@ -234,6 +234,13 @@ struct FixedReal {
 };
 const FixedReal* find_fixed_real(Prec p, const PassTable& pt, int N);
 
+// Tables of a convolution in the order its kernels read (kernels_plan.hip): the FP64 spectrum F
+// reordered and rounded, `count` values; a permutation of `live` entries blocked by tiles of C lines.
+hipError_t launch_order_spectrum(Prec pc, const void* F, void* out, const int* freq, int N1, int N2,
+                                 int C, int64_t count, hipStream_t st);
+hipError_t launch_block_perm(const int* perm, int* out, int N1, int N2, int C, int64_t live,
+                             int64_t count, hipStream_t st);
+
 // Sets per-kernel attributes (large LDS) once; called when a context is created.
 void init_kernels();
 

@@ -968,14 +968,14 @@ std::vector<int> conv_order(const FixedConv& f) {
 }
 
 int conv_spectrum(Ctx* ctx, const std::vector<cld>& b, Prec cprec, DevBuf& K,
-                  const std::vector<int>* order) {
+                  const SpectrumOrder* order) {
     const int64_t L = (int64_t)b.size();
     if (L <= 4096) {
         std::vector<cld> h = b;
         if (!host_fft_ld(h)) return fail(CFFT_ERR_UNSUPPORTED, "kernel spectrum length not smooth");
         if (order) {
-            std::vector<cld> o(order->size());
-            for (size_t i = 0; i < o.size(); ++i) o[i] = h[(*order)[i]];
+            std::vector<cld> o((size_t)order->count());
+            for (size_t i = 0; i < o.size(); ++i) o[i] = h[(size_t)order->at((int64_t)i)];
             h.swap(o);
         }
         return upload(K, h, cprec);
@@ -984,35 +984,39 @@ int conv_spectrum(Ctx* ctx, const std::vector<cld>& b, Prec cprec, DevBuf& K,
     std::shared_ptr<Plan> t;
     int rc = cached_plan_1d(ctx, L, 1, CFFT_C64, &t);
     if (rc) return rc;
+    const bool direct = cprec == Prec::F64 && !order;  // the transform's output is the spectrum
+    const SpectrumOrder natural{{0}, (int)L, 1};
+    const SpectrumOrder& o = order ? *order : natural;
+    const size_t kbytes = (size_t)o.count() * esize(cprec), lbytes = (size_t)L * 16;
+    const size_t fbytes = direct ? 0 : o.freq.size() * sizeof(int);
+    // FFT from `in` to K, and in F64 from there, ordered, back to `in`, which is then K (allocations
+    // and their release are a good part of planning a batch of many lengths); F32 has half the bytes
+    // and takes a buffer between.  The order's frequencies come after the rest of `in`.
+    const bool swapped = !direct && cprec == Prec::F64;
+    const size_t ibytes = swapped ? std::max(kbytes, lbytes) : lbytes;
     DevBuf in, out;
-    if ((rc = upload(in, b, Prec::F64))) return rc;
-    if ((rc = out.alloc((size_t)L * 16))) return rc;
-    if ((rc = plan_exec(*t, in.p, out.p, CFFT_FORWARD, 0, ctx->stream))) return rc;
+    if (K.bytes < std::max(kbytes, swapped ? lbytes : 0) &&
+        (rc = K.alloc(std::max(kbytes, swapped ? lbytes : 0))))
+        return rc;
+    if ((rc = in.alloc(ibytes + fbytes))) return rc;
+    if (!direct && !swapped && (rc = out.alloc(lbytes))) return rc;
+    int* const freq = (int*)((char*)in.p + ibytes);
+    {
+        std::vector<std::complex<double>> h(b.size());
+        for (size_t i = 0; i < h.size(); ++i) h[i] = {(double)b[i].real(), (double)b[i].imag()};
+        CFFT_HIP(hipMemcpy(in.p, h.data(), lbytes, hipMemcpyHostToDevice));
+    }
+    if (!direct) CFFT_HIP(hipMemcpy(freq, o.freq.data(), fbytes, hipMemcpyHostToDevice));
+    void* const spec = direct || swapped ? K.p : out.p;
+    if ((rc = plan_exec(*t, in.p, spec, CFFT_FORWARD, 0, ctx->stream))) return rc;
+    if (!direct)
+        CFFT_HIP(launch_order_spectrum(cprec, spec, swapped ? in.p : K.p, freq, o.N1,
+                                       (int)o.freq.size(), o.C, o.count(), ctx->stream));
     CFFT_HIP(hipStreamSynchronize(ctx->stream));
-    if (cprec == Prec::F64 && !order) {
-        std::swap(K.p, out.p);
-        std::swap(K.bytes, out.bytes);
-        return CFFT_OK;
+    if (swapped) {
+        std::swap(K.p, in.p);
+        std::swap(K.bytes, in.bytes);
     }
-    std::vector<std::complex<double>> h((size_t)L);
-    CFFT_HIP(hipMemcpy(h.data(), out.p, (size_t)L * 16, hipMemcpyDeviceToHost));
-    if (order) {
-        std::vector<std::complex<double>> o(order->size());
-        for (size_t i = 0; i < o.size(); ++i) o[i] = h[(*order)[i]];
-        h.swap(o);
-    }
-    if (cprec == Prec::F64) {
-        if ((rc = K.alloc(h.size() * 16))) return rc;
-        CFFT_HIP(hipMemcpy(K.p, h.data(), h.size() * 16, hipMemcpyHostToDevice));
-        return CFFT_OK;
-    }
-    std::vector<float> f(2 * h.size());
-    for (size_t i = 0; i < h.size(); ++i) {
-        f[2 * i] = (float)h[i].real();
-        f[2 * i + 1] = (float)h[i].imag();
-    }
-    if ((rc = K.alloc(h.size() * 8))) return rc;
-    CFFT_HIP(hipMemcpy(K.p, f.data(), h.size() * 8, hipMemcpyHostToDevice));
     return CFFT_OK;
 }
 
@@ -1063,35 +1067,28 @@ static int plan_fixed_convl(Ctx* ctx, Plan& p, const ConvData& d, bool alloc_wor
     p.convl_cc = convl_tile_lines(ctx, Cs, f1->max_b, table, &p.convl_lsc);
     if (!p.convl_ca || !p.convl_cb || !p.convl_cc) return CFFT_ERR_UNSUPPORTED;
     const int N1 = sp.N1, N2 = sp.N2;
-    auto blocks = [](int lines, int C) { return (size_t)((lines + C - 1) / C) * C; };
+    const FixedConv lineb{f2->rb, f2->np, f2->N, 0, 0, 0, false, nullptr, nullptr};
+    const SpectrumOrder order{conv_order(lineb), N1, p.convl_cb};
     if (p.mode == ConvMode::Rader) {
-        auto blocked = [&](const std::vector<int>& src, int C, DevBuf& buf) {
-            std::vector<int> v(blocks(N2, C) * N1, 0);
-            int* o = v.data();
-            for (int j0 = 0; j0 < N2; j0 += C)
-                for (int64_t e = 0; e < N1; ++e, o += C) {
-                    const int64_t i = e * N2 + j0;
-                    const int64_t m = std::min<int64_t>(std::min(C, N2 - j0), p.n - 1 - i);
-                    for (int64_t c = 0; c < m; ++c) o[c] = src[(size_t)(i + c)];
-                }
-            return upload_int(buf, v);
+        // the permutations go through the spectrum's memory, which is written after them
+        const size_t bytes = d.perm.size() * sizeof(int);
+        if ((rc = p.K.alloc((size_t)order.count() * el))) return rc;
+        int* const staged = (int*)p.K.p;
+        CFFT_HIP(hipMemcpy(staged, d.perm.data(), bytes, hipMemcpyHostToDevice));
+        CFFT_HIP(hipMemcpy(staged + d.perm.size(), d.iperm.data(), bytes, hipMemcpyHostToDevice));
+        auto blocked = [&](const int* src, int C, DevBuf& buf) {
+            const int64_t count = (int64_t)((N2 + C - 1) / C) * C * N1;
+            const int r = buf.alloc((size_t)count * sizeof(int));
+            if (r) return r;
+            CFFT_HIP(launch_block_perm(src, (int*)buf.p, N1, N2, C, p.n - 1, count, ctx->stream));
+            return (int)CFFT_OK;
         };
-        if ((rc = blocked(d.perm, p.convl_ca, p.perm))) return rc;
-        if ((rc = blocked(d.iperm, p.convl_cc, p.iperm))) return rc;
+        if ((rc = blocked(staged, p.convl_ca, p.perm))) return rc;
+        if ((rc = blocked(staged + d.perm.size(), p.convl_cc, p.iperm))) return rc;
     } else if ((rc = upload(p.chirp, d.chirp, p.cprec))) {
         return rc;
     }
-    {
-        const FixedConv lineb{f2->rb, f2->np, f2->N, 0, 0, 0, false, nullptr, nullptr};
-        const std::vector<int> f = conv_order(lineb);  // frequency of [k N2 / R + b]
-        const int C = p.convl_cb;
-        std::vector<int> order(blocks(N1, C) * N2, 0);
-        int* o = order.data();
-        for (int k0 = 0; k0 < N1; k0 += C)
-            for (int x = 0; x < N2; ++x, o += C)
-                for (int c = 0; c < std::min(C, N1 - k0); ++c) o[c] = k0 + c + N1 * f[(size_t)x];
-        if ((rc = conv_spectrum(ctx, d.b, p.cprec, p.K, &order))) return rc;
-    }
+    if ((rc = conv_spectrum(ctx, d.b, p.cprec, p.K, &order))) return rc;
     f1->prepare();
     f2->prepare();
     p.kind = Kind::ConvLarge;
@@ -1187,7 +1184,7 @@ static int plan_conv(Ctx* ctx, Plan& p, const PlanOptions& o) {
     } else {
         if ((rc = upload(p.chirp, chirp, p.cprec))) return rc;
     }
-    const std::vector<int> order = p.fconv ? conv_order(*p.fconv) : std::vector<int>();
+    const SpectrumOrder order{p.fconv ? conv_order(*p.fconv) : std::vector<int>(), 1, 1};
     if ((rc = conv_spectrum(ctx, d.b, p.cprec, p.K, p.fconv ? &order : nullptr))) return rc;
     if (small) {
         p.kind = Kind::ConvSmall;

@@ -263,9 +263,20 @@ struct ConvKernels {
 };
 // prec: the precision of the convolution; io: of the data.
 int conv_data(int64_t n, Prec prec, Prec io, ConvKernels own, ConvData& d);
-// K[i] = FFT_L(b)[order[i]] (nullptr: natural order).
+// Where the frequencies of a spectrum go: N1 lines of freq.size() positions side by side in tiles of
+// C, position x of line k (in its tile: x C + k mod C) holding frequency k + N1 freq[x].
+struct SpectrumOrder {
+    std::vector<int> freq;
+    int N1 = 1, C = 1;
+    int64_t count() const { return (int64_t)((N1 + C - 1) / C) * C * (int64_t)freq.size(); }
+    int64_t at(int64_t i) const {  // the frequency of value i (past the last line: 0)
+        const int64_t r = i / C, N2 = (int64_t)freq.size(), k = r / N2 * C + i % C;
+        return k < N1 ? k + (int64_t)N1 * freq[(size_t)(r % N2)] : 0;
+    }
+};
+// K[i] = FFT_L(b)[order->at(i)] (nullptr: natural order).
 int conv_spectrum(Ctx* ctx, const std::vector<std::complex<long double>>& b, Prec cprec, DevBuf& K,
-                  const std::vector<int>* order = nullptr);
+                  const SpectrumOrder* order = nullptr);
 // The frequency at each position of a fixed convolution's spectrum.
 std::vector<int> conv_order(const FixedConv& f);
 Prec conv_precision(int64_t n, Prec io, ConvMode mode);

@@ -504,6 +504,25 @@ def test_emulated_fixed_large_convolutions(emu, dt, lo, hi, count):
     emu.cfft_finalize(ctx)
 
 
+@pytest.mark.parametrize("n,dt", [(8219, np.complex64), (3 * 2803, np.complex64),
+                                  (5003, np.complex128), (3 * 1801, np.complex128)])
+def test_emulated_large_convolution_tables(emu, n, dt):
+    """Spectra longer than the host transforms (4096 points), in both precisions and both orders (fused
+    and two-line), and blocked permutations whose last tile is partly filled: rows of a batch, forward
+    and backward."""
+    ctx, p, code = ctypes.c_void_p(), ctypes.c_void_p(), (0 if dt == np.complex64 else 1)
+    assert emu.cfft_init(0, ctypes.byref(ctx)) == 0
+    assert emu.cfft_plan_1d(ctx, n, 2, n, n, code, 0, ctypes.byref(p)) == 0
+    assert "fixed" in _desc(emu, p), _desc(emu, p)
+    x = seeded_complex(n, batch=2, seed=n, dtype=dt)
+    for direction, ref in ((-1, np.fft.fft), (1, np.fft.ifft)):
+        y, want = np.zeros_like(x), ref(x.astype(np.clongdouble))
+        assert emu.cfft_exec(p, x.ctypes.data, y.ctypes.data, direction, int(direction > 0), None) == 0
+        assert float(np.linalg.norm(y - want) / np.linalg.norm(want)) < _bound(n, dt), _desc(emu, p)
+    emu.cfft_plan_destroy(p)
+    emu.cfft_finalize(ctx)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt,lo,hi,count", [(np.complex64, 8200, 1500000, 40),
                                             (np.complex128, 5200, 1500000, 40)])
