@@ -1130,7 +1130,7 @@ static int plan_conv(Ctx* ctx, Plan& p, const PlanOptions& o) {
     const bool rader = p.mode == ConvMode::Rader;
     int rc;
     // fused small shape?
-    const int E = o.E ? o.E : 16;
+    const int E = o.E ? o.E : o.rows_E ? o.rows_E : 16;
     bool small = false;
     // (4099 x 4093 lines in ComplexF32 283 us against 516 on the run-time kernel)
     if (own.fused) {
@@ -1348,17 +1348,18 @@ static int plan_fft_core(Ctx* ctx, Plan& p, const PlanOptions& o) {
         const bool rad_direct = !o.rad_a.empty() && rad_prod == p.n;
         const int64_t n1 = o.n1 ? o.n1 : (!o.rad_a.empty() && !rad_direct ? rad_prod : 0);
         if (n1 == 0) {
-            int Ed = o.E ? o.E : (line_fits(ctx, p.n, p.prec, 8) ? 8 : 16);
+            const int asked = o.E ? o.E : o.rows_E;
+            int Ed = asked ? asked : (line_fits(ctx, p.n, p.prec, 8) ? 8 : 16);
             const std::vector<int> dr = rad_direct ? o.rad_a : line_radices(p.n);
             const int rmax = dr.empty() ? 0 : *std::max_element(dr.begin(), dr.end());
-            if (!o.E && p.prec == Prec::F32 && rmax > 9 && p.n >= 512 &&
+            if (!asked && p.prec == Prec::F32 && rmax > 9 && p.n >= 512 &&
                 line_fits(ctx, p.n, p.prec, 16))
                 Ed = 16;
             const int pipe = o.pipe >= 0 ? o.pipe : 0;
             if (line_fits(ctx, p.n, p.prec, Ed) || rad_direct)
                 return plan_direct(ctx, p, Ed, o.target_threads, pipe,
                                    rad_direct ? &o.rad_a : nullptr, o.wave, o.lds_pad != 0,
-                                   !o.E);
+                                   !asked);
         }
         if (o.large) return plan_large(ctx, p, o);
         // Four-step lines default to E = 8 in F64 (twice the threads per tile), 16 in F32.

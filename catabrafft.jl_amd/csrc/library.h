@@ -137,6 +137,8 @@ struct ExecShape {
 // Planner knobs; the autotuner enumerates them, NO_FLAG uses the defaults.
 struct PlanOptions {
     int E = 0;                 // per-thread complex capacity (8 or 16), 0 = default
+    int rows_E = 0;            // that of direct lines and fused convolutions only, on the run-time
+                               // rows kernels (plans that run in work lists)
     int target_threads = 64;   // threads per workgroup the rows kernels aim for (short lines
                                // share a workgroup up to this; small workgroups measured fastest)
     int64_t n1 = 0;            // four-step split (0 = balanced / direct when it fits)
