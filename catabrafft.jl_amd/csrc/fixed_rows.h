@@ -59,6 +59,23 @@ constexpr int fixed_row_capacity() {
                : 12;
 }
 
+// Lengths that these capacities do not suit have threads and lines a workgroup from a list, and ran
+// 2-24 % slower by the rule than on the run-time kernel (240 MB batches; by the rule, now, run-time):
+// F32 50 256, 122, 219 us, 126 168, 118, 153, 280 124, 101, 109, 560 129, 104, 118, 600 142, 110, 121,
+// 7168 155, 117, 125; F64 30 242, 102, 200, 100 132, 89, 122, 3024 136, 98, 126.  Most are lines of whose
+// last butterflies the rule's threads leave a part for another round, which stores short runs.
+template <typename T>
+constexpr RowShape row_shape(int n) {
+    if constexpr (sizeof(T) == 4) {
+        for (const RowShape& s : kRowShapesF32)
+            if (s.n == n) return s;
+    } else {
+        for (const RowShape& s : kRowShapesF64)
+            if (s.n == n) return s;
+    }
+    return RowShape{n, 0, 0};
+}
+
 // a.C lines per workgroup, a.Tt = TT threads and a.Ls LDS elements each.  Bound by HBM: 2520 x
 // 4096 moves 4.4 TB/s in F32 and 4.2 in F64 (the run-time kernel 3.6 and 3.2), 1024 x 16384 F64
 // 5.8 (5.2).
@@ -81,10 +98,15 @@ k_rows_fixed(const V_t<T>* __restrict__ in, V_t<T>* __restrict__ out, RowsArgs a
 
 template <typename T, class Q>
 struct FixedRowOf {
-    static constexpr int TT = Q::threads(fixed_row_capacity<T, Q>());
+    static constexpr RowShape shape = row_shape<T>(Q::N);
+    static constexpr int TT =
+        shape.threads ? shape.threads : Q::threads(fixed_row_capacity<T, Q>());
     static constexpr int Ls = fixed_line_elems<Q>() | 1;  // odd: lines start in different banks
     // what k_rows_fixed is compiled for: one line where TT > 128, else up to 256 threads
     static constexpr int max_lines = TT > 128 ? 1 : 256 / TT;
+    // by default: workgroups of 64 threads
+    static constexpr int lines = shape.lines ? shape.lines : TT < 64 ? 64 / TT : 1;
+    static_assert(lines <= max_lines, "a listed shape exceeds the kernel's launch bounds");
     static_assert(TT <= 1024, "a line runs on one workgroup");
     static hipError_t launch(const void* in, void* out, const RowsArgs& a, const void* tw,
                              hipStream_t st) {
@@ -96,7 +118,7 @@ struct FixedRowOf {
         return hipGetLastError();
     }
     static void prepare() { detail::allow_big_lds(k_rows_fixed<T, Q, TT>); }
-    static FixedRow row() { return FixedRow{Q::r, Q::np, Q::N, TT, Ls, max_lines, launch, prepare}; }
+    static FixedRow row() { return FixedRow{Q::r, Q::np, Q::N, TT, Ls, lines, max_lines, launch, prepare}; }
 };
 
 }  // namespace cfft

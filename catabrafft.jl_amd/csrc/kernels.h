@@ -155,11 +155,11 @@ struct RealAuxArgs {
 
 // Rows kernel of one line whose radices are compile-time constants (fixed_line.h): np radices r
 // of a length N, Tt threads and Ls LDS elements per line; launch runs a.C <= max_lines lines per
-// workgroup (a.Ls = Ls; no convolution epilogue).  prepare lets the kernel use its LDS, once per
+// workgroup, `lines` by default (a.Ls = Ls; no convolution epilogue).  prepare lets the kernel use its LDS, once per
 // plan.
 struct FixedRow {
     const int* r;
-    int np, N, Tt, Ls, max_lines;
+    int np, N, Tt, Ls, lines, max_lines;
     hipError_t (*launch)(const void* in, void* out, const RowsArgs& a, const void* tw,
                          hipStream_t st);
     void (*prepare)();

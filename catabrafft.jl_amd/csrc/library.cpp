@@ -426,7 +426,8 @@ static int plan_direct(Ctx* ctx, Plan& p, int E, int target_threads, int pipe = 
         const FixedRow* f = at_rate ? nullptr : find_fixed_row(p.prec, p.line.pt, (int)p.n);
         const size_t fper = f ? (size_t)esize(p.prec) * f->Ls : 0;
         if (f && fper <= ctx->lds_max) {
-            int c = std::min(std::max(1, target_threads / f->Tt), f->max_lines);
+            const bool asked = target_threads != PlanOptions{}.target_threads;
+            int c = asked ? std::min(std::max(1, target_threads / f->Tt), f->max_lines) : f->lines;
             c = (int)std::min<int64_t>(c, std::max<int64_t>(1, p.batch));
             f->prepare();
             p.fixed = f;

@@ -52,6 +52,26 @@ def fourstep_radices(n):
     return [1 << (base + (i >= passes - extra)) for i in range(passes)]
 
 
+# Direct lines whose threads fixed_rows.h's rule does not suit: length: (threads, lines a workgroup),
+# the fastest of 2 to 12 thread counts (capacities 6 to 21, and those that the butterflies of the last
+# pass fill) and of workgroups of about 64, 128 and 256 threads, on MI355X over batches of 240 MB in
+# each of input and output.  They are the lengths that ran more than 2 % slower by the rule than on
+# the run-time rows kernel.
+ROW_SHAPES_F32 = {
+    30: (15, 4), 50: (25, 10), 70: (35, 7), 90: (15, 17), 98: (49, 2), 120: (24, 10),
+    126: (21, 12), 135: (45, 2), 150: (30, 8), 162: (27, 9), 225: (45, 5), 245: (49, 5),
+    280: (40, 3), 315: (63, 1), 324: (41, 6), 336: (24, 5), 378: (63, 1), 560: (40, 3),
+    600: (40, 6), 625: (125, 2), 648: (81, 3), 729: (81, 3), 784: (56, 1), 1792: (128, 2),
+    2048: (128, 2), 3200: (320, 1), 3584: (448, 1), 3840: (240, 1), 5488: (392, 1),
+    6272: (448, 1), 6400: (400, 1), 6720: (480, 1), 7168: (448, 1), 7680: (512, 1),
+}
+ROW_SHAPES_F64 = {
+    25: (5, 51), 30: (15, 17), 32: (8, 32), 50: (25, 10), 70: (35, 7), 75: (25, 10), 98: (49, 2),
+    100: (25, 10), 105: (35, 7), 140: (35, 3), 147: (49, 5), 196: (49, 5), 2048: (256, 1),
+    3024: (252, 1),
+}
+
+
 # Squared rounding error that a pass adds to a convolution, by its radix, in units of the square of
 # half an epsilon; REPEATED more for the square of the number of passes of such a radix (the roundings
 # of its constants add up in step).  Fitted to the errors of the convolutions of 2600
@@ -149,6 +169,11 @@ def main():
     ]
     for k in range(PARTS):
         parts.append(macro(f"CFFT_ROW_LINES_{k}", rows[k::PARTS]))
+    parts.append("// Direct lines with threads and lines a workgroup of their own (gen_lines.py: ROW_SHAPES_*).")
+    parts.append("struct RowShape {\n    int n, threads, lines;\n};")
+    for name, of in (("kRowShapesF32", ROW_SHAPES_F32), ("kRowShapesF64", ROW_SHAPES_F64)):
+        parts.append(f"constexpr RowShape {name}[] = {{\n    "
+                     + "\n    ".join(f"{{{n}, {t}, {c}}}," for n, (t, c) in of.items()) + "\n};")
     fs = [fourstep_radices(n) for n in list(range(16, 2049)) + [4096] if line_radices(n)]
     fs += [[2, 8, 8], [4, 8, 8]]  # the strided axes of N-D transforms: no radix 16
     parts.append(macro("CFFT_FS_LINES_FEW", [r for i, r in enumerate(fs) if i % 16 == 3]
