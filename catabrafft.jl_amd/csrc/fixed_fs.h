@@ -267,6 +267,13 @@ struct FixedFsOf {
         detail::allow_big_lds(k_fs_a_fixed<T, G, Q, TT>);
         detail::allow_big_lds(k_fs_b_fixed<T, G, Q, TT>);
     }
+    // pass B alone: the strided axes' sequences
+    static FixedFs strided_entry() {
+        FixedFs f = FixedFs{Q::r, Q::np, Q::N, TT, fixed_fs_threads<T, Q, TT>(), W, (int)sizeof(V_t<T>),
+                            fixed_pad<Q>(), nullptr, launch_b, nullptr};
+        f.prepare = [] { detail::allow_big_lds(k_fs_b_fixed<T, G, Q, TT>); };
+        return f;
+    }
     static FixedFs entry() {
         return FixedFs{Q::r, Q::np, Q::N, TT, fixed_fs_threads<T, Q, TT>(), W, (int)sizeof(V_t<T>), fixed_pad<Q>(),
                        launch_a, launch_b, prepare};

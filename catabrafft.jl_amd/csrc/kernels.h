@@ -170,7 +170,8 @@ const FixedRow* find_fixed_row(Prec p, const PassTable& pt, int N);
 // Four-step passes of one line as compile-time constants (fixed_fs.h): Tt threads and elements
 // of `elem` LDS bytes per line (per pair of adjacent lines where width = 2; then in, out and the
 // distances must keep every pair aligned).  a.Ls: LDS elements per line (pair), at least
-// fixed_at(N - 1) + 1 with one pad element per 2^pad (pad < 0: none).
+// fixed_at(N - 1) + 1 with one pad element per 2^pad (pad < 0: none).  launch_a is null for the
+// sequences of strided axes, which are pass B alone.
 struct FixedFs {
     const int* r;
     int np, N, Tt, max_threads, width, elem, pad;

@@ -5,11 +5,15 @@
 namespace cfft {
 #ifdef CFFT_EMU_LANES
 #define CFFT_LINES CFFT_FS_LINES_FEW
+#define CFFT_STRIDED CFFT_STRIDED_LINES_FEW
 #else
 #define CFFT_LINES CFFT_FS_LINES
+#define CFFT_STRIDED CFFT_STRIDED_LINES_F64
 #endif
 #define CFFT_FS(...) rows.push_back(FixedFsOf<double, double2, Rad<__VA_ARGS__>>::entry());
+#define CFFT_B(...) rows.push_back(FixedFsOf<double, double2, Rad<__VA_ARGS__>>::strided_entry());
 void fixed_fs_f64(std::vector<FixedFs>& rows) {
     CFFT_LINES(CFFT_FS)
+    CFFT_STRIDED(CFFT_B)
 }
 }  // namespace cfft

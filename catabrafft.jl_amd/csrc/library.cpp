@@ -18,6 +18,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -615,9 +616,9 @@ static int fixed_stride(Ctx* ctx, const FixedShape& f, int cols, size_t reserve)
 // A fixed pass for a line (nullptr: none, or its tile does not fit): `C` lines per workgroup, a
 // power of two, halved until they fit the workgroup and the LDS beside `reserve` bytes.
 static const FixedFs* pick_fixed_fs(Ctx* ctx, FixedFsKind kind, const LinePlan& lp, size_t reserve,
-                                    int* C, int* Ls) {
+                                    int* C, int* Ls, bool pass_a = false) {
     const FixedFs* f = find_fixed_fs(kind, lp.pt, lp.N);
-    if (!f) return nullptr;
+    if (!f || (pass_a && !f->launch_a)) return nullptr;
     const size_t per = (size_t)f->elem * ((f->pad < 0 ? lp.N : lp.N + (lp.N >> f->pad)) + 64);
     int c = *C / f->width;
     auto fits = [&](int k) {
@@ -1301,7 +1302,7 @@ static void fs_fixed_setup(Ctx* ctx, Plan& p) {
     // (4 and 4 lines: 20,000 x 512 145.6 -> 157.7 us, 2^18 x 128 453 -> 475, 2^17 x 64 123 -> 127).
     fs.FCA = f64 ? 8 : 4;
     fs.FCB = 16;
-    fs.fixed_a = pick_fixed_fs(ctx, kind(fs.N2), fs.a, 16, &fs.FCA, &fs.FLsA);
+    fs.fixed_a = pick_fixed_fs(ctx, kind(fs.N2), fs.a, 16, &fs.FCA, &fs.FLsA, true);
     fs.fixed_b = pick_fixed_fs(ctx, kind(fs.N1), fs.b, table + 16, &fs.FCB, &fs.FLsB);
 }
 
@@ -1997,6 +1998,31 @@ static int plan_exec_noalloc(const Plan& p, const void* in, void* out, int direc
 }
 
 // ------------------------------------------------------------------------------- N-D
+// Radices of a strided axis.  A tile of strided lines waits for memory in every pass of registers it
+// holds, and a radix 16 holds twice those of an 8: from 80 points to 512 (F32: 1024) lines whose
+// four-step sequence has one split their power of two in the fewest passes of up to 8, largest radix
+// first.  MI355X, one axis of arrays of 128 MB, then of 240 MB (four-step sequence, this one; us): F32
+// 112 41.7, 33.8, 98.9, 94.2; 240 62.8, 36.0, 139, 97; 256 41.7, 34.0, 96.9, 95.0; 400 75.7, 35.0, 175,
+// 113; 720 60.4, 39.8, 140, 118; 768 58.0, 38.7, 116, 118; F64 256 40.6, 34.0, 97.2, 95.2; 400 43.5,
+// 35.5, 113, 115; 448 46.5, 38.5, 104, 98.  From 512 in F64 arrays larger than the cache lose more than
+// the others gain (576 45.0, 36.8, 105, 117), and 1024 and 2048 points lose either way (F32 1024 39.6,
+// 40.3, 108.6, 110.4).
+static std::vector<int> strided_line_radices(int64_t n, Prec pr) {
+    const std::vector<int> r = fourstep_line_radices(n);
+    if (!is_smooth7(n) || n < 80 || n >= (pr == Prec::F64 ? 512 : 1024) ||
+        std::find(r.begin(), r.end(), 16) == r.end())
+        return r;  // (lengths with a factor 11 or 13 have no kernels of their own)
+    std::vector<int> out;
+    int k = 0;
+    for (; n % 2 == 0; n /= 2) ++k;
+    const int passes = (k + 2) / 3, base = k / passes, extra = k % passes;
+    for (int i = 0; i < passes; ++i) out.push_back(1 << (base + (i < extra)));
+    if (n > 1)
+        for (int R : line_radices(n)) out.push_back(R);
+    std::sort(out.begin(), out.end(), std::greater<int>());
+    return out;
+}
+
 // Multi-dimensional transforms over the axes in axes_mask (bit a = axis a, row-major dims, the
 // last axis contiguous): the role of plan_fft's `region` (CatabraFFT.jl:169, accepted there and
 // ignored).  The contiguous axis runs as a batch of 1-D transforms; every other axis runs as
@@ -2079,11 +2105,7 @@ int plan_nd_create(Ctx* ctx, int rank, const int64_t* dims, int64_t axes_mask, i
             s->idist = s->odist = inner * N2;
             s->fs.N1 = (int)inner;
             s->fs.N2 = (int)N2;
-            // lines of 128 and 256 points in three light passes instead of two with a radix 16
-            // (which holds twice the registers): 256^3 F32 144.5 -> 135.5 us
-            std::vector<int> rad = fourstep_line_radices(N2);
-            if (N2 == 128) rad = {2, 8, 8};
-            if (N2 == 256) rad = {4, 8, 8};
+            const std::vector<int> rad = strided_line_radices(N2, p->prec);
             if ((rc = make_line(s->fs.b, N2, p->prec, 16, 1024, &rad))) return rc;
             s->fs.CB = pick_tile(ctx, s->fs.b, p->prec, p->prec == Prec::F32 ? 16 : 8);
             s->fs.b.Ls = fs_line_stride(ctx, p->prec, s->fs.b, s->fs.CB, 16);

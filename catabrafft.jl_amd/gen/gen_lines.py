@@ -6,7 +6,8 @@
 A line is a length and its radix sequence, the one the planner takes by default for that length
 (line_radices in library.cpp).  The rows kernels cover every 7-smooth length from 16 to 8192: the
 lengths a workgroup holds in both precisions.  The four-step passes cover every 7-smooth length
-from 16 to 2048, and 4096: the factors of the lengths up to 2^22 and of 2^24.  The fused convolutions pad to
+from 16 to 2048, and 4096: the factors of the lengths up to 2^22 and of 2^24; strided axes have
+sequences of their own under 1024 points.  The fused convolutions pad to
 the lengths of conv_lines (and those of short primes that need no padding have the lengths of
 conv_exact_lines), the large ones to products of two of convl_lines.  The lists are split in parts
 so that several translation units compile them in parallel; the _FEW list is the part that the CPU
@@ -70,6 +71,19 @@ ROW_SHAPES_F64 = {
     100: (25, 10), 105: (35, 7), 140: (35, 3), 147: (49, 5), 196: (49, 5), 2048: (256, 1),
     3024: (252, 1),
 }
+
+
+def strided_radices(n):
+    """The strided axes of N-D transforms: no radix 16, the powers of two in the fewest passes of up to
+    8, largest first (strided_line_radices in library.cpp); None where the four-step's sequence stays."""
+    r = fourstep_radices(n)
+    if r is None or 16 not in r or not 80 <= n < 1024:
+        return None
+    k = (n & -n).bit_length() - 1
+    passes = (k + 2) // 3
+    base, extra = divmod(k, passes)
+    two = [1 << (base + (i < extra)) for i in range(passes)]
+    return sorted(two + [q for q in line_radices(n >> k) or []], reverse=True)
 
 
 # Squared rounding error that a pass adds to a convolution, by its radix, in units of the square of
@@ -175,10 +189,14 @@ def main():
         parts.append(f"constexpr RowShape {name}[] = {{\n    "
                      + "\n    ".join(f"{{{n}, {t}, {c}}}," for n, (t, c) in of.items()) + "\n};")
     fs = [fourstep_radices(n) for n in list(range(16, 2049)) + [4096] if line_radices(n)]
-    fs += [[2, 8, 8], [4, 8, 8]]  # the strided axes of N-D transforms: no radix 16
     parts.append(macro("CFFT_FS_LINES_FEW", [r for i, r in enumerate(fs) if i % 16 == 3]
-                       + [fourstep_radices(n) for n in (16, 128, 256, 1024)] + fs[-2:]))
+                       + [fourstep_radices(n) for n in (16, 128, 256, 1024)]))
     parts.append(macro("CFFT_FS_LINES", fs))
+    strided = [strided_radices(n) for n in range(16, 1024) if strided_radices(n)]
+    parts.append(macro("CFFT_STRIDED_LINES_FEW", [r for i, r in enumerate(strided) if i % 8 == 1]
+                       + [strided_radices(n) for n in (128, 256)]))
+    parts.append(macro("CFFT_STRIDED_LINES", strided))
+    parts.append(macro("CFFT_STRIDED_LINES_F64", [r for r in strided if math.prod(r) < 512]))
     parts.append("// Squared rounding errors of the passes of a convolution by radix (gen_lines.py: noise).")
     for name, of in (("kPassNoise", NOISE), ("kRepeatedNoise", REPEATED)):
         parts.append(f"constexpr double {name}[17] = {{"

@@ -239,6 +239,53 @@ def test_fixed_four_step_matches_the_run_time_kernels(gpu_ready, tmp_path, dt):
             assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]), (n1, n2)
 
 
+# ------------------------------------------------------------------------------ strided axes
+STRIDED_FEW = _lengths("CFFT_STRIDED_LINES_FEW")
+STRIDED = _lengths("CFFT_STRIDED_LINES")
+
+
+def _nd_reference(x):
+    return np.fft.fft(x.astype(np.clongdouble), axis=0)
+
+
+@pytest.mark.parametrize("dt", [np.complex64, np.complex128])
+@pytest.mark.parametrize("n", STRIDED_FEW + [64, 80, 176, 1000])
+@pytest.mark.parametrize("inner", [18, 5])  # line pairs, and an odd number of lines
+def test_emulated_strided_axes(emu, n, inner, dt):
+    """A strided axis on both sides of the range whose sequences have no radix 16."""
+    ctx, p, code = ctypes.c_void_p(), ctypes.c_void_p(), (0 if dt == np.complex64 else 1)
+    assert emu.cfft_init(0, ctypes.byref(ctx)) == 0
+    dims = (ctypes.c_int64 * 2)(n, inner)
+    assert emu.cfft_plan_nd(ctx, 2, dims, 1, code, 0, ctypes.byref(p)) == 0
+    d = _desc(emu, p)
+    if n in STRIDED_FEW and (code == 0 or n < 512):
+        assert "fixed" in d, d
+    x = seeded_complex(n * inner, seed=n, dtype=dt).reshape(n, inner)
+    y = np.zeros_like(x)
+    assert emu.cfft_exec(p, x.ctypes.data, y.ctypes.data, -1, 0, None) == 0
+    want = _nd_reference(x)
+    assert float(np.linalg.norm(y - want) / np.linalg.norm(want)) < _bound(n, dt), d
+    emu.cfft_plan_destroy(p)
+    emu.cfft_finalize(ctx)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [np.complex64, np.complex128])
+def test_strided_axes(gpu_ready, dt):
+    import torch
+
+    import catabrafft as C
+
+    for n in STRIDED + [64, 1000, 1024]:
+        for inner in (40, 5):
+            print(f"{np.dtype(dt)} strided n={n} x {inner}", flush=True)
+            x = seeded_complex(2 * n * inner, seed=n, dtype=dt).reshape(2, n, inner)
+            y = C.fftn(torch.from_numpy(x).cuda(), (1,)).cpu().numpy()
+            want = np.fft.fft(x.astype(np.clongdouble), axis=1)
+            err = float(np.linalg.norm(y - want) / np.linalg.norm(want))
+            assert err < _bound(n, dt), (n, inner, err)
+
+
 # ------------------------------------------------------------------------------ convolutions
 def _factor_smooth(n, primes=(2, 3, 5, 7, 11, 13)):
     for p in primes:
