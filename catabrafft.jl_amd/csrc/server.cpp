@@ -127,7 +127,7 @@ struct SrvSlot {
     hipStream_t side[kSideStreams] = {};
     hipEvent_t fork = nullptr, join[kSideStreams] = {};
     bool busy = false;
-    DevBuf dplans, ditems, dtable;
+    DevBuf tables;
     HostStage stage;
     void destroy() {
         if (stream) (void)hipStreamDestroy(stream);
@@ -346,7 +346,7 @@ static int srv_launch_round(Server* s, std::vector<SrvRequest*>& admitted, int s
     lk.unlock();
     rc = CFFT_OK;
     for (auto& kv : groups) R->wl.add_transforms(entries[kv.first], kv.second);
-    rc = R->wl.finalize(sl.dplans, sl.ditems, sl.dtable, R->launches, st, true, &sl.stage);
+    rc = R->wl.finalize(sl.tables, R->launches, st, &sl.stage);
     // Everything left is independent (the work lists hold rows and fused convolutions only, one
     // launch each; a request launched by its plan has its own buffers): the costliest first, each
     // on the stream with the least work so far.

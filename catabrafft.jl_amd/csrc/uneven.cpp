@@ -435,8 +435,7 @@ void WorkList::add_transforms(const PlanEntry& e, const std::vector<XformRef>& x
     }
 }
 
-int WorkList::finalize(DevBuf& dplans, DevBuf& ditems, DevBuf& dtable,
-                       std::vector<MultiLaunch>& out, hipStream_t st, bool async,
+int WorkList::finalize(DevBuf& tables, std::vector<MultiLaunch>& out, hipStream_t st,
                        HostStage* stage) {
     int rc;
     out.clear();
@@ -513,16 +512,12 @@ int WorkList::finalize(DevBuf& dplans, DevBuf& ditems, DevBuf& dtable,
     const size_t bp = mplans_.size() * sizeof(MPlan);
     const size_t bt = std::max<size_t>(1, table_.size()) * sizeof(uint64_t);
     const size_t bi = std::max<size_t>(1, nitems) * sizeof(MItem);
-    // grow with headroom, so that buffers reused round after round are rarely reallocated
-    // (a staged upload puts the three tables into dplans, one copy)
-    const bool staged = async && stage;
+    // plans, line table and items one after the other; grows with headroom, so that a buffer reused
+    // round after round is rarely reallocated
     const size_t ot = (bp + 255) & ~(size_t)255, oi = (ot + bt + 255) & ~(size_t)255;
-    const size_t need = staged ? oi + bi : bp;
-    if (dplans.bytes < need && (rc = dplans.alloc(need + need / 2))) return rc;
-    if (!staged && dtable.bytes < bt && (rc = dtable.alloc(bt + bt / 2))) return rc;
-    if (!staged && ditems.bytes < bi && (rc = ditems.alloc(bi + bi / 2))) return rc;
-    unsigned char* const table_at = staged ? (unsigned char*)dplans.p + ot : (unsigned char*)dtable.p;
-    unsigned char* const items_at = staged ? (unsigned char*)dplans.p + oi : (unsigned char*)ditems.p;
+    const size_t need = oi + bi;
+    if (tables.bytes < need && (rc = tables.alloc(stage ? need + need / 2 : need))) return rc;
+    unsigned char* const base = (unsigned char*)tables.p;
     std::vector<MItem> all;
     all.reserve(nitems);
     for (const Group* g : gs) {
@@ -545,9 +540,9 @@ int WorkList::finalize(DevBuf& dplans, DevBuf& ditems, DevBuf& dtable,
         L.cprec = g->cprec;
         L.block = g->block;
         L.lds = g->lds;
-        L.items = reinterpret_cast<const MItem*>(items_at) + all.size();
+        L.items = reinterpret_cast<const MItem*>(base + oi) + all.size();
         L.nitems = (int64_t)order.size();
-        L.plans = reinterpret_cast<const MPlan*>(dplans.p);
+        L.plans = reinterpret_cast<const MPlan*>(base);
         L.phase = g->phase;
         // microseconds, roughly: the longest item alone (1.5e-4 per unit of its cost on MI355X: a
         // rows item of 8192 points 22 us, a convolution of 8190 points 55), then the rest of the
@@ -561,36 +556,27 @@ int WorkList::finalize(DevBuf& dplans, DevBuf& ditems, DevBuf& dtable,
         L.cost = 1.5e-4 * (longest + total / 400) * (g->cprec == (int)Prec::F64 ? 1.5 : 1.0);
         for (size_t k : order) {
             MItem it = g->items[k];
-            if (it.flags & kLineTable) it.aux += (uint64_t)table_at;
+            if (it.flags & kLineTable) it.aux += (uint64_t)(base + ot);
             all.push_back(it);
         }
         out.push_back(L);
     }
-    if (staged) {
+    std::vector<unsigned char> host;
+    unsigned char* h;
+    if (stage) {
         if (stage->reserve(need)) return fail(CFFT_ERR_NOMEM, "pinned staging failed");
-        unsigned char* h = static_cast<unsigned char*>(stage->p);
-        std::memcpy(h, mplans_.data(), bp);
-        if (!table_.empty()) std::memcpy(h + ot, table_.data(), table_.size() * 8);
-        if (!all.empty()) std::memcpy(h + oi, all.data(), all.size() * sizeof(MItem));
-        CFFT_HIP(hipMemcpyAsync(dplans.p, h, need, hipMemcpyHostToDevice, st));
-        return CFFT_OK;
+        h = static_cast<unsigned char*>(stage->p);
+    } else {
+        host.resize(need);
+        h = host.data();
     }
-    if (async) {
-        host_.resize(bp + bt + bi);
-        unsigned char* h = host_.data();
-        std::memcpy(h, mplans_.data(), bp);
-        if (!table_.empty()) std::memcpy(h + bp, table_.data(), table_.size() * 8);
-        if (!all.empty()) std::memcpy(h + bp + bt, all.data(), all.size() * sizeof(MItem));
-        CFFT_HIP(hipMemcpyAsync(dplans.p, h, bp, hipMemcpyHostToDevice, st));
-        CFFT_HIP(hipMemcpyAsync(dtable.p, h + bp, bt, hipMemcpyHostToDevice, st));
-        CFFT_HIP(hipMemcpyAsync(ditems.p, h + bp + bt, bi, hipMemcpyHostToDevice, st));
-        return CFFT_OK;
-    }
-    if (bp) CFFT_HIP(hipMemcpy(dplans.p, mplans_.data(), bp, hipMemcpyHostToDevice));
-    if (!table_.empty())
-        CFFT_HIP(hipMemcpy(dtable.p, table_.data(), table_.size() * 8, hipMemcpyHostToDevice));
-    if (!all.empty())
-        CFFT_HIP(hipMemcpy(ditems.p, all.data(), all.size() * sizeof(MItem), hipMemcpyHostToDevice));
+    std::memcpy(h, mplans_.data(), bp);
+    if (!table_.empty()) std::memcpy(h + ot, table_.data(), table_.size() * 8);
+    if (!all.empty()) std::memcpy(h + oi, all.data(), all.size() * sizeof(MItem));
+    if (stage)
+        CFFT_HIP(hipMemcpyAsync(base, h, need, hipMemcpyHostToDevice, st));
+    else
+        CFFT_HIP(hipMemcpy(base, h, need, hipMemcpyHostToDevice));
     return CFFT_OK;
 }
 
@@ -602,7 +588,7 @@ constexpr int kCaptureSides = 3;
 
 struct UnevenState {
     std::vector<std::unique_ptr<Plan>> plans;
-    DevBuf dplans, ditems, dtable, work;
+    DevBuf tables, work;
     std::vector<MultiLaunch> launches;
     hipStream_t cap = nullptr;
     hipStream_t side[kCaptureSides] = {};
@@ -845,14 +831,14 @@ int uneven_create(Ctx* ctx, int64_t count, const int64_t* lengths, const int64_t
         }
         W.add_transforms(q.e, xs);
     }
-    if ((rc = W.finalize(st->dplans, st->ditems, st->dtable, st->launches))) return rc;
+    if ((rc = W.finalize(st->tables, st->launches))) return rc;
     CFFT_HIP(hipStreamCreateWithFlags(&st->cap, hipStreamNonBlocking));
     CFFT_HIP(hipEventCreateWithFlags(&st->fork, hipEventDisableTiming));
     for (int i = 0; i < kCaptureSides; ++i) {
         CFFT_HIP(hipStreamCreateWithFlags(&st->side[i], hipStreamNonBlocking));
         CFFT_HIP(hipEventCreateWithFlags(&st->join[i], hipEventDisableTiming));
     }
-    size_t bytes = st->dplans.bytes + st->ditems.bytes + st->dtable.bytes + st->work.bytes;
+    size_t bytes = st->tables.bytes + st->work.bytes;
     for (auto& p : st->plans) bytes += plan_device_bytes(*p);
     P->uneven_bytes = bytes;
     std::ostringstream os;

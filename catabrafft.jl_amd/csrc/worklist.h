@@ -36,12 +36,11 @@ class WorkList {
     PlanEntry add_plan(const Plan& p);
     // Adds every item of the given transforms of one plan entry.
     void add_transforms(const PlanEntry& e, const std::vector<XformRef>& xs);
-    // Uploads descriptors, line tables and items; returns the launches in execution order.
-    // Uploads the tables (growing the device buffers when too small) and fills `out`.  With
-    // async, the uploads are enqueued on `st` from `stage` (pinned host memory that must stay
-    // untouched until they complete) or, without one, from this work list's own host buffer.
-    int finalize(DevBuf& dplans, DevBuf& ditems, DevBuf& dtable, std::vector<MultiLaunch>& out,
-                 hipStream_t st = nullptr, bool async = false, HostStage* stage = nullptr);
+    // Uploads descriptors, line tables and items (growing the device buffer when too small) and
+    // fills `out` with the launches in execution order.  With a stage (pinned host memory that must
+    // stay untouched until then) the upload is enqueued on `st`.
+    int finalize(DevBuf& tables, std::vector<MultiLaunch>& out, hipStream_t st = nullptr,
+                 HostStage* stage = nullptr);
     size_t item_count() const;
 
    private:
@@ -61,7 +60,6 @@ class WorkList {
     std::pair<Key, Group*> recent_[4];
     int recent_next_ = 0;
     std::vector<uint64_t> table_;
-    std::vector<unsigned char> host_;  // staging for async uploads (kept alive by the caller)
 
     int add_mplan(const MPlan& m) {
         mplans_.push_back(m);
@@ -72,9 +70,6 @@ class WorkList {
     void add_lines(int phase, MultiKernel k, const Plan& lp, int mplan, Prec prec, int C,
                    int block, size_t lds, const std::vector<XformRef>& xs, double line_cost,
                    bool epilogue, int variant);
-
-   public:
-    const std::vector<unsigned char>& staging() const { return host_; }
 };
 
 MLine make_mline(const LinePlan& lp);
