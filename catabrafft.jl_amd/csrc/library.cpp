@@ -613,23 +613,22 @@ static int fixed_stride(Ctx* ctx, const FixedShape& f, int cols, size_t reserve)
     return best;
 }
 
-// A fixed pass for a line (nullptr: none, or its tile does not fit): `C` lines per workgroup, a
+// A fixed pass for a line (f = nullptr: none, or its tile does not fit): `C` lines per workgroup, a
 // power of two, halved until they fit the workgroup and the LDS beside `reserve` bytes.
-static const FixedFs* pick_fixed_fs(Ctx* ctx, FixedFsKind kind, const LinePlan& lp, size_t reserve,
-                                    int* C, int* Ls, bool pass_a = false) {
+static FixedPass pick_fixed_fs(Ctx* ctx, FixedFsKind kind, const LinePlan& lp, size_t reserve, int C,
+                               bool pass_a = false) {
     const FixedFs* f = find_fixed_fs(kind, lp.pt, lp.N);
-    if (!f || (pass_a && !f->launch_a)) return nullptr;
+    if (!f || (pass_a && !f->launch_a)) return {};
     const size_t per = (size_t)f->elem * ((f->pad < 0 ? lp.N : lp.N + (lp.N >> f->pad)) + 64);
-    int c = *C / f->width;
+    int c = C / f->width;
     auto fits = [&](int k) {
         return k >= 1 && k * f->Tt <= f->max_threads && k * per + reserve <= ctx->lds_max;
     };
     while (c > 1 && !fits(c)) c /= 2;
-    if (!fits(c)) return nullptr;
-    *C = c * f->width;
-    *Ls = fixed_stride(ctx, FixedShape{f->r, f->np, f->N, f->Tt, f->elem, f->pad, false}, c, reserve);
+    if (!fits(c)) return {};
     f->prepare();
-    return f;
+    return {f, c * f->width,
+            fixed_stride(ctx, FixedShape{f->r, f->np, f->N, f->Tt, f->elem, f->pad, false}, c, reserve)};
 }
 
 static int pick_tile(Ctx* ctx, const LinePlan& lp, Prec pr, int want, size_t reserve = 0) {
@@ -1300,10 +1299,12 @@ static void fs_fixed_setup(Ctx* ctx, Plan& p) {
     // 4, 8, 16 and pass B tiles of 4 to 32 lines.  F32: pass A 4 (8 lines: 24,000 x 512 105.7 ->
     // 116.9 us, 2^20 x 64 505 -> 556), pass B 16 (8 lines: 2^20 x 64 525, 4: 580).  F64: 8 and 16
     // (4 and 4 lines: 20,000 x 512 145.6 -> 157.7 us, 2^18 x 128 453 -> 475, 2^17 x 64 123 -> 127).
-    fs.FCA = f64 ? 8 : 4;
-    fs.FCB = 16;
-    fs.fixed_a = pick_fixed_fs(ctx, kind(fs.N2), fs.a, 16, &fs.FCA, &fs.FLsA, true);
-    fs.fixed_b = pick_fixed_fs(ctx, kind(fs.N1), fs.b, table + 16, &fs.FCB, &fs.FLsB);
+    const int ca = f64 ? 8 : 4, cb = 16;
+    fs.fixed_a = pick_fixed_fs(ctx, kind(fs.N2), fs.a, 16, ca, true);
+    fs.fixed_b = pick_fixed_fs(ctx, kind(fs.N1), fs.b, table + 16, cb);
+    if (f64 || half) return;
+    fs.single_a = pick_fixed_fs(ctx, FixedFsKind::F32, fs.a, 16, ca, true);
+    fs.single_b = pick_fixed_fs(ctx, FixedFsKind::F32, fs.b, table + 16, cb);
 }
 
 // Two lines per thread for the ComplexF32 four-step passes in `mask` (bit 0: A, bit 1: B) whose
@@ -1454,8 +1455,8 @@ static std::string describe(const Plan& p) {
                << " Ls=" << p.fs.a.Ls << " N2=" << p.fs.N2 << " " << rad(p.fs.b)
                << " CB=" << p.fs.CB << " Ls=" << p.fs.b.Ls;
             if (p.fs.chunk) os << " chunk=" << p.fs.chunk;
-            if (p.fs.fixed_a || p.fs.fixed_b)
-                os << " fixed=" << (p.fs.fixed_a ? "A" : "") << (p.fs.fixed_b ? "B" : "");
+            if (p.fs.fixed_a.f || p.fs.fixed_b.f)
+                os << " fixed=" << (p.fs.fixed_a.f ? "A" : "") << (p.fs.fixed_b.f ? "B" : "");
             if (p.fs.pipe_a || p.fs.pipe_b)
                 os << " pipe=" << (p.fs.pipe_a ? "A" : "") << (p.fs.pipe_b ? "B" : "");
             if (p.fs.pair_a || p.fs.pair_b)
@@ -1500,8 +1501,8 @@ static int run_fft(const Plan& p, const void* in, void* out, int sgn, double sca
 static bool al16(const void* q) { return ((uintptr_t)q & 15) == 0; }
 // Whether a fixed pass may run on lines of elements of `elem` bytes at q: its pairs of adjacent
 // lines are read and written as one access of 2 elem bytes.
-static bool pair_fits(const FixedFs* f, const void* q, int64_t dist, size_t elem) {
-    return f->width == 1 || (((uintptr_t)q & (2 * elem - 1)) == 0 && dist % 2 == 0);
+static bool pair_fits(const FixedPass& p, const void* q, int64_t dist, size_t elem) {
+    return p.f && (p.f->width == 1 || (((uintptr_t)q & (2 * elem - 1)) == 0 && dist % 2 == 0));
 }
 
 // Pass A of nb transforms.
@@ -1523,10 +1524,11 @@ static int fourstep_pass_a(const Plan& p, const void* inb, void* midb, int64_t i
     a.mid_plain = fs.chunk > 0;  // a chunk's middle is read back while still cached
     const int64_t es_ = esize(p.prec);
     const size_t eio = io_esize(p);
-    if (fs.fixed_a && pair_fits(fs.fixed_a, inb, idist, eio)) {
-        a.C = fs.FCA;
-        a.Ls = fs.FLsA;
-        CFFT_HIP(fs.fixed_a->launch_a(inb, midb, a, fs.a.dtw.p, st));
+    const FixedPass& own = pair_fits(fs.fixed_a, inb, idist, eio) ? fs.fixed_a : fs.single_a;
+    if (own.f) {
+        a.C = own.C;
+        a.Ls = own.Ls;
+        CFFT_HIP(own.f->launch_a(inb, midb, a, fs.a.dtw.p, st));
     } else if (p.half) {
         CFFT_HIP(launch_fourstep_a_f16(inb, midb, a, fs.a.pt, fs.a.dtw.p, st));
     } else if (fs.pair_a && al16(inb) && al16(midb) && idist % 2 == 0 && mdist % 2 == 0) {
@@ -1567,11 +1569,12 @@ static int fourstep_pass_b(const Plan& p, const void* midb, void* outb, int64_t 
     b.tnc = fs.tnc;
     b.tw3 = fs.tw3.p;
     b.xcd = 1;
-    if (fs.fixed_b && !epi.K && pair_fits(fs.fixed_b, midb, mdist, es) &&
-        pair_fits(fs.fixed_b, outb, odist, eio)) {
-        b.C = fs.FCB;
-        b.Ls = fs.FLsB;
-        CFFT_HIP(fs.fixed_b->launch_b(midb, outb, b, fs.b.dtw.p, st));
+    const bool pairs = pair_fits(fs.fixed_b, midb, mdist, es) && pair_fits(fs.fixed_b, outb, odist, eio);
+    const FixedPass& own = pairs ? fs.fixed_b : fs.single_b;
+    if (own.f && !epi.K) {
+        b.C = own.C;
+        b.Ls = own.Ls;
+        CFFT_HIP(own.f->launch_b(midb, outb, b, fs.b.dtw.p, st));
     } else if (p.half) {
         CFFT_HIP(launch_fourstep_b_f16(midb, outb, b, fs.b.pt, fs.b.dtw.p, st));
     } else if (fs.pair_b && !epi.K && al16(midb) && al16(outb) && mdist % 2 == 0 &&
@@ -1751,11 +1754,14 @@ static int run_fft_s(const Plan& p, const void* in, void* out, int sgn, double s
             b.scale = scale;
             b.epi = epi;
             b.xcd = 1;
-            const FixedFs* f = p.fs.fixed_b;
-            if (f && (f->width == 1 || ((((uintptr_t)in | (uintptr_t)out) & 15) == 0))) {
-                b.C = p.fs.FCB;
-                b.Ls = p.fs.FLsB;
-                CFFT_HIP(f->launch_b(in, out, b, p.fs.b.dtw.p, st));
+            const size_t es = esize(p.prec);
+            const bool pairs = pair_fits(p.fs.fixed_b, in, p.idist, es) &&
+                               pair_fits(p.fs.fixed_b, out, p.odist, es);
+            const FixedPass& own = pairs ? p.fs.fixed_b : p.fs.single_b;
+            if (own.f) {
+                b.C = own.C;
+                b.Ls = own.Ls;
+                CFFT_HIP(own.f->launch_b(in, out, b, p.fs.b.dtw.p, st));
                 return CFFT_OK;
             }
             CFFT_HIP(launch_fourstep_b(p.prec, in, out, b, p.fs.b.pt, p.fs.b.dtw.p, st));
@@ -2111,14 +2117,16 @@ int plan_nd_create(Ctx* ctx, int rank, const int64_t* dims, int64_t axes_mask, i
             s->fs.b.Ls = fs_line_stride(ctx, p->prec, s->fs.b, s->fs.CB, 16);
             // its own kernel where the block's byte offsets fit 32 bits
             if (inner * N2 * esize(p->prec) < ((int64_t)1 << 32)) {
-                s->fs.FCB = p->prec == Prec::F32 ? 16 : 8;
+                const int cb = p->prec == Prec::F32 ? 16 : 8;
                 s->fs.fixed_b = pick_fixed_fs(ctx, p->prec == Prec::F64 ? FixedFsKind::F64
                                                    : inner % 2          ? FixedFsKind::F32
                                                                         : FixedFsKind::F32Pair,
-                                              s->fs.b, 16, &s->fs.FCB, &s->fs.FLsB);
+                                              s->fs.b, 16, cb);
+                if (p->prec == Prec::F32)
+                    s->fs.single_b = pick_fixed_fs(ctx, FixedFsKind::F32, s->fs.b, 16, cb);
             }
             os << " | axis " << a << ": strided lines N=" << N2 << " x " << inner << " C="
-               << (s->fs.fixed_b ? s->fs.FCB : s->fs.CB) << (s->fs.fixed_b ? " fixed" : "");
+               << (s->fs.fixed_b.f ? s->fs.fixed_b.C : s->fs.CB) << (s->fs.fixed_b.f ? " fixed" : "");
         }
         p->parts.push_back(std::move(s));
     }
@@ -2145,8 +2153,8 @@ static void real_fixed_setup(Ctx* ctx, Plan& p) {
     const Plan& f = *p.rsub_fwd;
     const FourStepPlan& fs = f.fs;
     // both passes' own kernels, so that the sub-plans run unchunked default shapes
-    if (f.kind != Kind::FourStep || p.rsub_bwd->kind != Kind::FourStep || !fs.fixed_a ||
-        !fs.fixed_b || !p.rsub_bwd->fs.fixed_b || p.rsub_bwd->fs.N1 != fs.N1)
+    if (f.kind != Kind::FourStep || p.rsub_bwd->kind != Kind::FourStep || !fs.fixed_a.f ||
+        !fs.fixed_b.f || !p.rsub_bwd->fs.fixed_b.f || p.rsub_bwd->fs.N1 != fs.N1)
         return;
     const FixedReal* rb = find_fixed_real(p.prec, fs.b.pt, fs.N2);
     const FixedReal* ra = find_fixed_real(p.prec, fs.a.pt, fs.N1);

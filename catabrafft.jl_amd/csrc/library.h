@@ -36,6 +36,12 @@ struct LinePlan {
     DevBuf dtw;
 };
 
+// A fixed four-step pass with its tile and LDS line stride.
+struct FixedPass {
+    const FixedFs* f = nullptr;
+    int C = 1, Ls = 0;
+};
+
 struct FourStepPlan {
     int N1 = 0, N2 = 0, CA = 1, CB = 1;
     LinePlan a, b;
@@ -48,10 +54,9 @@ struct FourStepPlan {
     // of a line pair; a call whose addresses or distances are not 16-byte aligned runs the float
     // kernels on the same tiles
     int pair_a = 0, pair_b = 0, LsA2 = 0, LsB2 = 0;
-    // the passes' own kernels, their tiles and LDS line strides (nullptr: the run-time kernels,
-    // which also run where a pair kernel's alignment is not met)
-    const FixedFs *fixed_a = nullptr, *fixed_b = nullptr;
-    int FCA = 1, FCB = 1, FLsA = 0, FLsB = 0;
+    // the passes' own kernels (f = nullptr: the run-time kernels), and those with one line per thread
+    // that run where a ComplexF32 pair kernel's alignment is not met
+    FixedPass fixed_a, fixed_b, single_a, single_b;
     int64_t chunk = 0;  // transforms per pass-A/pass-B round (0 = the whole batch)
 };
 
