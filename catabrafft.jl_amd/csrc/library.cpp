@@ -571,7 +571,8 @@ static int fixed_stride(Ctx* ctx, const FixedShape& f, int cols, size_t reserve)
     const int base = at(f.N - 1) + 1;
     int best = base, word[64], acc[64];
     long best_cost = -1;
-    for (int Ls = base; Ls < base + 64; ++Ls) {
+    // (strides that differ by a whole round of the 64 banks cost the same)
+    for (int Ls = base; Ls < base + 64 / ew; ++Ls) {
         if ((size_t)f.elem * cols * Ls + reserve > ctx->lds_max) break;
         long cost = 0;
         auto over = [&] { return best_cost >= 0 && cost >= best_cost; };
