@@ -546,14 +546,20 @@ int WorkList::finalize(DevBuf& tables, std::vector<MultiLaunch>& out, hipStream_
         L.phase = g->phase;
         // microseconds, roughly: the longest item alone (1.5e-4 per unit of its cost on MI355X: a
         // rows item of 8192 points 22 us, a convolution of 8190 points 55), then the rest of the
-        // items on about 400 resident workgroups
+        // items on about 400 resident workgroups; the launches of large convolutions, which gather
+        // and scatter, take 2.5 times as long (1000 lengths up to 2^18: estimated 200 us, measured
+        // 500 on a GPU shared with the rest of the batch)
         double total = 0, longest = 0;
         for (size_t k = 0; k < g->runs.size(); ++k) {
             const size_t end = k + 1 < g->runs.size() ? g->runs[k + 1].second : g->items.size();
             total += g->runs[k].first * (double)(end - g->runs[k].second);
             longest = std::max(longest, g->runs[k].first);
         }
-        L.cost = 1.5e-4 * (longest + total / 400) * (g->cprec == (int)Prec::F64 ? 1.5 : 1.0);
+        const MultiKernel mk = (MultiKernel)g->kernel;
+        const bool large = mk == MultiKernel::ConvFA || mk == MultiKernel::ConvFBA ||
+                           mk == MultiKernel::ConvFC;
+        L.cost = 1.5e-4 * (longest + total / 400) * (g->cprec == (int)Prec::F64 ? 1.5 : 1.0) *
+                 (large ? 2.5 : 1.0);
         for (size_t k : order) {
             MItem it = g->items[k];
             if (it.flags & kLineTable) it.aux += (uint64_t)(base + ot);
