@@ -106,25 +106,27 @@ struct SrvRequest {
     std::string err;
 };
 
+// The independent launches of a round are spread over its slot's stream and this many others, which
+// the slots share: a request's kernels have tens to hundreds of workgroups, too few to fill the GPU
+// in turn.  (A burst of 48 requests of 64 to 2^18 points: 850 -> 692 us.  Streams of each slot's own
+// are more than the four hardware queues: two of a round's four then fell on one, 572 -> 603 us.)
+// What rounds in flight have put on a shared stream counts where a round chooses, so that a short
+// round does not queue behind a long one.  Created by the first round that spreads; where they cannot
+// be, rounds run on their slots' streams alone.
+constexpr int kSideStreams = 3;
+
 struct SrvRound {
     std::vector<SrvRequest*> reqs;
     WorkList wl;
     std::vector<MultiLaunch> launches;
     int slot = 0;
+    double side_cost[kSideStreams] = {};  // what it has put on the shared streams
 };
-
-// The independent launches of a round are spread over its slot's stream and this many others of the
-// slot: a request's kernels have tens to hundreds of workgroups, too few to fill the GPU in turn.
-// (A burst of 48 requests of 64 to 2^18 points: 850 -> 692 us.)  No other slot's rounds run on them:
-// a round waits for none of another round's kernels in stream order.  Created by the slot's first
-// round that spreads; where they cannot be, the slot's rounds run on its own stream.
-constexpr int kSideStreams = 3;
 
 // A stream with the resources its rounds reuse (one round at a time per slot).
 struct SrvSlot {
     hipStream_t stream = nullptr;
     hipEvent_t done = nullptr;
-    hipStream_t side[kSideStreams] = {};
     hipEvent_t fork = nullptr, join[kSideStreams] = {};
     bool busy = false;
     DevBuf tables;
@@ -133,8 +135,6 @@ struct SrvSlot {
         if (stream) (void)hipStreamDestroy(stream);
         if (done) (void)hipEventDestroy(done);
         if (fork) (void)hipEventDestroy(fork);
-        for (hipStream_t s : side)
-            if (s) (void)hipStreamDestroy(s);
         for (hipEvent_t e : join)
             if (e) (void)hipEventDestroy(e);
     }
@@ -144,6 +144,8 @@ struct Server {
     Ctx* ctx = nullptr;
     size_t cap = 0;
     std::vector<SrvSlot> slots;
+    hipStream_t side[kSideStreams] = {};
+    double side_load[kSideStreams] = {};  // estimated us of the rounds in flight (server thread)
     std::thread worker;
     std::mutex mu;
     std::condition_variable cv_work, cv_done;
@@ -223,15 +225,15 @@ static void srv_release(Server* s, SrvRequest* r) {
     r->bytes = 0;
 }
 
-// Whether the slot has its side streams and their events (created here at the first call).
-static bool srv_side_streams(SrvSlot& sl) {
+// Whether the shared streams and the slot's events are there (created here at the first call).
+static bool srv_side_streams(Server* s, SrvSlot& sl) {
     auto event = [](hipEvent_t* e) {
         return *e || hipEventCreateWithFlags(e, hipEventDisableTiming) == hipSuccess;
     };
     bool ok = event(&sl.fork);
     for (int i = 0; i < kSideStreams && ok; ++i)
-        ok = (sl.side[i] ||
-              hipStreamCreateWithFlags(&sl.side[i], hipStreamNonBlocking) == hipSuccess) &&
+        ok = (s->side[i] ||
+              hipStreamCreateWithFlags(&s->side[i], hipStreamNonBlocking) == hipSuccess) &&
              event(&sl.join[i]);
     if (!ok) (void)hipGetLastError();
     return ok;
@@ -374,9 +376,10 @@ static int srv_launch_round(Server* s, std::vector<SrvRequest*>& admitted, int s
                      [](const Task& a, const Task& b) { return a.cost > b.cost; });
     const MultiArgs ma{0, 0, 1, 0};
     double load[kSideStreams + 1] = {};
+    for (int i = 0; i < kSideStreams; ++i) load[i + 1] = s->side_load[i];
     bool forked[kSideStreams] = {};
     // a round of work lists alone is short: the events would cost it more than they give
-    const bool spread = direct.size() > 1 && rc == CFFT_OK && srv_side_streams(sl);
+    const bool spread = direct.size() > 1 && rc == CFFT_OK && srv_side_streams(s, sl);
     if (spread && hipEventRecord(sl.fork, st) != hipSuccess)
         rc = fail(CFFT_ERR_HIP, "forking the round's streams failed");
     for (const Task& t : tasks) {
@@ -385,7 +388,8 @@ static int srv_launch_round(Server* s, std::vector<SrvRequest*>& admitted, int s
         for (int i = 1; i <= kSideStreams && spread; ++i)
             if (load[i] < load[k]) k = i;
         load[k] += t.cost;
-        hipStream_t ts = k ? sl.side[k - 1] : st;
+        if (k) R->side_cost[k - 1] += t.cost;
+        hipStream_t ts = k ? s->side[k - 1] : st;
         if (k && !forked[k - 1]) {
             if (hipStreamWaitEvent(ts, sl.fork, 0) != hipSuccess) {
                 rc = fail(CFFT_ERR_HIP, "stream wait failed");
@@ -408,7 +412,7 @@ static int srv_launch_round(Server* s, std::vector<SrvRequest*>& admitted, int s
     }
     for (int i = 0; i < kSideStreams; ++i) {
         if (!forked[i]) continue;
-        if ((hipEventRecord(sl.join[i], sl.side[i]) != hipSuccess ||
+        if ((hipEventRecord(sl.join[i], s->side[i]) != hipSuccess ||
              hipStreamWaitEvent(st, sl.join[i], 0) != hipSuccess) &&
             rc == CFFT_OK)
             rc = fail(CFFT_ERR_HIP, "stream join failed");
@@ -429,12 +433,13 @@ static int srv_launch_round(Server* s, std::vector<SrvRequest*>& admitted, int s
     lk.lock();
     if (rc != CFFT_OK) {
         // nothing of this round may still run when its buffers return to the pool
-        for (hipStream_t ss : sl.side)
+        for (hipStream_t ss : s->side)
             if (ss) (void)hipStreamSynchronize(ss);
         (void)hipStreamSynchronize(st);
         sl.busy = false;
         return rc;
     }
+    for (int i = 0; i < kSideStreams; ++i) s->side_load[i] += R->side_cost[i];
     s->inflight.push_back(std::move(R));
     return CFFT_OK;
 }
@@ -458,6 +463,7 @@ static void srv_retire(Server* s) {
             s->flops += 5.0 * r->n * std::log2((double)std::max<int64_t>(r->n, 2)) * r->batch;
         }
         s->slots[R->slot].busy = false;
+        for (int i = 0; i < kSideStreams; ++i) s->side_load[i] -= R->side_cost[i];
         it = s->inflight.erase(it);
         s->cv_done.notify_all();
     }
@@ -672,6 +678,8 @@ int cfft_server_destroy(cfft_server srv) {
     if (s->worker.joinable()) s->worker.join();
     (void)hipSetDevice(s->ctx->device);
     for (auto& sl : s->slots) sl.destroy();
+    for (hipStream_t st : s->side)
+        if (st) (void)hipStreamDestroy(st);
     delete s;
     delete srv;
     return CFFT_OK;
