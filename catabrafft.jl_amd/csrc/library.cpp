@@ -796,10 +796,13 @@ static double line_noise(const std::vector<int>& r) {
         v += count[R] * kPassNoise[R] + count[R] * count[R] * kRepeatedNoise[R];
     return v;
 }
-// Two-line lengths in F32 round by 5 to 10 % more than the sum of their passes says where they have no
-// factor 5 (98 lengths from 16,464 to 2^21, on these kernels and on the run-time ones).
+// What two-line lengths round by besides (squared errors, on these kernels and on the run-time ones):
+// in F32 5 to 10 % more where they have no factor 5 (98 lengths from 16,464 to 2^21); in F64 up to
+// 1.4 times as much where they have a factor 2^15 and no 3 (100 lengths from 17,496 to 983,040; 2^17 5,
+// 2^18 and 2^16 5 most).
 static double two_line_noise(int64_t L, Prec prec) {
-    return prec == Prec::F32 && L % 5 ? 1.1 : 1.0;
+    if (prec == Prec::F32) return L % 5 ? 1.1 : 1.0;
+    return L % 32768 == 0 && L % 3 ? 1.25 : 1.0;
 }
 // The split of length L itself (L = 0 in the result: none): N1 >= N2, the most even one (launch A
 // reads its columns in longer runs), but N2 > N1 where that keeps the F64 lines of launch C at 1024
@@ -838,8 +841,8 @@ static const std::vector<ConvSplit>& conv_splits(Prec prec) {  // one per length
     return t[prec == Prec::F64];
 }
 // Length of a convolution that needs at least m points: of the fixed kernels' lengths that the plan
-// may run, the cheapest whose rounding noise is no more than that of the shortest 7-smooth length;
-// else that length.  (The shortest or cheapest one by itself had up to 18 % larger errors: F32 n =
+// may run, the cheapest whose rounding noise is no more than that of the shortest 7-smooth length
+// (which may have a kernel of its own, with another order of radices); else that length.  (The shortest or cheapest one by itself had up to 18 % larger errors: F32 n =
 // 317 at L = 648 = 8 9 9 instead of 640 = 16 8 5.)  io: the transform's precision (the results of an
 // F64 convolution round by far more than it does where they are F32).
 static int64_t conv_length(int64_t m, Prec prec, Prec io, ConvKernels own) {
@@ -851,7 +854,8 @@ static int64_t conv_length(int64_t m, Prec prec, Prec io, ConvKernels own) {
     if (f && own.fused) {
         for (; f; f = find_fixed_conv(prec, f->N + 1, false)) {
             const double cost = f->N * (f->np + 0.3);
-            if (cost < best && line_noise(std::vector<int>(f->r, f->r + f->np)) <= noise) {
+            if (cost < best && (f->N == shortest ||
+                                line_noise(std::vector<int>(f->r, f->r + f->np)) <= noise)) {
                 best = cost;
                 L = f->N;
             }
@@ -864,7 +868,7 @@ static int64_t conv_length(int64_t m, Prec prec, Prec io, ConvKernels own) {
         double least = 1e300;
         int64_t quiet = 0;  // the least noisy of the lengths up to 1.5 m, where all are noisier
         for (; it != v.end(); ++it) {
-            if (it->cost < best && (prec != io || it->noise <= noise)) {
+            if (it->cost < best && (prec != io || it->L == shortest || it->noise <= noise)) {
                 best = it->cost;
                 L = it->L;
             }

@@ -426,6 +426,31 @@ def test_emulated_padded_convolutions_are_as_accurate_as_the_shortest(emu, tmp_p
     emu.cfft_finalize(ctx)
 
 
+@pytest.mark.parametrize("n,dt", [(25087, np.complex64), (100351, np.complex128), (129023, np.complex128),
+                                  (156734, np.complex128)])
+def test_emulated_large_convolutions_are_as_accurate_as_the_shortest(emu, tmp_path, n, dt):
+    """The same for convolutions of two lines, and the same bound: 100351 and 129023, whose shortest
+    length has kernels of its own, and 156734, whose shortest length has none."""
+    code = 0 if dt == np.complex64 else 1
+    x = seeded_complex(n, batch=2, seed=n, dtype=dt)
+    ref = np.fft.fft(x.astype(np.clongdouble))
+    w = tmp_path / "w.txt"
+    w.write_text(f"{n} 2 {n} {n} {code} 1 : 16 64 0 0 0 -1 0 0\n")
+    ctx, err, L = ctypes.c_void_p(), [], []
+    assert emu.cfft_init(0, ctypes.byref(ctx)) == 0
+    assert emu.cfft_wisdom_import(ctx, str(w).encode()) == 0
+    for flags in (0, 1):
+        p, y = ctypes.c_void_p(), np.zeros_like(x)
+        assert emu.cfft_plan_1d(ctx, n, 2, n, n, code, flags, ctypes.byref(p)) == 0
+        L.append(int(_desc(emu, p).split(" L=")[1].split()[0]))
+        assert emu.cfft_exec(p, x.ctypes.data, y.ctypes.data, -1, 0, None) == 0
+        err.append(float(np.linalg.norm(y - ref) / np.linalg.norm(ref)))
+        emu.cfft_plan_destroy(p)
+    assert (L[0] == L[1]) == (n != 156734), L
+    assert err[0] < (1 + 2 * np.sqrt(2) * 0.04) * err[1], (n, L, err)
+    emu.cfft_finalize(ctx)
+
+
 SHORT_PRIMES = [n for n in range(17, 2050) if _prime(n) and _factor_smooth(n - 1)]
 
 
