@@ -811,18 +811,22 @@ static double two_line_noise(int64_t L, Prec prec) {
 static ConvSplit conv_split_of(int64_t L, Prec prec) {
     const int most = prec == Prec::F64 ? 1024 : 1 << 30;
     ConvSplit best;
+    size_t passes = 99;  // the fewest of any split of L (below)
     auto rank = [&](int a, int b) { return std::make_tuple(a > most, a < b, std::max(a, b)); };
     for (int a : fixed_convl_lengths())
         for (int b : fixed_convl_lengths())
-            if ((int64_t)a * b == L && a <= 4 * b && b <= 4 * a &&
-                (!best.L || rank(a, b) < rank(best.N1, best.N2))) {
-                best = ConvSplit{L, a, b, 0, 0};
+            if ((int64_t)a * b == L && a <= 4 * b && b <= 4 * a) {
                 std::vector<int> r = fourstep_line_radices(a);
                 const std::vector<int> rb = fourstep_line_radices(b);
                 r.insert(r.end(), rb.begin(), rb.end());
-                best.cost = (double)L * (2 * r.size() + 6);
-                best.noise = line_noise(r) * two_line_noise(L, prec);
+                passes = std::min(passes, r.size());
+                if (!best.L || rank(a, b) < rank(best.N1, best.N2))
+                    best = ConvSplit{L, a, b, 0, line_noise(r) * two_line_noise(L, prec)};
             }
+    // Lengths that split into a few passes, evenly or not, have few and large factors: 2^16 3 as
+    // 512 x 384 (6 passes; 768 x 256 has 5) takes 51 us for 8 lines of 88607 in ComplexF32, 184320 =
+    // 576 x 320 (6) 60; 2^18 for 119101 58, 245760 = 640 x 384 68.
+    best.cost = (double)L * (2 * passes + 6);
     return best;
 }
 static const std::vector<ConvSplit>& conv_splits(Prec prec) {  // one per length, ascending

@@ -451,6 +451,17 @@ def test_emulated_large_convolutions_are_as_accurate_as_the_shortest(emu, tmp_pa
     emu.cfft_finalize(ctx)
 
 
+@pytest.mark.parametrize("n,L", [(88607, 1 << 16 | 1 << 17), (119101, 1 << 18)])
+def test_emulated_large_convolutions_prefer_few_large_factors(emu, n, L):
+    """2^16 3 before 2^12 45 and 2^18 before 2^14 15, which are shorter and slower."""
+    ctx, p = ctypes.c_void_p(), ctypes.c_void_p()
+    assert emu.cfft_init(0, ctypes.byref(ctx)) == 0
+    assert emu.cfft_plan_1d(ctx, n, 1, n, n, 0, 0, ctypes.byref(p)) == 0
+    assert f" L={L} " in _desc(emu, p)
+    emu.cfft_plan_destroy(p)
+    emu.cfft_finalize(ctx)
+
+
 SHORT_PRIMES = [n for n in range(17, 2050) if _prime(n) and _factor_smooth(n - 1)]
 
 
