@@ -9,9 +9,11 @@
 //   - the last forward pass, the product with the spectrum and the first pass of the second
 //     FFT_L use the same elements and stay in registers: 2 np - 1 passes instead of 2 np, and no
 //     pass of its own for the product.
-// What bounds it: VALU issue and the LDS exchanges of those passes (HBM moves 2 n elements a line).
+// What bounds it: VALU issue and the LDS exchanges of those passes (HBM moves 2 n elements a line),
+// and, where a line takes more than 512 threads, that the 120 or so registers of the middle pass leave
+// a CU one workgroup, whose barriers nothing hides.
 // n = 4099 x 4093 lines in ComplexF32, 269 MB: 516 us on the run-time kernel (L = 8232, 10 passes
-// and a product), 283 us here (L = 9216, 7 passes).
+// and a product), 275 us here (L = 8960, 7 passes of 560 threads).
 #pragma once
 #include "fixed_line.h"
 #include "fixed_table.h"

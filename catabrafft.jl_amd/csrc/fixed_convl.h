@@ -4,8 +4,9 @@
 // precision of x and y; Tc: precision of the convolution.
 //
 // What bounds them: A and C the gather and the scatter by the primitive root (8-byte elements all
-// over a line), BA the two work lines and K, 16 L bytes each in F64, and one workgroup a CU where a
-// tile is 4 lines of 2048.  n = 1048573 x 16 lines (ComplexF32, convolved in F64, L = 2^21): 387 +
+// over a line), BA the two work lines and K, 16 L bytes each in F64, and one workgroup a CU: F64 lines
+// with a radix 16 take 132 registers, where 128 would let a second one in (LDS would: a tile is two
+// lines of 2048).  n = 1048573 x 16 lines (ComplexF32, convolved in F64, L = 2^21): 387 +
 // 438 + 456 us on the run-time kernels, 327 + 533 + 352 here.  Short lines, whose index arithmetic
 // weighs more, gain more: n = 20011 x 512 in ComplexF32 406 us -> 326, x 256 in F64 354 -> 279.
 //

@@ -9,7 +9,8 @@
 //      resident plan (twiddles, Rader permutations, kernel spectra stay on the device) and their
 //      rows are packed together into the same work-list launches, transforms of other lengths
 //      go into the same launches too, and the round is enqueued on one of `nstreams` slots, its
-//      independent launches spread over the slot's streams.
+//      independent launches spread over the slot's stream and the streams that all slots share,
+//      by what the rounds in flight have queued there.
 // A request that arrives while earlier rounds run is admitted into the next round as soon as
 // memory and a stream slot free up, so its kernels overlap the running ones on the device.
 // Each transform's arithmetic depends only on its own plan, so a result is the same alone and in
